@@ -44,7 +44,7 @@ PEAK_BF16_TFLOPS = 2516.6  # MI355X dense bf16 MFMA (256 CU x 4096 FLOP/clk x 2.
 NS_KERNELS = {
     "fused": "ns5 stage: ns_st_kernel<0> (X X^T) + ns_ba_kernel (c A A^T + b A, then B X + a X with B kept in LDS) per iteration",
     "stream": "ns5 stage: ns_st_kernel<0> (X X^T), <1> (c A A^T + b A), <2> (B X + a X) per iteration",
-    "lds": "ns5 stage: ns5_lds_kernel (all 5 iterations of a 128-row tile resident in LDS)",
+    "lds": "ns5 stage: ns5_lds_kernel (128-row tiles) or ns5_reg_kernel (256x256): all 5 iterations of a tile on chip",
     "small": "ns5 stage: ns_gram_kernel x2 + ns_apply_kernel per iteration",
     "few_rows": "ns5 stage: ns5_small_kernel (all 5 iterations of a tile's 16, 32 or 64 rows resident in LDS)",
 }
@@ -56,8 +56,8 @@ def ns_family(mp: int, np_: int, family: str = "auto", rows: int = 0) -> str:
     everywhere; with "stream3" the three streamed 256-block products wherever
     both edges are multiples of 256; with "auto", the operand's own 16, 32 or
     64 rows in LDS when it has rows <= 32 real rows, or <= 64 at np = 128
-    ("few_rows"), LDS-resident
-    for mp == 128 and np in {128, 256, 512}, the Gram kernel plus the fused
+    ("few_rows"), on chip
+    for mp == 128 and np in {128, 256, 512} and for 256 x 256 tiles ("lds"), the Gram kernel plus the fused
     GramB/Apply kernel for 512 x 512 tiles, streamed 256-blocks for other
     multiples of 256, else 128-blocks."""
     if family == "block128":
@@ -66,7 +66,7 @@ def ns_family(mp: int, np_: int, family: str = "auto", rows: int = 0) -> str:
             (rows > 32 and np_ == 128) or (rows <= 32 and np_ in (128, 256, 384, 512, 768, 1024))
             or (rows <= 16 and np_ in (1536, 2048))):
         return "few_rows"
-    if mp == 128 and np_ in (128, 256, 512):
+    if mp == 128 and np_ in (128, 256, 512) or (family == "auto" and mp == 256 and np_ == 256):
         return "lds"
     if mp % 256 == 0 and np_ % 256 == 0:
         return "fused" if (family == "auto" and mp == 512 and np_ == 512) else "stream"
@@ -90,8 +90,9 @@ KERNEL_TRAFFIC = {
 }
 KERNEL_SOURCES = {
     "ns_ba_kernel": ["ns5_ba.hip", "ns5_kernels.h", "common.h"],
-    "ns5_lds_kernel": ["ns5_lds.hip", "ns5_kernels.h", "common.h", "elem_ops.h"],
-    "lds_step_kernel": ["ns5_lds.hip", "ns5_kernels.h", "common.h", "elem_ops.h"],
+    "ns5_lds_kernel": ["ns5_lds.hip", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
+    "lds_step_kernel": ["ns5_lds.hip", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
+    "ns5_reg_kernel": ["ns5_reg.hip", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
     "ns_st_kernel": ["ns5_stream.hip", "ns5_kernels.h", "common.h"],
 }
 
@@ -257,7 +258,7 @@ def time_dominant_kernel(opt, reps: int) -> dict:
     steps = g["steps"]
     ms = _event_loop(lambda: nat.ns5(x, y, inv, n, m, nn, steps, opt._workspace, n, round_once=grp.round_once),
                      reps, prep=grp.gather)
-    name = {"lds": "ns5_lds_kernel", "stream": "ns_st_kernel", "small": "ns_gram_kernel/ns_apply_kernel"}[fam]
+    name = {"lds": "ns5_lds_kernel" if m == 128 else "ns5_reg_kernel", "stream": "ns_st_kernel", "small": "ns_gram_kernel/ns_apply_kernel"}[fam]
     return {"kernel": name, "family": fam, "launch_tiles": n, "launch_ms": ms,
             "flops_per_launch": float(ns_flops(grp.m, grp.n)) * n}
 

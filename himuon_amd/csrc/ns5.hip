@@ -325,7 +325,10 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   uint16_t* wsB = wsA + sb * sq;
   // Family AUTO: tiles whose padded edges are multiples of 256 run the
   // persistent streamed-operand kernels (ns5_stream.hip); tiles with mp == 128
-  // and np in {128, 256, 512} run the fused LDS-resident kernel (ns5_lds.hip); other tiles
+  // and np in {128, 256, 512} run the fused LDS-resident kernel (ns5_lds.hip),
+  // 256 x 256 tiles the one that keeps X in registers (ns5_reg.hip: 16 tiles
+  // 0.086 against 0.187 ms for the streamed products, 256 tiles 0.105 against
+  // 0.34, 6,720 tiles 2.45-2.55 against 6.13-6.25 ms, same box); other tiles
   // run the 128-block kernels below, which family BLOCK128 selects for every
   // geometry.
   // 512 x 512 tiles run the first product on the stream kernels and the
@@ -335,6 +338,7 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   const bool st = ns5_stream_supported(mp, np) && !small;
   const bool lds = ns5_lds_supported(mp, np) && !small;
   const bool ba = ns5_ba_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
+  const bool reg = ns5_reg_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
   const int nb = mp / BM;
   const int npairs = nb * (nb + 1) / 2;
   const int apply_blocks = (mp / BM) * (np / BN);
@@ -346,6 +350,8 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
       if (!ns5_small_run(x + o, y + o, inv + s0, cnt, rows, np, steps, a, b, c, round_once, s)) return HIMUON_EINVAL;
     } else if (lds) {
       ns5_lds_run(x + o, y + o, inv + s0, cnt, mp, np, steps, a, b, c, round_once, s);
+    } else if (reg) {
+      ns5_reg_run(x + o, y + o, inv + s0, cnt, steps, a, b, c, round_once, s);
     } else if (st) {
       BaUntile u{};
       if (untile) {

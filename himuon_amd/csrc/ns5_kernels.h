@@ -229,3 +229,9 @@ bool ns5_small_run(const uint16_t* x, uint16_t* y, const float* inv, int64_t cnt
 bool ns5_lds_supported(int mp, int np);
 void ns5_lds_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int mp, int np, int steps,
                  float a, float b, float c, bool round_once, hipStream_t s);
+// NS tiles with mp == np == 256, X held in registers (ns5_reg.hip): all
+// `steps` >= 1 iterations in one launch, one workgroup per tile; reads x,
+// leaves the result in x (even `steps`) or y (odd).
+bool ns5_reg_supported(int mp, int np);
+void ns5_reg_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int steps, float a, float b, float c,
+                 bool round_once, hipStream_t s);

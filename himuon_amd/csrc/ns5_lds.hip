@@ -42,70 +42,13 @@
 // of one chunk and 4 consecutive rows of 2 chunks hit distinct bank groups.
 // np = 128: 52 KiB per workgroup, three workgroups per CU; np = 256: 84 KiB,
 // np = 512: 148 KiB, one per CU (eight waves).
-#include "elem_ops.h"
-#include "ns5_kernels.h"
+#include "lds_tiles.h"
+#include "tile_step.h"
 
 namespace {
 
 constexpr int NT = 256;
 constexpr int M = 128;  // NS rows (mp)
-
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-typedef __attribute__((address_space(3))) u32x4_t lds_u32x4;
-
-HM_DEV uint32_t lds_pos(int r, int ch, int chunks) {
-  const int sw = ((r & 3) << 2) | ((r >> 2) & 3);
-  return (uint32_t)(r * chunks + (ch ^ sw)) * 16u;
-}
-
-// Stored lower 32x32 tile (ti >= tj) of a symmetric 128 x 128 matrix:
-// byte offset of 16-byte chunk ch (columns 8 ch ..) of its row r.
-constexpr int TRI_TILE = 32 * 32 * 2;
-constexpr int TRI_BYTES = 10 * TRI_TILE;
-HM_DEV uint32_t tri_pos(int ti, int tj, int r, int ch) {
-  return (uint32_t)((ti * (ti + 1) / 2 + tj) * TRI_TILE + r * 64 + ((ch ^ ((r >> 2) & 3)) << 4));
-}
-
-// Transposing read: 4 bf16 of the 8-byte row segment at `off`, redistributed
-// across each group of 16 lanes (lane 4a + b receives element b of the
-// segments addressed by lanes a, a + 4, a + 8, a + 12).
-HM_DEV u32x2_t read_tr(const lds_u8* base, uint32_t off) {
-  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(base + off));
-  return __builtin_bit_cast(u32x2_t, r);
-}
-
-// The lane index, opaque to the optimiser: addresses derived from it are
-// formed inside each phase instead of being hoisted out of the iteration loop
-// for all four per-wave variants at once (which would not fit the registers).
-HM_DEV int opaque_lane(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
-// Row fragment of a symmetric matrix S stored as its lower tiles: lane (l32,
-// hi) receives S[32 R + l32][16 ks + 8 hi .. + 7] (the MFMA operand of row
-// tile R, k-step ks). Column tile k = ks / 2 > R is read from the stored tile
-// (k, R) as the transposing reads of the X operand do.
-template <int R, int KS>
-HM_DEV u32x4_t tri_frag(const lds_u8* S, int l32, int hi, int tr_krow, int tr_col) {
-  constexpr int TK = KS >> 1;
-  if constexpr (TK <= R) {
-    return *reinterpret_cast<lds_cu32x4*>(S + tri_pos(R, TK, l32, 2 * (KS & 1) + hi));
-  } else {
-    const int kr = 16 * (KS & 1) + tr_krow;
-    const u32x2_t l2 = read_tr(S, tri_pos(TK, R, kr, tr_col >> 3) + (tr_col & 7) * 2);
-    const u32x2_t u2 = read_tr(S, tri_pos(TK, R, kr + 4, tr_col >> 3) + (tr_col & 7) * 2);
-    return u32x4_t{l2[0], l2[1], u2[0], u2[1]};
-  }
-}
-
-// Transposing-read lane roles (the X operand of Apply, the upper fragments of
-// A and B): lane (a', b') of each 16-lane group addresses k-row 8 hi + a' (+ 4
-// for the second read) and columns 16 ((lane >> 4) & 1) + 4 b' .. + 3 of a
-// 32-column tile.
-HM_DEV int tr_krow_of(int lane) { return 8 * (lane >> 5) + ((lane & 15) >> 2); }
-HM_DEV int tr_col_of(int lane) { return 16 * ((lane >> 4) & 1) + 4 * (lane & 3); }
 
 // Wave W's share of a Gram product's lower 32x32 tiles: it loads the row tiles
 // ROW[0 .. NR-1] of the operand and computes tiles k < NTL, tile k being
@@ -390,7 +333,7 @@ __global__ __launch_bounds__(NTQ, NQ == 1 ? 3 : 1) void ns5_lds_kernel(const uin
   constexpr int N = 128 * NQ;   // NS columns (np)
   constexpr int XCH = N / 8;    // 16-byte chunks per X row
   __shared__ __attribute__((aligned(16))) uint8_t sx_raw[M * N * 2];
-  __shared__ __attribute__((aligned(16))) uint8_t sa_raw[TRI_BYTES];
+  __shared__ __attribute__((aligned(16))) uint8_t sa_raw[tri_bytes(4)];
   lds_u8* const X = (lds_u8*)sx_raw;
   lds_u8* const A = (lds_u8*)sa_raw;
 
@@ -458,154 +401,18 @@ __global__ __launch_bounds__(NTQ, NQ == 1 ? 3 : 1) void ns5_lds_kernel(const uin
 // 8-element vectors t, t + 256, ..., t + 1792 of the 128 x 128 tile, each in
 // element order; then the same wave and block reductions, and the same
 // 1 / (sqrt(s) + eps)).
-constexpr int SV_N = 128, SV_VPR = SV_N / 8;  // 16 vectors of 8 per NS row
-constexpr int SV_VPT = M * SV_VPR / NT;       // vectors per thread (8)
-// vectors loaded before any is used: the untile all 8 (8 VGPRs each), the
-// gather 4 (16 VGPRs each; 8 would spill)
-constexpr int SV_BATCH_UNT = 8, SV_BATCH_GAT = 4;
-
-struct TileAt {
-  const HimuonParamDesc* P;
-  int r, c;
-};
-
-HM_DEV TileAt tile_at(const HimuonParamDesc* __restrict__ params, int n_params, int64_t t) {
-  const HimuonParamDesc* P = params + find_param(params, n_params, t);
-  const int64_t lt = t - P->tile0;
-  return TileAt{P, (int)(lt / P->C), (int)(lt % P->C)};
-}
-
-// Exactly one of UNT and GAT. UNT: untile with WD/LR of tile tu from X (X'
-// of the NS iterations). GAT: momentum and gather of tile tg into X (bf16(e),
-// not yet normalised); returns this thread's sum of squares of it. Each
-// thread reads and writes only its own vectors v = k NT + tid of X.
-template <int DT, int PDT, bool UNT, bool GAT>
-HM_DEV float step_io(const HimuonParamDesc* __restrict__ params, int n_params, lds_u8* X, int64_t tu, int64_t tg,
-                     int tile_h, int tile_w, const float* __restrict__ sa) {
-#pragma clang fp contract(off)
-  static_assert(UNT != GAT, "one tile pass per call");
-  constexpr int XCH = SV_N / 8;
-  TileAt U{nullptr, 0, 0}, G{nullptr, 0, 0};
-  float s = 0.f, alpha = 0.f, sc = 0.f, mu = 0.f;
-  bool has_mom = false, nesterov = false;
-  if constexpr (UNT) {
-    U = tile_at(params, n_params, tu);
-    s = sa[2 * U.P->group];
-    alpha = sa[2 * U.P->group + 1];
-    sc = U.P->upd_scale;
-  }
-  if constexpr (GAT) {
-    G = tile_at(params, n_params, tg);
-    has_mom = G.P->momentum != nullptr;
-    mu = G.P->mu;
-    nesterov = G.P->nesterov != 0;
-  }
-  // (addresses from an opaque copy of the thread index: shared with the other
-  // pass and kept live across the NS iterations they would not fit beside
-  // those iterations' registers)
-  const int tq = opaque_lane((int)threadIdx.x);
-  float ssq = 0.f;
-  constexpr int SV_BATCH = UNT ? SV_BATCH_UNT : SV_BATCH_GAT;
-#pragma unroll 1
-  for (int b0 = 0; b0 < SV_VPT; b0 += SV_BATCH) {
-    // phase 1: every global load of the batch (parameters of tile tu, or
-    // grads and momentum of tile tg) before any is used
-    float pv[SV_BATCH][8], g[SV_BATCH][8], m[SV_BATCH][8];
-    bool uok[SV_BATCH], ufull[SV_BATCH], fast[SV_BATCH];
-#pragma unroll
-    for (int k = 0; k < SV_BATCH; ++k) {
-      const int v = (b0 + k) * NT + tq;
-      const int i = v / SV_VPR, j0 = (v % SV_VPR) * 8;
-      if constexpr (UNT) {
-        const int64_t pr = (int64_t)U.r * tile_h + i, pc = (int64_t)U.c * tile_w + j0;
-        const int64_t ou = pr * U.P->ld_upd + pc;
-        uok[k] = i < tile_h && j0 < tile_w && pr < U.P->h && pc < U.P->w;
-        ufull[k] = uok[k] && j0 + 8 <= tile_w && pc + 8 <= U.P->w && aligned16<PDT>(U.P->update, ou);
-        if (ufull[k]) load8<PDT>(U.P->update, ou, pv[k]);
-      }
-      if constexpr (GAT) {
-        const int64_t pr = (int64_t)G.r * tile_h + i, pc = (int64_t)G.c * tile_w + j0;
-        const int64_t og = pr * G.P->ld_grad + pc, om = pr * G.P->ld_mom + pc;
-        fast[k] = i < tile_h && pr < G.P->h && j0 + 8 <= tile_w && pc + 8 <= G.P->w &&
-                  aligned16<DT>(G.P->grad, og) && (!has_mom || aligned16<DT>(G.P->momentum, om));
-        if (fast[k]) {
-          load8<DT>(G.P->grad, og, g[k]);
-          if (has_mom) load8<DT>(G.P->momentum, om, m[k]);
-        }
-      }
-    }
-    // phase 2: the untile reads X' of vector v, or the gather writes it
-#pragma unroll
-    for (int k = 0; k < SV_BATCH; ++k) {
-      const int v = (b0 + k) * NT + tq;
-      const int i = v / SV_VPR, j0 = (v % SV_VPR) * 8;
-      lds_u32x4* const px = reinterpret_cast<lds_u32x4*>(X + lds_pos(i, v % SV_VPR, XCH));
-      if constexpr (UNT) {
-        if (uok[k]) {
-          const u32x4_t w = *px;
-          float y[8];
-#pragma unroll
-          for (int e2 = 0; e2 < 4; ++e2) {
-            y[2 * e2] = sc * bf16_to_f32(w[e2] & 0xffffu);
-            y[2 * e2 + 1] = sc * __uint_as_float(w[e2] & 0xffff0000u);
-          }
-          const int64_t pr = (int64_t)U.r * tile_h + i, pc = (int64_t)U.c * tile_w + j0;
-          const int64_t ou = pr * U.P->ld_upd + pc;
-          if (ufull[k]) {  // put8<true>'s full form, its load issued above
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              pv[k][e] = __builtin_fmaf(alpha, round_to<PDT>(y[e]), round_to<PDT>(pv[k][e] * s));
-            store8<PDT>(U.P->update, ou, pv[k]);
-          } else {
-            const int valid = (int)min<int64_t>(min(8, tile_w - j0), U.P->w - pc);
-            put8<true, PDT>(*U.P, ou, y, false, valid, sa);
-          }
-        }
-      }
-      if constexpr (GAT) {
-        const int64_t pr = (int64_t)G.r * tile_h + i, pc = (int64_t)G.c * tile_w + j0;
-        const int64_t og = pr * G.P->ld_grad + pc, om = pr * G.P->ld_mom + pc;
-        float x[8];
-        if (fast[k]) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] = momentum_elem<DT>(g[k][e], &m[k][e], mu, nesterov, has_mom);
-          if (has_mom) store8<DT>(G.P->momentum, om, m[k]);
-        } else {
-          const bool row_ok = i < tile_h && pr < G.P->h;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            x[e] = 0.f;
-            if (row_ok && j0 + e < tile_w && pc + e < G.P->w) {
-              const float gv = load_elem<DT>(G.P->grad, og + e);
-              float mv = has_mom ? load_elem<DT>(G.P->momentum, om + e) : 0.f;
-              x[e] = momentum_elem<DT>(gv, &mv, mu, nesterov, has_mom);
-              if (has_mom) store_elem<DT>(G.P->momentum, om + e, mv);
-            }
-          }
-        }
-        uint32_t h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          h[e] = f32_to_bf16(x[e]);
-          const float f = bf16_to_f32(h[e]);
-          ssq = fmaf(f, f, ssq);
-        }
-        *px = u32x4_t{pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
-      }
-    }
-  }
-  return ssq;
-}
-
+// (The untile issues all 8 of a thread's parameter loads before using any,
+// 8 VGPRs each; the gather 4 grad and momentum pairs, 16 VGPRs each: 8 would
+// spill.)
 template <int DT, int PDT>
 __global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* __restrict__ params, int n_params,
                                                          int64_t tile_begin, int64_t ntiles, int tile_h,
                                                          int tile_w, int steps, float ca, float cb, float cc,
                                                          float eps, int round_once,
                                                          const float* __restrict__ sa) {
-  constexpr int XCH = SV_N / 8;
-  __shared__ __attribute__((aligned(16))) uint8_t sx_raw[M * SV_N * 2];
-  __shared__ __attribute__((aligned(16))) uint8_t sa_raw[TRI_BYTES];
+  constexpr int XCH = M / 8;
+  __shared__ __attribute__((aligned(16))) uint8_t sx_raw[M * M * 2];
+  __shared__ __attribute__((aligned(16))) uint8_t sa_raw[tri_bytes(4)];
   __shared__ float red[NT / 64];
   __shared__ float s_inv;
   lds_u8* const X = (lds_u8*)sx_raw;
@@ -614,7 +421,8 @@ __global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* 
 
   const int64_t tt = blockIdx.x;  // the grid has one workgroup per tile
   if (tt >= ntiles) return;
-  const float ssq = step_io<DT, PDT, false, true>(params, n_params, X, 0, tile_begin + tt, tile_h, tile_w, sa);
+  const float ssq =
+      step_io<M, NT, DT, PDT, false, true, 4>(params, n_params, X, 0, tile_begin + tt, tile_h, tile_w, sa, 0);
   // ---- normaliser (the gather's block sum, then tile_scale), X0 in place ----------
   const float sum = block_sum<NT>(ssq, red);
   if (threadIdx.x == 0) s_inv = 1.0f / (sqrtf(0.f + sum) + eps);
@@ -622,9 +430,9 @@ __global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* 
   const float inv = s_inv;
   const int ts = opaque_lane((int)threadIdx.x);
 #pragma unroll
-  for (int k = 0; k < SV_VPT; ++k) {
+  for (int k = 0; k < M * XCH / NT; ++k) {
     const int v = k * NT + ts;
-    lds_u32x4* const px = reinterpret_cast<lds_u32x4*>(X + lds_pos(v / SV_VPR, v % SV_VPR, XCH));
+    lds_u32x4* const px = reinterpret_cast<lds_u32x4*>(X + lds_pos(v / XCH, v % XCH, XCH));
     *px = scale8(*px, inv);
   }
   __syncthreads();
@@ -632,7 +440,7 @@ __global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* 
   ns_iterations<1, 4>(X, A, lane, steps, ca, cb, cc, round_once);
 
   // ---- untile with WD/LR ----------------------------------------------------------
-  step_io<DT, PDT, true, false>(params, n_params, X, tile_begin + tt, 0, tile_h, tile_w, sa);
+  step_io<M, NT, DT, PDT, true, false, 8>(params, n_params, X, tile_begin + tt, 0, tile_h, tile_w, sa, 0);
 }
 
 int num_cus() {
