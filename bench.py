@@ -179,10 +179,10 @@ def time_ns_stage(opt, reps: int) -> float:
 
 
 def time_lds_step_stage(opt, reps: int) -> float | None:
-    """Average ms of the step's LDS-resident launches (himuon_lds_step, one
-    per chunk: momentum to WD/LR) over every group that runs them; None when
-    no group does."""
-    groups = [g for g in opt._groups if opt._fuse_lds_step and g["tiles"].lds_step_ok()]
+    """Average ms of the step's one-launch chunks (himuon_lds_step or
+    himuon_reg_step: momentum to WD/LR) over every group that runs them; None
+    when no group does."""
+    groups = [g for g in opt._groups if opt._fuse_lds_step and g["tiles"].whole_step()]
     if not groups:
         return None
 
@@ -190,7 +190,7 @@ def time_lds_step_stage(opt, reps: int) -> float | None:
         for g in groups:
             ofs = 0
             for c in g["chunks"]:
-                g["tiles"].lds_step(ofs, c, g["steps"], opt._lrwd)
+                g["tiles"].whole_step()(ofs, c, g["steps"], opt._lrwd)
                 ofs += c
 
     return _event_loop(run, reps)
@@ -233,14 +233,15 @@ def time_dominant_kernel(opt, reps: int) -> dict:
     grp = g["tiles"]
     fam = ns_family(grp.mp, grp.np)
     n = min(g["sub_batch"], grp.n_tiles)
-    if opt._fuse_lds_step and grp.lds_step_ok():
-        # the whole step of n tiles in one launch (himuon_lds_step): the
-        # momentum buffers and parameters of those tiles are read and written
-        # once each, the grads read once
-        ms = _event_loop(lambda: grp.lds_step(0, n, g["steps"], opt._lrwd), reps)
+    whole_step = grp.whole_step() if opt._fuse_lds_step else None
+    if whole_step:
+        # the whole step of n tiles in one launch (himuon_lds_step,
+        # himuon_reg_step): the momentum buffers and parameters of those tiles
+        # are read and written once each, the grads read once
+        ms = _event_loop(lambda: whole_step(0, n, g["steps"], opt._lrwd), reps)
         gb = torch.empty(0, dtype=grp.dtype).element_size()
         pb = torch.empty(0, dtype=grp.upd_dtype).element_size()
-        return {"kernel": "lds_step_kernel", "family": "lds_step", "launch_tiles": n, "launch_ms": ms,
+        return {"kernel": "lds_step_kernel" if grp.mp == 128 else "reg_step_kernel", "family": "lds_step", "launch_tiles": n, "launch_ms": ms,
                 "flops_per_launch": float(ns_flops(grp.m, grp.n)) * n,
                 "bytes_per_launch": float(_tile_elements(grp, n)) * (3 * gb + 2 * pb)}
     m, nn = grp.mp, grp.np
@@ -332,7 +333,7 @@ def time_ns_untile_stage(opt, reps: int) -> float | None:
     stream; each rep re-gathers first (untimed). None when no group takes
     the fused path (ns5_ms + untile_ms then cover the same work)."""
     groups = [g for g in opt._groups
-              if not (opt._fuse_lds_step and g["tiles"].lds_step_ok())]
+              if not (opt._fuse_lds_step and g["tiles"].whole_step())]
     if not any(opt._fuse_ns_untile and g["tiles"].ns_untile_ok(g["steps"]) for g in groups):
         return None
     s = torch.cuda.current_stream()
@@ -1063,14 +1064,14 @@ def main():
         # NS iteration of 512 x 512 buckets (ns5_ms and untile_ms above time
         # the two launches that this replaces)
         "ns5_untile_fused_ms": None if nsu_ms is None else round(nsu_ms, 3),
-        # 128 x 128-tile buckets run the whole step as one LDS-resident launch
+        # 128 x 128 and 256 x 256-tile buckets run the whole step as one launch
         # per chunk; ns5/gather/untile above then time the launches it replaces
         "lds_step_ms": None if lds_step_ms is None else round(lds_step_ms, 3),
         "apply_ms": round(apply_ms, 3),
         "apply_gbs": None if fused else round((2 * pb + ub) * n_el / (apply_ms * 1e-3) / 1e9, 1),
         "update_dtype": None if fused else str(opt._groups[0]["tiles"].upd_dtype).replace("torch.", ""),
-        "ns5_stage_kernels": ("step: lds_step_kernel (momentum, gather, normaliser, NS5 and untile with "
-                              "WD/LR of 128x128 tiles in one launch per chunk)" if lds_step_ms is not None
+        "ns5_stage_kernels": ("step: lds_step_kernel or reg_step_kernel (momentum, gather, normaliser, NS5 and untile "
+                              "with WD/LR of 128x128 or 256x256 tiles in one launch per chunk)" if lds_step_ms is not None
                               else "; ".join(NS_KERNELS[f] for f in fams)),
         # the dominant kernel, one launch on one sub-batch (HIP events)
         "roofline": kernel_roofline(args.config, dk),

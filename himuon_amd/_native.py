@@ -18,7 +18,7 @@ import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libhimuon_hip.so"
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 NS_ALIGN = 128
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 # Operand dtypes of the typed stage products (himuon_*_typed): the above and fp8 e5m2.
@@ -136,6 +136,8 @@ _SIGNATURES = {
     "himuon_bmm_add_typed": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_int,
                                      c_void_p]),
     "himuon_lds_step": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float,
+                                c_float, c_float, c_float, c_int, c_void_p, c_void_p]),
+    "himuon_reg_step": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float,
                                 c_float, c_float, c_float, c_int, c_void_p, c_void_p]),
     "himuon_ns5_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_float,
                                    c_float, c_int, c_void_p]),
@@ -440,19 +442,39 @@ def lds_step_supported(tile_h: int, tile_w: int, dtype, param_dtype) -> bool:
             and param_dtype in (torch.float32, torch.bfloat16))
 
 
-def lds_step(desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype, steps, scale_alpha,
-             round_once=False, coeffs=(NS_A, NS_B, NS_C), eps=NS_EPS):
-    """Momentum, gather, normaliser, NS5 and the untile with WD/LR for bucket
-    tiles tile_begin .. + n_tiles - 1 in one launch (128 x 128 NS tiles)."""
+def reg_step_supported(tile_h: int, tile_w: int, dtype, param_dtype) -> bool:
+    """Buckets himuon_reg_step takes: 256 x 256 NS tiles without transpose,
+    fp32/bf16 grads and parameters."""
+    return (128 < tile_h <= tile_w <= 256 and dtype in (torch.float32, torch.bfloat16)
+            and param_dtype in (torch.float32, torch.bfloat16))
+
+
+def _tile_step(name, desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype, steps,
+               scale_alpha, round_once, coeffs, eps):
     a, b, c = coeffs
     _check(
-        load().himuon_lds_step(
+        getattr(load(), name)(
             desc_table.data_ptr(), n_params, tile_begin, n_tiles, tile_h, tile_w, dtype_code(dtype),
             dtype_code(param_dtype), steps, a, b, c, eps, NS_ROUND_ONCE if round_once else 0,
             scale_alpha.data_ptr(), _stream(),
         ),
-        "himuon_lds_step",
+        name,
     )
+
+
+def lds_step(desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype, steps, scale_alpha,
+             round_once=False, coeffs=(NS_A, NS_B, NS_C), eps=NS_EPS):
+    """Momentum, gather, normaliser, NS5 and the untile with WD/LR for bucket
+    tiles tile_begin .. + n_tiles - 1 in one launch (128 x 128 NS tiles)."""
+    _tile_step("himuon_lds_step", desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype,
+               steps, scale_alpha, round_once, coeffs, eps)
+
+
+def reg_step(desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype, steps, scale_alpha,
+             round_once=False, coeffs=(NS_A, NS_B, NS_C), eps=NS_EPS):
+    """lds_step for 256 x 256 NS tiles."""
+    _tile_step("himuon_reg_step", desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype,
+               steps, scale_alpha, round_once, coeffs, eps)
 
 
 def untile(desc_table, n_params, n_tiles, tile_h, tile_w, mp, np_, dtype, tiles):

@@ -235,3 +235,9 @@ void ns5_lds_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int mp
 bool ns5_reg_supported(int mp, int np);
 void ns5_reg_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int steps, float a, float b, float c,
                  bool round_once, hipStream_t s);
+// The whole step of a bucket of NS tiles with 128 < tile_h <= tile_w <= 256
+// in one launch (ns5_reg.hip), as lds_step_run for 128 x 128.
+bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype);
+void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
+                  int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
+                  bool round_once, const float* sa, hipStream_t s);

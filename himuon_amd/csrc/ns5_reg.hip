@@ -41,6 +41,9 @@ constexpr int NT = 512;         // threads: eight waves
 constexpr int CH = T / 8;       // 16-byte chunks per row
 constexpr int KS = T / 16;      // MFMA k-steps
 constexpr int LDS_BYTES = T * T * 2;
+// 8-element vectors whose loads are in flight per thread in the step's memory
+// passes (grad and momentum: 16 VGPRs each, parameters: 8 or 4)
+constexpr int GAT_BATCH = 4, UNT_BATCH = 8;
 
 // Wave W's share of a Gram product: row tiles ROW[0 .. 3] as fragments, tile k
 // (k < NTL) being (row tile ROW[I[k]], column tile ROW[J[k]]), row >= column.
@@ -301,7 +304,80 @@ __global__ __launch_bounds__(NT, 1) void ns5_reg_kernel(const uint16_t* x, uint1
   }
 }
 
+// The whole optimizer step of a bucket of 256 x 256 NS tiles in one launch
+// (tiles not transposed), as lds_step_kernel does it for 128 x 128: momentum
+// and gather into LDS, the normaliser, the iterations, the untile with WD/LR.
+// Per-element arithmetic and the order of the sum of squares are the separate
+// kernels' (tile_step.h), so the step is bit-identical to gather ->
+// tile_scale -> NS5 -> untile_apply. It saves the tile buffer's write and read
+// and two reads of it by other launches; one workgroup fits a CU, so a tile's
+// memory passes overlap only with the iterations of other CUs' tiles, which
+// the one-tile-per-workgroup grid lets drift out of phase. Qwen3-0.6B set
+// (6,720 tiles, bf16 parameters, fp32 grads): 3.53-3.54 ms a step against 4.24
+// with the separate gather and untile launches; one 1024 x 1024 matrix (16
+// tiles) 0.108 against 0.110 ms. 2 or 8 vectors in the gather's load batch and
+// 4 in the untile's: within 0.6 %.
+template <int DT, int PDT>
+__global__ __launch_bounds__(NT, 1) void reg_step_kernel(const HimuonParamDesc* __restrict__ params, int n_params,
+                                                         int64_t tile_begin, int64_t ntiles, int tile_h, int tile_w,
+                                                         int steps, float ca, float cb, float cc, float eps,
+                                                         int round_once, const float* __restrict__ sa) {
+  __shared__ __attribute__((aligned(16))) uint8_t raw[LDS_BYTES];
+  __shared__ float red[2][NT / 64];
+  __shared__ float s_inv;
+  lds_u8* const L = (lds_u8*)raw;
+  const int64_t tt = blockIdx.x;
+  if (tt >= ntiles) return;
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) {
+    const float w = wave_sum(
+        step_io<T, NT, DT, PDT, false, true, GAT_BATCH>(params, n_params, L, 0, tile_begin + tt, tile_h, tile_w, sa, s));
+    if ((threadIdx.x & 63) == 0) red[s][threadIdx.x >> 6] = w;
+  }
+  __syncthreads();  // the tile and the waves' sums are in
+  if (threadIdx.x == 0) {
+    // slab 2 s + g: waves 4 g .. + 3 of pass s; slabs in order, as tile_scale adds them
+    float sum = 0.f;
+    for (int q = 0; q < 4; ++q) {
+      float p = 0.f;
+      for (int i = 0; i < 4; ++i) p += red[q >> 1][4 * (q & 1) + i];
+      sum += p;
+    }
+    s_inv = 1.0f / (sqrtf(sum) + eps);
+  }
+  __syncthreads();
+  ns_iterations(L, s_inv, steps, ca, cb, cc, round_once);
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s)
+    step_io<T, NT, DT, PDT, true, false, UNT_BATCH>(params, n_params, L, tile_begin + tt, 0, tile_h, tile_w, sa, s);
+}
+
 }  // namespace
+
+bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype) {
+  return tile_h > T / 2 && tile_h <= tile_w && tile_w <= T &&
+         (dtype == HIMUON_DTYPE_F32 || dtype == HIMUON_DTYPE_BF16) &&
+         (param_dtype == HIMUON_DTYPE_F32 || param_dtype == HIMUON_DTYPE_BF16);
+}
+
+void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
+                  int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
+                  bool round_once, const float* sa, hipStream_t s) {
+  for (int64_t off = 0; off < cnt; off += (int64_t)1 << 30) {
+    const int64_t n = std::min<int64_t>(cnt - off, (int64_t)1 << 30);
+    const auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(NT), 0, s, params, n_params, tile_begin + off, n, tile_h,
+                         tile_w, steps, a, b, c, eps, round_once ? 1 : 0, sa);
+    };
+    if (dtype == HIMUON_DTYPE_F32) {
+      if (param_dtype == HIMUON_DTYPE_F32) run(reg_step_kernel<HIMUON_DTYPE_F32, HIMUON_DTYPE_F32>);
+      else run(reg_step_kernel<HIMUON_DTYPE_F32, HIMUON_DTYPE_BF16>);
+    } else {
+      if (param_dtype == HIMUON_DTYPE_F32) run(reg_step_kernel<HIMUON_DTYPE_BF16, HIMUON_DTYPE_F32>);
+      else run(reg_step_kernel<HIMUON_DTYPE_BF16, HIMUON_DTYPE_BF16>);
+    }
+  }
+}
 
 bool ns5_reg_supported(int mp, int np) { return mp == T && np == T; }
 

@@ -90,8 +90,9 @@ class TileGroup:
         self.tile0 = [sum(counts[:i]) for i in range(len(counts))]
         self.n_tiles = sum(counts)
         self.ppt = nat.gather_partials_per_tile(self.tile_h, self.tile_w, self.mp, self.np)
-        # NS tile buffers, allocated on first use: a group whose step runs in
-        # LDS (lds_step) never needs them.
+        # NS tile buffers, allocated on first use: a group whose step runs on
+        # chip (lds_step, reg_step) never needs them.
+        self._tiles = None
         self._bufs = None
         self.updates = [] if self.fused else [torch.empty(g.shape, device=device, dtype=self.upd_dtype) for g in grads]
         self.upd_scales = list(upd_scales)
@@ -101,13 +102,19 @@ class TileGroup:
         self.bind(grads, moms, mus, nesterovs)
 
     # -- NS tile buffers ------------------------------------------------------
+    def tile_buffer(self) -> torch.Tensor:
+        """The NS tile buffer alone, without the others that NS launches need."""
+        if self._tiles is None:
+            self._tiles = torch.empty((self.n_tiles, self.mp, self.np), device=self.device, dtype=torch.bfloat16)
+        return self._tiles
+
     def _buffers(self):
         if self._bufs is None:
-            shape = (self.n_tiles, self.mp, self.np)
             # X ping-pongs between tiles and alt through the NS iterations.
+            tiles = self.tile_buffer()
             self._bufs = (
-                torch.empty(shape, device=self.device, dtype=torch.bfloat16),
-                torch.empty(shape, device=self.device, dtype=torch.bfloat16),
+                tiles,
+                torch.empty_like(tiles),
                 torch.empty((self.n_tiles, self.ppt), device=self.device, dtype=torch.float32),
                 torch.empty((self.n_tiles,), device=self.device, dtype=torch.float32),
             )
@@ -252,6 +259,25 @@ class TileGroup:
             return
         nat.lds_step(self.desc, len(self.tile0), start, count, self.tile_h, self.tile_w, self.dtype,
                      self.upd_dtype, steps, scale_alpha, round_once=self.round_once)
+
+    def reg_step_ok(self) -> bool:
+        """True when the whole step of this group runs as one launch per chunk
+        on 256 x 256 NS tiles (himuon_reg_step): fused mode, family "auto",
+        no transpose, fp32/bf16 grads and parameters."""
+        return (self.fused and self.ns_family == "auto"
+                and nat.reg_step_supported(self.tile_h, self.tile_w, self.dtype, self.upd_dtype))
+
+    def reg_step(self, start: int, count: int, steps: int, scale_alpha: torch.Tensor) -> None:
+        """lds_step() for 256 x 256 NS tiles."""
+        if count <= 0:
+            return
+        nat.reg_step(self.desc, len(self.tile0), start, count, self.tile_h, self.tile_w, self.dtype,
+                     self.upd_dtype, steps, scale_alpha, round_once=self.round_once)
+
+    def whole_step(self):
+        """lds_step or reg_step, the launch that runs the group's whole step
+        (momentum to WD/LR) on one chunk, or None when neither takes it."""
+        return self.lds_step if self.lds_step_ok() else self.reg_step if self.reg_step_ok() else None
 
     def result(self, steps: int) -> torch.Tensor:
         """Buffer holding the NS output after `steps` iterations."""

@@ -65,9 +65,10 @@ class HiMuon(Optimizer):
     # when their parameters allow it; False keeps update tensors and the
     # separate WD/LR pass for every bucket (same parameters, bit for bit).
     _fuse_untile: bool = True
-    # Such buckets on 128 x 128 NS tiles run the whole step (momentum to
-    # WD/LR) as one LDS-resident launch per chunk (himuon_lds_step); False
-    # keeps the gather / NS / untile launches (same results, bit for bit).
+    # Such buckets on 128 x 128 and 256 x 256 NS tiles run the whole step
+    # (momentum to WD/LR) as one launch per chunk with each tile held on chip
+    # (himuon_lds_step, himuon_reg_step); False keeps the gather / NS / untile
+    # launches (same results, bit for bit).
     _fuse_lds_step: bool = True
     # fused-untile buckets of 512 x 512 tiles: the untile with WD/LR runs
     # inside the last NS iteration (himuon_ns5_untile_apply)
@@ -566,7 +567,9 @@ class HiMuon(Optimizer):
                 # A bucket whose step runs in LDS (himuon_lds_step: 128 x 128
                 # NS tiles) has no tile buffer at all, so it registers none:
                 # its tiles exist only in LDS, one workgroup at a time.
-                self._concat_buffers[bucket["bucket_key"]] = grp.tiles
+                # (256 x 256 tiles on himuon_reg_step: the buffer exists, unused)
+                reg = self._fuse_lds_step and grp.reg_step_ok()
+                self._concat_buffers[bucket["bucket_key"]] = grp.tile_buffer() if reg else grp.tiles
             out.append(
                 {
                     "tiles": grp,
@@ -745,9 +748,9 @@ class HiMuon(Optimizer):
         total_B = 0
         for g in groups:
             grp: TileGroup = g["tiles"]
-            lds = self._fuse_lds_step and grp.lds_step_ok()
-            nsu = not lds and self._fuse_ns_untile and grp.ns_untile_ok(g["steps"])
-            if not lds:
+            whole_step = grp.whole_step() if self._fuse_lds_step else None
+            nsu = whole_step is None and self._fuse_ns_untile and grp.ns_untile_ok(g["steps"])
+            if whole_step is None:
                 grp.gather()
             ofs = 0
             for c in g["chunks"]:
@@ -755,8 +758,8 @@ class HiMuon(Optimizer):
                     ev0 = torch.cuda.Event(enable_timing=True)
                     ev1 = torch.cuda.Event(enable_timing=True)
                     ev0.record()
-                if lds:
-                    grp.lds_step(ofs, c, g["steps"], self._lrwd)
+                if whole_step is not None:
+                    whole_step(ofs, c, g["steps"], self._lrwd)
                 elif nsu:
                     grp.ns_untile(ofs, c, g["steps"], self._workspace, g["sub_batch"], self._lrwd)
                 else:
@@ -768,11 +771,11 @@ class HiMuon(Optimizer):
                 total_B += c
                 ofs += c
             if grp.fused:
-                # WD/LR applied by the untile itself (or by the LDS-resident
+                # WD/LR applied by the untile itself (or by the one-launch
                 # step, or inside the last NS iteration), from the (scale,
                 # alpha) table written before this step; the graph path still
                 # lists the parameters as pending (without an update tensor).
-                if not (lds or nsu):
+                if whole_step is None and not nsu:
                     grp.untile(g["steps"], self._lrwd)
                 if self._in_graph_region:
                     for (p, _), gi in zip(g["entries"], g["group_idx"]):

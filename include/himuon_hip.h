@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define HIMUON_ABI_VERSION 5
+#define HIMUON_ABI_VERSION 6
 
 /* Element type codes for gradients / momentum / updates. */
 #define HIMUON_DTYPE_F32 0
@@ -274,6 +274,17 @@ int himuon_ba_bmm_add(const uint16_t* a, const uint16_t* x, uint16_t* out,
  * and dtypes are an argument error.
  */
 int himuon_lds_step(const HimuonParamDesc* params_dev, int n_params,
+                    int64_t tile_begin, int64_t n_tiles, int tile_h,
+                    int tile_w, int dtype, int param_dtype, int steps,
+                    float a, float b, float c, float eps, int flags,
+                    const float* scale_alpha_dev, void* stream);
+
+/*
+ * himuon_lds_step for buckets of 256 x 256 NS tiles (128 < tile_h <= tile_w
+ * <= 256): the same arguments and results, each tile held in one workgroup's
+ * registers and LDS. Other geometries and dtypes are an argument error.
+ */
+int himuon_reg_step(const HimuonParamDesc* params_dev, int n_params,
                     int64_t tile_begin, int64_t n_tiles, int tile_h,
                     int tile_w, int dtype, int param_dtype, int steps,
                     float a, float b, float c, float eps, int flags,
