@@ -1,23 +1,19 @@
 // Batched quintic Newton-Schulz (NS5) on gfx950 bf16 MFMA, fp32 accumulation.
 //
 // Per NS tile (m x n, m <= n, zero padded to mp x np) and per iteration:
-//   A = bf16(X X^T)                      -> ns_gram_kernel (alpha=1, beta=0)
-//   B = bf16(c A A^T + b A)              -> ns_gram_kernel (alpha=c, beta=b)
-//   X = bf16(bf16(B X) + a X)            -> ns_apply_kernel
+//   A = bf16(X X^T)
+//   B = bf16(c A A^T + b A)
+//   X = bf16(bf16(B X) + a X)
 // following the rounding points of the reference kernels
 // (triton_kernels/XXT.py:55-75, ba_plus_cAA.py:58-85, fused_bmm_add.py:65-88,
-// ns5_smem.py:84-101). A and B are symmetric: the gram kernel computes only
-// the lower-triangular 128x128 blocks and stores each block twice (as itself
-// and mirrored), so both products cost half the dense FLOPs.
+// ns5_smem.py:84-101). A and B are symmetric: only their lower-triangular
+// blocks are computed, each stored twice (as itself and mirrored).
 //
 // Iteration 0 reads the raw bf16 tile and applies the per-tile Frobenius
-// normaliser while staging operands into LDS: X0 = bf16(x * inv[t])
+// normaliser as the operands enter: X0 = bf16(x * inv[t])
 // (himuon.py:242, ns5_smem.py:84-87).
 //
-// Block tile 128x128x64, 256 threads = 4 waves in a 2x2 grid, each wave owns a
-// 64x64 sub-block = 2x2 MFMA 32x32x16 tiles. Operands are double buffered in
-// LDS with register prefetch of the next K slab. Blocks are mapped to XCDs so
-// all blocks of one NS tile share an L2.
+// This file holds the C entry points and the choice of kernels for a geometry.
 #include <algorithm>
 #include <atomic>
 #include <mutex>
@@ -27,247 +23,7 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int kLd = BK + 8;  // padded LDS row pitch (elements) of k-contiguous operands
-
-HM_DEV f32x16_t mfma_32x32x16(u32x4_t a, u32x4_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
-// ---------------------------------------------------------------------------
-// C = bf16(alpha * S S^T + beta * S) for each tile; S is M x K (row pitch ldS),
-// C is M x M (row pitch ldC). Only blocks bi >= bj are computed; every block
-// is written at (bi, bj) and mirrored at (bj, bi), so C is exactly symmetric.
-// beta != 0 requires K == M (S square).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads, 2) void ns_gram_kernel(
-    const uint16_t* __restrict__ S, int64_t s_bs, int ldS, uint16_t* __restrict__ C,
-    int64_t c_bs, int ldC, const float* __restrict__ inv, int M, int K, int64_t ntiles,
-    float alpha, float beta) {
-  __shared__ __attribute__((aligned(16))) uint16_t sI[2][BM * kLd];
-  __shared__ __attribute__((aligned(16))) uint16_t sJ[2][BN * kLd];
-
-  const int nb = M / BM;
-  const int npairs = nb * (nb + 1) / 2;
-  const int64_t total = ntiles * npairs;
-  const int64_t item = xcd_item(total);
-  if (item >= total) return;
-  const int64_t tile = item / npairs;
-  const int p = (int)(item % npairs);
-  int bi = 0;
-  while ((bi + 1) * (bi + 2) / 2 <= p) ++bi;
-  const int bj = p - bi * (bi + 1) / 2;
-
-  const uint16_t* St = S + tile * s_bs;
-  const uint16_t* Si = St + (int64_t)bi * BM * ldS;
-  const uint16_t* Sj = St + (int64_t)bj * BN * ldS;
-  const bool scaled = inv != nullptr;
-  const float sc = scaled ? inv[tile] : 1.f;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = tid >> 3, lkv = (tid & 7) * 8;  // loader: rows lrow + 32q, k offset lkv
-
-  u32x4_t ra[4], rb[4];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = lrow + 32 * q;
-      ra[q] = *reinterpret_cast<const u32x4_t*>(Si + (int64_t)row * ldS + k0 + lkv);
-      rb[q] = *reinterpret_cast<const u32x4_t*>(Sj + (int64_t)row * ldS + k0 + lkv);
-    }
-  };
-  auto lstore = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = lrow + 32 * q;
-      u32x4_t a = ra[q], b = rb[q];
-      if (scaled) {
-        a = scale8(a, sc);
-        b = scale8(b, sc);
-      }
-      *reinterpret_cast<u32x4_t*>(&sI[buf][row * kLd + lkv]) = a;
-      *reinterpret_cast<u32x4_t*>(&sJ[buf][row * kLd + lkv]) = b;
-    }
-  };
-
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
-
-  const int nk = K / BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * BK);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int kk = ks * 16 + (lane >> 5) * 8;
-      u32x4_t a[2], b[2];
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-        a[mi] = *reinterpret_cast<const u32x4_t*>(
-            &sI[cur][(wm * 64 + mi * 32 + (lane & 31)) * kLd + kk]);
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni)
-        b[ni] = *reinterpret_cast<const u32x4_t*>(
-            &sJ[cur][(wn * 64 + ni * 32 + (lane & 31)) * kLd + kk]);
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = mfma_32x32x16(a[mi], b[ni], acc[mi][ni]);
-    }
-    if (kt + 1 < nk) lstore(cur ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue. MFMA 32x32 output layout: register r of lane l holds
-  // row 8*(r/4) + 4*(l/32) + r%4, column l%32.
-  uint16_t* Ct = C + tile * c_bs;
-  const bool offdiag = bi > bj;
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = bi * BM + wm * 64 + mi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int j = bj * BN + wn * 64 + ni * 32 + (lane & 31);
-        float v = alpha * acc[mi][ni][r];
-        if (beta != 0.f) {
-          float s = bf16_to_f32(St[(int64_t)i * ldS + j]);
-          if (scaled) s = round_bf16(s * sc);
-          v = fmaf(beta, s, v);
-        }
-        const uint16_t h = (uint16_t)f32_to_bf16(v);
-        if (offdiag || i >= j) Ct[(int64_t)i * ldC + j] = h;
-        if (offdiag || i > j) Ct[(int64_t)j * ldC + i] = h;
-      }
-}
-
-// ---------------------------------------------------------------------------
-// Y = bf16(bf16(Bm X) + a X) for each tile; Bm is M x M symmetric (pitch M),
-// X and Y are M x N (pitch N). X is the MFMA B operand with the contraction
-// along its rows, so each 4x8 register block of X is transposed into a
-// k-octet-major LDS layout sX[k/8][j][k%8] that serves 16-byte operand reads.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads, 2) void ns_apply_kernel(
-    const uint16_t* __restrict__ Bm, int64_t b_bs, const uint16_t* __restrict__ X, int64_t x_bs,
-    uint16_t* __restrict__ Y, int64_t y_bs, const float* __restrict__ inv, int M, int N,
-    int64_t ntiles, float a, int round_once) {
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * kLd];
-  __shared__ __attribute__((aligned(16))) uint16_t sX[2][(BK / 8) * BN * 8];
-
-  const int nbi = M / BM, nbj = N / BN;
-  const int blocks = nbi * nbj;
-  const int64_t total = ntiles * blocks;
-  const int64_t item = xcd_item(total);
-  if (item >= total) return;
-  const int64_t tile = item / blocks;
-  const int blk = (int)(item % blocks);
-  const int bi = blk / nbj, bj = blk % nbj;
-
-  const uint16_t* Ai = Bm + tile * b_bs + (int64_t)bi * BM * M;
-  const uint16_t* Xt = X + tile * x_bs;
-  const bool scaled = inv != nullptr;
-  const float sc = scaled ? inv[tile] : 1.f;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = tid >> 3, lkv = (tid & 7) * 8;    // Bm loader
-  const int xkq = tid >> 4, xjo = (tid & 15) * 8;    // X loader: rows 4*xkq..+3, cols xjo..+7
-
-  u32x4_t ra[4], rx[4];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = lrow + 32 * q;
-      ra[q] = *reinterpret_cast<const u32x4_t*>(Ai + (int64_t)row * M + k0 + lkv);
-    }
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr)
-      rx[rr] = *reinterpret_cast<const u32x4_t*>(Xt + (int64_t)(k0 + 4 * xkq + rr) * N +
-                                                 bj * BN + xjo);
-  };
-  auto lstore = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = lrow + 32 * q;
-      *reinterpret_cast<u32x4_t*>(&sA[buf][row * kLd + lkv]) = ra[q];
-    }
-    u32x4_t x[4];
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) x[rr] = scaled ? scale8(rx[rr], sc) : rx[rr];
-    uint16_t* base = &sX[buf][(xkq >> 1) * BN * 8 + (xkq & 1) * 4];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int w = e >> 1, h = e & 1;
-      u32x2_t d;
-      d[0] = pack2(half16(x[0][w], h), half16(x[1][w], h));
-      d[1] = pack2(half16(x[2][w], h), half16(x[3][w], h));
-      *reinterpret_cast<u32x2_t*>(base + (xjo + e) * 8) = d;
-    }
-  };
-
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
-
-  const int nk = M / BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * BK);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int kk = ks * 16 + (lane >> 5) * 8;
-      const int koct = ks * 2 + (lane >> 5);
-      u32x4_t av[2], bv[2];
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-        av[mi] = *reinterpret_cast<const u32x4_t*>(
-            &sA[cur][(wm * 64 + mi * 32 + (lane & 31)) * kLd + kk]);
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni)
-        bv[ni] = *reinterpret_cast<const u32x4_t*>(
-            &sX[cur][(koct * BN + wn * 64 + ni * 32 + (lane & 31)) * 8]);
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = mfma_32x32x16(av[mi], bv[ni], acc[mi][ni]);
-    }
-    if (kt + 1 < nk) lstore(cur ^ 1);
-    __syncthreads();
-  }
-
-  uint16_t* Yt = Y + tile * y_bs;
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = bi * BM + wm * 64 + mi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int j = bj * BN + wn * 64 + ni * 32 + (lane & 31);
-        float xv = bf16_to_f32(Xt[(int64_t)i * N + j]);
-        if (scaled) xv = round_bf16(xv * sc);
-        const float bx = round_once ? acc[mi][ni][r] : round_bf16(acc[mi][ni][r]);
-        Yt[(int64_t)i * N + j] = (uint16_t)f32_to_bf16(fmaf(a, xv, bx));
-      }
-}
+constexpr int BM = 128;  // edges are multiples of this
 
 // Y = bf16(X * inv[t]) (steps == 0) or a plain copy (inv == nullptr).
 __global__ __launch_bounds__(kThreads) void ns_scale_copy_kernel(const uint16_t* __restrict__ X,
@@ -329,7 +85,7 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   // 256 x 256 tiles the one that keeps X in registers (ns5_reg.hip: 16 tiles
   // 0.086 against 0.187 ms for the streamed products, 256 tiles 0.105 against
   // 0.34, 6,720 tiles 2.45-2.55 against 6.13-6.25 ms, same box); other tiles
-  // run the 128-block kernels below, which family BLOCK128 selects for every
+  // run the 128-block kernels (ns5_blk.hip), which family BLOCK128 selects for every
   // geometry.
   // 512 x 512 tiles run the first product on the stream kernels and the
   // other two fused (ns5_ba.hip); family STREAM3 keeps three stream kernels.
@@ -339,9 +95,6 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   const bool lds = ns5_lds_supported(mp, np) && !small;
   const bool ba = ns5_ba_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
   const bool reg = ns5_reg_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
-  const int nb = mp / BM;
-  const int npairs = nb * (nb + 1) / 2;
-  const int apply_blocks = (mp / BM) * (np / BN);
 
   for (int64_t s0 = 0; s0 < n_tiles; s0 += sb) {
     const int64_t cnt = std::min<int64_t>(sb, n_tiles - s0);
@@ -366,15 +119,12 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
       uint16_t* nxt = y + o;
       const float* cur_inv = inv + s0;
       for (int it = 0; it < steps; ++it) {
-        hipLaunchKernelGGL(ns_gram_kernel, dim3((unsigned)xcd_grid(cnt * npairs)),
-                           dim3(kThreads), 0, s, cur, rect, np, wsA, sq, mp, cur_inv, mp, np,
-                           cnt, 1.0f, 0.0f);
-        hipLaunchKernelGGL(ns_gram_kernel, dim3((unsigned)xcd_grid(cnt * npairs)),
-                           dim3(kThreads), 0, s, wsA, sq, mp, wsB, sq, mp, nullptr, mp, mp, cnt,
-                           c, b);
-        hipLaunchKernelGGL(ns_apply_kernel, dim3((unsigned)xcd_grid(cnt * apply_blocks)),
-                           dim3(kThreads), 0, s, wsB, sq, cur, rect, nxt, rect, cur_inv, mp, np,
-                           cnt, a, round_once ? 1 : 0);
+        ns_blk_product(0, BlkArgs{cur, rect, np, cur, rect, np, nullptr, 0, 0, wsA, sq, mp, mp, mp, np, cnt, 1.f, 0.f,
+                                  0, cur_inv}, s);
+        ns_blk_product(1, BlkArgs{wsA, sq, mp, wsA, sq, mp, wsA, sq, mp, wsB, sq, mp, mp, mp, mp, cnt, c, b, 0,
+                                  nullptr}, s);
+        ns_blk_product(2, BlkArgs{wsB, sq, mp, cur, rect, np, cur, rect, np, nxt, rect, np, mp, np, mp, cnt, 1.f, a,
+                                  round_once ? 1 : 0, cur_inv}, s);
         const uint16_t* t = cur;
         cur = nxt;
         nxt = const_cast<uint16_t*>(t);
@@ -534,9 +284,7 @@ extern "C" int himuon_xxt(const uint16_t* x, uint16_t* out, int64_t batch, int M
   if (family == HIMUON_NS_FAMILY_AUTO && M % 256 == 0 && K % 256 == 0) {
     ns_stream_product(0, x, xs, K, x, xs, K, nullptr, 0, 0, out, os, M, M, M, K, batch, 1.f, 0.f, false, s);
   } else {
-    const int nb = M / BM;
-    hipLaunchKernelGGL(ns_gram_kernel, dim3((unsigned)xcd_grid(batch * (nb * (nb + 1) / 2))), dim3(kThreads), 0,
-                       s, x, xs, K, out, os, M, nullptr, M, K, batch, 1.0f, 0.0f);
+    ns_blk_product(0, BlkArgs{x, xs, K, x, xs, K, nullptr, 0, 0, out, os, M, M, M, K, batch, 1.f, 0.f, 0, nullptr}, s);
   }
   return (int)hipGetLastError();
 }
@@ -552,9 +300,7 @@ extern "C" int himuon_ba_plus_caa(const uint16_t* a, uint16_t* out, int64_t batc
   if (family == HIMUON_NS_FAMILY_AUTO && M % 256 == 0) {
     ns_stream_product(1, a, sq, M, a, sq, M, a, sq, M, out, sq, M, M, M, M, batch, alpha, beta, false, s);
   } else {
-    const int nb = M / BM;
-    hipLaunchKernelGGL(ns_gram_kernel, dim3((unsigned)xcd_grid(batch * (nb * (nb + 1) / 2))), dim3(kThreads), 0,
-                       s, a, sq, M, out, sq, M, nullptr, M, M, batch, alpha, beta);
+    ns_blk_product(1, BlkArgs{a, sq, M, a, sq, M, a, sq, M, out, sq, M, M, M, M, batch, alpha, beta, 0, nullptr}, s);
   }
   return (int)hipGetLastError();
 }
@@ -563,7 +309,7 @@ extern "C" int himuon_bmm_add(const uint16_t* b, const uint16_t* x, uint16_t* ou
                               float a, int flags, void* stream) {
   int family = 0;
   const bool round_once = (flags & HIMUON_NS_ROUND_ONCE) != 0;
-  if (!b || !x || !out || out == x || out == b || batch < 0 || M <= 0 || N <= 0 || M % BM || N % BN ||
+  if (!b || !x || !out || out == x || out == b || batch < 0 || M <= 0 || N <= 0 || M % BM || N % BM ||
       !stage_family(flags & ~HIMUON_NS_ROUND_ONCE, &family))
     return HIMUON_EINVAL;
   if (batch == 0) return 0;
@@ -572,8 +318,8 @@ extern "C" int himuon_bmm_add(const uint16_t* b, const uint16_t* x, uint16_t* ou
   if (family == HIMUON_NS_FAMILY_AUTO && M % 256 == 0 && N % 256 == 0) {
     ns_stream_product(2, b, sq, M, x, rect, N, x, rect, N, out, rect, N, M, N, M, batch, 1.f, a, round_once, s);
   } else {
-    hipLaunchKernelGGL(ns_apply_kernel, dim3((unsigned)xcd_grid(batch * (M / BM) * (N / BN))), dim3(kThreads), 0,
-                       s, b, sq, x, rect, out, rect, nullptr, M, N, batch, a, round_once ? 1 : 0);
+    ns_blk_product(2, BlkArgs{b, sq, M, x, rect, N, x, rect, N, out, rect, N, M, N, M, batch, 1.f, a,
+                              round_once ? 1 : 0, nullptr}, s);
   }
   return (int)hipGetLastError();
 }

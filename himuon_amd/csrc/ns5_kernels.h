@@ -241,3 +241,19 @@ bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype);
 void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
                   int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
                   bool round_once, const float* sa, hipStream_t s);
+// One NS product over a batch (modes, strides and rounding as
+// ns_stream_product) on 128 x 128 output blocks (ns5_blk.hip): M, N, K
+// multiples of 128. inv non-null (modes 0 and 2): X is the raw tile, X0 =
+// bf16(X inv[tile]).
+struct BlkArgs {
+  const uint16_t* P; int64_t p_bs; int ldp;
+  const uint16_t* Q; int64_t q_bs; int ldq;
+  const uint16_t* R; int64_t r_bs; int ldr;
+  uint16_t* C; int64_t c_bs; int ldc;
+  int M, N, K;
+  int64_t ntiles;
+  float alpha, beta;
+  int round_once;
+  const float* inv;
+};
+void ns_blk_product(int mode, const BlkArgs& g, hipStream_t s);
