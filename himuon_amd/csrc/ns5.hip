@@ -79,16 +79,16 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
 
   uint16_t* wsA = static_cast<uint16_t*>(workspace);
   uint16_t* wsB = wsA + sb * sq;
-  // Family AUTO: tiles whose padded edges are multiples of 256 run the
-  // persistent streamed-operand kernels (ns5_stream.hip); tiles with mp == 128
+  // Family AUTO: tiles whose padded edges are multiples of 256 run three
+  // products per iteration, each on the faster block size (ns_product); tiles with mp == 128
   // and np in {128, 256, 512} run the fused LDS-resident kernel (ns5_lds.hip),
   // 256 x 256 tiles the one that keeps X in registers (ns5_reg.hip: 16 tiles
   // 0.086 against 0.187 ms for the streamed products, 256 tiles 0.105 against
   // 0.34, 6,720 tiles 2.45-2.55 against 6.13-6.25 ms, same box); other tiles
   // run the 128-block kernels (ns5_blk.hip), which family BLOCK128 selects for every
   // geometry.
-  // 512 x 512 tiles run the first product on the stream kernels and the
-  // other two fused (ns5_ba.hip); family STREAM3 keeps three stream kernels.
+  // 512 x 512 tiles run the other two products fused (ns5_ba.hip); family
+  // STREAM3 runs three products on 256 x 256 blocks.
   const bool small = family == HIMUON_NS_FAMILY_BLOCK128;
   const bool few_rows = family == HIMUON_NS_FAMILY_AUTO && ns5_small_supported(rows, mp, np);
   const bool st = ns5_stream_supported(mp, np) && !small;
@@ -111,19 +111,19 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
         u = *untile;
         u.tile0 += s0;
       }
-      const int rc = ns5_stream_run(x + o, y + o, inv + s0, cnt, mp, np, steps, a, b, c, round_once, ba, wsA,
-                                    wsB, s, untile ? &u : nullptr);
+      const int rc = ns5_stream_run(x + o, y + o, inv + s0, cnt, mp, np, steps, a, b, c, round_once, ba,
+                                    family == HIMUON_NS_FAMILY_AUTO, wsA, wsB, s, untile ? &u : nullptr);
       if (rc) return rc;
     } else {
       const uint16_t* cur = x + o;
       uint16_t* nxt = y + o;
       const float* cur_inv = inv + s0;
       for (int it = 0; it < steps; ++it) {
-        ns_blk_product(0, BlkArgs{cur, rect, np, cur, rect, np, nullptr, 0, 0, wsA, sq, mp, mp, mp, np, cnt, 1.f, 0.f,
+        ns_blk_product(kGramA, NsProduct{cur, rect, np, cur, rect, np, nullptr, 0, 0, wsA, sq, mp, mp, mp, np, cnt, 1.f, 0.f,
                                   0, cur_inv}, s);
-        ns_blk_product(1, BlkArgs{wsA, sq, mp, wsA, sq, mp, wsA, sq, mp, wsB, sq, mp, mp, mp, mp, cnt, c, b, 0,
+        ns_blk_product(kGramB, NsProduct{wsA, sq, mp, wsA, sq, mp, wsA, sq, mp, wsB, sq, mp, mp, mp, mp, cnt, c, b, 0,
                                   nullptr}, s);
-        ns_blk_product(2, BlkArgs{wsB, sq, mp, cur, rect, np, cur, rect, np, nxt, rect, np, mp, np, mp, cnt, 1.f, a,
+        ns_blk_product(kApply, NsProduct{wsB, sq, mp, cur, rect, np, cur, rect, np, nxt, rect, np, mp, np, mp, cnt, 1.f, a,
                                   round_once ? 1 : 0, cur_inv}, s);
         const uint16_t* t = cur;
         cur = nxt;
@@ -260,10 +260,37 @@ extern "C" int himuon_ns5(uint16_t* x, uint16_t* y, const float* inv, int64_t n_
 }
 
 // ---------------------------------------------------------------------------
+// One product on the faster block size. Rounds of 256 x 256 blocks (one per
+// CU) cost the same whether full or not, so r = blocks / CUs of them cost
+// ceil(r); 64 x 64 and 128 x 128 blocks (two workgroups per CU) fill the chip
+// at any count at a lower rate, about 1.25 r for Apply and 1.3 r for a Gram
+// product; a Gram product on 128 x 128 blocks computes fewer elements (36 of 64
+// blocks against 10 of 16 at 1024), which makes it the faster one at any count
+// when M and K are large enough for its operand stream. Measured (us, smaller
+// blocks / 256 x 256): Apply of 28 1024 x 1024 (448 blocks) 76 / 66, of 7 1024 x
+// 2560 (280) 52 / 63, of one 1024 x 3072 (48) 15 / 30; GramA of 28 1024 x 1024
+// 43-48 / 63, of 56 1024 x 3072 229-235 / 264-302, of 4 4096 x 4096 326 / 340,
+// of one 1024 x 3072 24 / 75, of 128 512 x 512 (r = 1.5) 32 / 34, of 256 (r = 3)
+// 58 / 53, of 1,024 272 / 250, of 200 256 x 2048 (r = 0.78) 59 / 47.
+// ---------------------------------------------------------------------------
+void ns_product(int mode, const NsProduct& g, hipStream_t s) {
+  bool small = g.M % 256 || g.N % 256 || g.K % 256;
+  if (!small && mode != kApply && g.M >= 512 && g.K >= 1024) small = true;
+  if (!small) {
+    const int64_t nb = g.M / 256, cus = num_cus();
+    const int64_t items = g.ntiles * (mode == kApply ? nb * (g.N / 256) : nb * (nb + 1) / 2);
+    const double r = (double)items / cus;
+    small = (mode == kApply ? 1.25 : 1.3) * r < (double)((items + cus - 1) / cus);
+  }
+  if (small) ns_blk_product(mode, g, s);
+  else ns_stream_product(mode, g, s);
+}
+
+// ---------------------------------------------------------------------------
 // The three NS products one at a time (the reference's kernel entry points
 // XXT, ba_plus_cAA and fused_bmm_add): contiguous batches, dimensions
-// multiples of 128; edges that are multiples of 256 take the stream kernels
-// (unless the flags ask for the 128-block family), others the 128-block ones.
+// multiples of 128; on the faster block size, or with the 128-block family on
+// 64 x 64 or 128 x 128 blocks.
 // ---------------------------------------------------------------------------
 namespace {
 bool stage_family(int flags, int* family) {
@@ -281,11 +308,9 @@ extern "C" int himuon_xxt(const uint16_t* x, uint16_t* out, int64_t batch, int M
   if (batch == 0) return 0;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t xs = (int64_t)M * K, os = (int64_t)M * M;
-  if (family == HIMUON_NS_FAMILY_AUTO && M % 256 == 0 && K % 256 == 0) {
-    ns_stream_product(0, x, xs, K, x, xs, K, nullptr, 0, 0, out, os, M, M, M, K, batch, 1.f, 0.f, false, s);
-  } else {
-    ns_blk_product(0, BlkArgs{x, xs, K, x, xs, K, nullptr, 0, 0, out, os, M, M, M, K, batch, 1.f, 0.f, 0, nullptr}, s);
-  }
+  const NsProduct g{x, xs, K, x, xs, K, nullptr, 0, 0, out, os, M, M, M, K, batch, 1.f, 0.f, 0, nullptr};
+  if (family == HIMUON_NS_FAMILY_AUTO) ns_product(kGramA, g, s);
+  else ns_blk_product(kGramA, g, s);
   return (int)hipGetLastError();
 }
 
@@ -297,11 +322,9 @@ extern "C" int himuon_ba_plus_caa(const uint16_t* a, uint16_t* out, int64_t batc
   if (batch == 0) return 0;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t sq = (int64_t)M * M;
-  if (family == HIMUON_NS_FAMILY_AUTO && M % 256 == 0) {
-    ns_stream_product(1, a, sq, M, a, sq, M, a, sq, M, out, sq, M, M, M, M, batch, alpha, beta, false, s);
-  } else {
-    ns_blk_product(1, BlkArgs{a, sq, M, a, sq, M, a, sq, M, out, sq, M, M, M, M, batch, alpha, beta, 0, nullptr}, s);
-  }
+  const NsProduct g{a, sq, M, a, sq, M, a, sq, M, out, sq, M, M, M, M, batch, alpha, beta, 0, nullptr};
+  if (family == HIMUON_NS_FAMILY_AUTO) ns_product(kGramB, g, s);
+  else ns_blk_product(kGramB, g, s);
   return (int)hipGetLastError();
 }
 
@@ -315,12 +338,9 @@ extern "C" int himuon_bmm_add(const uint16_t* b, const uint16_t* x, uint16_t* ou
   if (batch == 0) return 0;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t sq = (int64_t)M * M, rect = (int64_t)M * N;
-  if (family == HIMUON_NS_FAMILY_AUTO && M % 256 == 0 && N % 256 == 0) {
-    ns_stream_product(2, b, sq, M, x, rect, N, x, rect, N, out, rect, N, M, N, M, batch, 1.f, a, round_once, s);
-  } else {
-    ns_blk_product(2, BlkArgs{b, sq, M, x, rect, N, x, rect, N, out, rect, N, M, N, M, batch, 1.f, a,
-                              round_once ? 1 : 0, nullptr}, s);
-  }
+  const NsProduct g{b, sq, M, x, rect, N, x, rect, N, out, rect, N, M, N, M, batch, 1.f, a, round_once ? 1 : 0, nullptr};
+  if (family == HIMUON_NS_FAMILY_AUTO) ns_product(kApply, g, s);
+  else ns_blk_product(kApply, g, s);
   return (int)hipGetLastError();
 }
 

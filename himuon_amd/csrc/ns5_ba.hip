@@ -721,14 +721,6 @@ __global__ __launch_bounds__(NTH, 1) void ns_ba_kernel(BaArgs g) {
   if (grp == 0) lds_barrier();
 }
 
-int num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  return n;
-}
-
 }  // namespace
 
 bool ns5_ba_supported(int mp, int np) { return mp == T && np == T; }

@@ -1,16 +1,16 @@
-// The three NS5 products on 128 x 128 output blocks, for NS tiles whose padded
-// edges are any multiples of 128:
+// The three NS5 products on 128 x 128 (BT = 128) or 64 x 64 output blocks, for NS
+// tiles whose padded edges are any multiples of 128:
 //
 //   GramA : C = A = bf16(X X^T)            P = Q = X (rows, K = n)   lower blocks + mirror
 //   GramB : C = B = bf16(c A A^T + b A)    P = Q = A (rows, K = m)   lower blocks + mirror
 //   Apply : C = X' = bf16(bf16(B X) + a X) P = B (rows, K = m), Q = X read as [k][j]
 // (ns5_smem.py:89-101, XXT.py:55-75, ba_plus_cAA.py:58-85, fused_bmm_add.py:65-88).
 //
-// One workgroup per block: 4 waves in 2 x 2, each 64 x 64 as 2 x 2
-// v_mfma_f32_32x32x16_bf16 tiles; two workgroups fit a CU (64 KiB of LDS
-// each), so one's MFMAs run while the other waits at a barrier, starts or
+// One workgroup per block: 4 waves in 2 x 2, each 64 x 64 as 2 x 2 (BT = 64: 32 x
+// 32 as one) v_mfma_f32_32x32x16_bf16 tiles; two workgroups fit a CU (64 KiB of
+// LDS each at BT = 128), so one's MFMAs run while the other waits at a barrier, starts or
 // stores. K advances in units of 64, straight from global memory into one of
-// two 32 KiB LDS slots, one unit ahead of the MFMAs; the epilogue operand R
+// two LDS slots (32 KiB each at BT = 128), one unit ahead of the MFMAs; the epilogue operand R
 // (A for GramB, X for Apply) follows as one more unit. The swapped MFMA
 // operand order and the mirrored store are those of the 256-block kernels
 // (ns5_stream.hip), and every element sums its k terms in one accumulator in
@@ -31,26 +31,33 @@
 namespace {
 
 constexpr int NT = 256;           // four waves
-constexpr int BT = 128;           // output block edge
 constexpr int BK = 64;            // K per unit
-constexpr int HALF = BT * BK * 2; // bytes of one operand's unit (16 KiB)
-constexpr int SLOT = 2 * HALF;
 
-enum { kGramA = 0, kGramB = 1, kApply = 2 };
-
-// Chunk swizzles (16-byte chunk index XOR a function of the row): row panels
-// of P / Q and the output staging (128-byte rows): 16 consecutive rows of one
-// chunk on distinct bank groups; the X panel of Apply (256-byte rows): 4 rows
-// x 4 chunks of a transposing read. R (256-byte rows): chunk ^ (row & 15).
-HM_DEV int swz_p(int r) { return (r >> 1) & 7; }
-HM_DEV int swz_x(int r) { return 4 * (r & 3); }
+// Chunk swizzles (16-byte chunk index XOR a function of the row): rows of 128
+// bytes (panels of P / Q; R and the output staging of some block edges): 16
+// consecutive rows of one chunk on distinct bank groups; likewise rows of 64
+// and 256 bytes; X panel rows of 256 or 128 bytes: the 4 rows x 4 chunks of a
+// transposing read.
+template <int BYTES>
+HM_DEV int swz(int r) {
+  return BYTES == 256 ? r & 15 : BYTES == 128 ? (r >> 1) & 7 : (r >> 2) & 3;
+}
+template <int BYTES>
+HM_DEV int swz_x(int r) {
+  return BYTES == 256 ? 4 * (r & 3) : 4 * ((r >> 1) & 1);
+}
 
 // One block. DIAG: Gram diagonal block, Q = P (one panel streamed), no mirror.
 // SC: the X operand is the raw tile, every X value replaced by bf16(x inv) as
 // it enters the computation.
-template <int MODE, bool SC, bool DIAG>
-HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj) {
+template <int MODE, bool SC, bool DIAG, int BT>
+HM_DEV void blk_item(const NsProduct& g, lds_u8* lds, int64_t tile, int bi, int bj) {
   constexpr bool kTr = MODE == kApply;
+  constexpr int HALF = BT * BK * 2, SLOT = 2 * HALF;  // bytes of an operand's unit, of a unit
+  constexpr int XB = BT * 2;                          // bytes per row of the X panel and of R
+  constexpr int XR = 1024 / XB, XC = XB / 16;         // their rows per 1 KiB, chunks per row
+  constexpr int PI = BT / 32;                         // panel loads per wave
+  constexpr int WT = BT / 64, WC = BT / 2;            // MFMA tiles, rows / columns per wave
   constexpr bool kR = MODE != kGramA;  // an epilogue operand
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -62,15 +69,15 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
 
   // ---- loaders: wave instruction n = 4 i + wave fills 1 KiB n of a panel ----------
   // Row panel: rows 8 n .. + 7; lane l lands at row 8 n + l / 8, position
-  // l % 8. X panel: k-rows 4 n .. + 3, lane l at row 4 n + l / 16, position l % 16.
-  const int prl = 8 * wave + (lane >> 3), pch = (lane & 7) ^ swz_p(prl);
+  // l % 8. X panel: XR k-rows, lane l at row XR n + l / XC, position l % XC.
+  const int prl = 8 * wave + (lane >> 3), pch = (lane & 7) ^ swz<128>(prl);
   const uint16_t* const psrc = g.P + tile * g.p_bs + (int64_t)(bi * BT + prl) * g.ldp + pch * 8;
   const uint16_t* qsrc;
   int64_t qstep, qunit;
   if constexpr (kTr) {
-    const int xr = 4 * wave + (lane >> 4);
-    qsrc = g.Q + tile * g.q_bs + (int64_t)xr * g.ldq + bj * BT + ((lane & 15) ^ swz_x(xr)) * 8;
-    qstep = 16 * (int64_t)g.ldq;
+    const int xr = XR * wave + lane / XC;
+    qsrc = g.Q + tile * g.q_bs + (int64_t)xr * g.ldq + bj * BT + ((lane & (XC - 1)) ^ swz_x<XB>(xr)) * 8;
+    qstep = 4 * XR * (int64_t)g.ldq;
     qunit = BK * (int64_t)g.ldq;
   } else {
     qsrc = g.Q + tile * g.q_bs + (int64_t)(bj * BT + prl) * g.ldq + pch * 8;
@@ -83,17 +90,17 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
     const uint32_t d = wdst + slot * SLOT;
     if (v < nk) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) dma16(psrc + i * pstep + v * BK, d + i * 4096);
+      for (int i = 0; i < PI; ++i) dma16(psrc + i * pstep + v * BK, d + i * 4096);
       if constexpr (!DIAG) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dma16(qsrc + i * qstep + v * qunit, d + HALF + i * 4096);
+        for (int i = 0; i < PI; ++i) dma16(qsrc + i * qstep + v * qunit, d + HALF + i * 4096);
       }
-    } else if constexpr (kR) {  // R: 128 rows of 256 bytes
+    } else if constexpr (kR) {  // R: the block's rows
       const uint16_t* const r0 = g.R + tile * g.r_bs + (int64_t)(bi * BT) * g.ldr + bj * BT;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = 4 * wave + (lane >> 4) + 16 * i;
-        dma16(r0 + (int64_t)r * g.ldr + ((lane & 15) ^ (r & 15)) * 8, d + i * 4096);
+      for (int i = 0; i < BT / XR / 4; ++i) {
+        const int r = XR * (4 * i + wave) + lane / XC;
+        dma16(r0 + (int64_t)r * g.ldr + ((lane & (XC - 1)) ^ swz<XB>(r)) * 8, d + i * 4096);
       }
     }
   };
@@ -104,7 +111,7 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
       asm volatile("" ::: "memory");  // the reads below follow the vmcnt wait
       lds_u8* const d = lds + slot * SLOT + wave * 1024 + 16 * lane;
 #pragma unroll
-      for (int i = 0; i < (DIAG ? 4 : 8); ++i) {
+      for (int i = 0; i < (DIAG ? PI : 2 * PI); ++i) {
         lds_u32x4* const p = reinterpret_cast<lds_u32x4*>(d + i * 4096);
         *p = scale8_rne(*p, xs);
       }
@@ -112,21 +119,21 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
   };
 
   // ---- fragments: fb rows i of P, fa rows (columns) j of Q --------------------------
-  const int sp = swz_p(l32);
-  const int prow = (wm * 64 + l32) * 128, qrow = (wn * 64 + l32) * 128;
+  const int sp = swz<128>(l32);
+  const int prow = (wm * WC + l32) * 128, qrow = (wn * WC + l32) * 128;
   const int tr_krow = tr_krow_of(lane), tr_col = tr_col_of(lane);
-  const uint32_t tr_lane = HALF + tr_krow * 256 + (tr_col & 7) * 2;
-  auto frags = [&](int slot, int ks, u32x4_t(&fa)[2], u32x4_t(&fb)[2]) {
+  const uint32_t tr_lane = HALF + tr_krow * XB + (tr_col & 7) * 2;
+  auto frags = [&](int slot, int ks, u32x4_t(&fa)[WT], u32x4_t(&fb)[WT]) {
     const lds_u8* s = lds + slot * SLOT;
     const int pos = ((2 * ks + hi) ^ sp) * 16;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) fb[t] = *reinterpret_cast<lds_cu32x4*>(s + prow + t * 4096 + pos);
+    for (int t = 0; t < WT; ++t) fb[t] = *reinterpret_cast<lds_cu32x4*>(s + prow + t * 4096 + pos);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < WT; ++t) {
       if constexpr (kTr) {  // (rows kr and kr + 4 have one swizzle)
-        const int ch = (wn * 8 + 4 * t + (tr_col >> 3)) ^ swz_x(tr_krow);
-        const uint32_t off = tr_lane + 16 * ks * 256 + ch * 16;
-        const u32x2_t l2 = read_tr(s, off), u2 = read_tr(s, off + 4 * 256);
+        const int ch = (wn * (WC / 8) + 4 * t + (tr_col >> 3)) ^ swz_x<XB>(tr_krow);
+        const uint32_t off = tr_lane + 16 * ks * XB + ch * 16;
+        const u32x2_t l2 = read_tr(s, off), u2 = read_tr(s, off + 4 * XB);
         fa[t] = u32x4_t{l2[0], l2[1], u2[0], u2[1]};
         if constexpr (SC) fa[t] = scale8_rne(fa[t], xs);
       } else {
@@ -134,18 +141,18 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
       }
     }
   };
-  f32x16_t acc[2][2];
+  f32x16_t acc[WT][WT];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < WT; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < WT; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
-  auto mma = [&](const u32x4_t(&fa)[2], const u32x4_t(&fb)[2]) {
+  auto mma = [&](const u32x4_t(&fa)[WT], const u32x4_t(&fb)[WT]) {
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj)
+    for (int tj = 0; tj < WT; ++tj)
 #pragma unroll
-      for (int ti = 0; ti < 2; ++ti) acc[tj][ti] = mfma(fa[tj], fb[ti], acc[tj][ti]);
+      for (int ti = 0; ti < WT; ++ti) acc[tj][ti] = mfma(fa[tj], fb[ti], acc[tj][ti]);
   };
 
   // ---- K loop ----------------------------------------------------------------------
@@ -159,7 +166,7 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
   scale_unit(0);
   lds_barrier();
   issue(1, 1);  // (nk >= 2)
-  u32x4_t fa0[2], fb0[2], fa1[2], fb1[2];
+  u32x4_t fa0[WT], fb0[WT], fa1[WT], fb1[WT];
   frags(0, 0, fa0, fb0);
 #pragma unroll 1
   for (int u = 0; u < nk; ++u) {
@@ -189,22 +196,22 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
   }
 
   // ---- epilogue --------------------------------------------------------------------
-  // out[ti][tj][q]: 4 bf16 of C[i][j .. j + 3], i = wm 64 + 32 ti + l32,
-  // j = wn 64 + 32 tj + 8 q + 4 hi (block-local).
-  u32x2_t out[2][2][4];
+  // out[ti][tj][q]: 4 bf16 of C[i][j .. j + 3], i = wm WC + 32 ti + l32,
+  // j = wn WC + 32 tj + 8 q + 4 hi (block-local).
+  u32x2_t out[WT][WT][4];
   wait_vm<0>();
   lds_barrier();  // R is in; every fragment read is done
 #pragma unroll
-  for (int ti = 0; ti < 2; ++ti)
+  for (int ti = 0; ti < WT; ++ti)
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj)
+    for (int tj = 0; tj < WT; ++tj)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         float y[4];
         if constexpr (kR) {
-          const int il = wm * 64 + 32 * ti + l32, ch = wn * 8 + 4 * tj + q;
-          const u32x2_t rv = *reinterpret_cast<lds_cu32x2*>(lds + (nk & 1) * SLOT + il * 256 +
-                                                            ((ch ^ (il & 15)) * 16) + hi * 8);
+          const int il = wm * WC + 32 * ti + l32, ch = wn * (WC / 8) + 4 * tj + q;
+          const u32x2_t rv = *reinterpret_cast<lds_cu32x2*>(lds + (nk & 1) * SLOT + il * XB +
+                                                            ((ch ^ swz<XB>(il)) * 16) + hi * 8);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             float x = bf16_to_f32(half16(rv[e >> 1], e & 1));
@@ -222,50 +229,51 @@ HM_DEV void blk_item(const BlkArgs& g, lds_u8* lds, int64_t tile, int bi, int bj
         out[ti][tj][q] = u32x2_t{pk_bf16(y[0], y[1]), pk_bf16(y[2], y[3])};
       }
   if constexpr (kR) lds_barrier();  // every R read is done
-  // Staging: each wave's 64 x 64 result in its own 8 KiB (LDS operations of a
-  // wave execute in order), then whole 128-byte rows per 8 lanes.
-  lds_u8* const W = lds + wave * 8192;
-  const int srow = lane >> 3, sch = lane & 7;
+  // Staging: each wave's WC x WC result in its own LDS (LDS operations of a
+  // wave execute in order), then whole rows, 16 bytes per lane.
+  constexpr int SB = WC * 2, SC16 = SB / 16, SR = 64 / SC16;  // row bytes, chunks, rows per store
+  lds_u8* const W = lds + wave * (WC * SB);
+  const int srow = lane / SC16, sch = lane % SC16;
   uint16_t* const Ct = g.C + tile * g.c_bs;
   auto store_rows = [&](uint16_t* dst) {
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      const int r = 8 * n + srow;
-      const u32x4_t v = *reinterpret_cast<lds_cu32x4*>(W + r * 128 + ((sch ^ swz_p(r)) * 16));
+    for (int n = 0; n < WC / SR; ++n) {
+      const int r = SR * n + srow;
+      const u32x4_t v = *reinterpret_cast<lds_cu32x4*>(W + r * SB + ((sch ^ swz<SB>(r)) * 16));
       *reinterpret_cast<u32x4_t*>(dst + (int64_t)r * g.ldc + sch * 8) = v;
     }
   };
 #pragma unroll
-  for (int ti = 0; ti < 2; ++ti)
+  for (int ti = 0; ti < WT; ++ti)
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj)
+    for (int tj = 0; tj < WT; ++tj)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int r = 32 * ti + l32, ch = 4 * tj + q;
-        *reinterpret_cast<lds_u32x2*>(W + r * 128 + ((ch ^ swz_p(r)) * 16) + hi * 8) = out[ti][tj][q];
+        *reinterpret_cast<lds_u32x2*>(W + r * SB + ((ch ^ swz<SB>(r)) * 16) + hi * 8) = out[ti][tj][q];
       }
-  store_rows(Ct + (int64_t)(bi * BT + wm * 64) * g.ldc + bj * BT + wn * 64);
+  store_rows(Ct + (int64_t)(bi * BT + wm * WC) * g.ldc + bj * BT + wn * WC);
   if constexpr (MODE != kApply && !DIAG) {
     // mirror: after the quad transpose lane (a = l32 / 4, k = l32 % 4) holds
     // C^T[j][i .. i + 3], j = 32 tj + 8 q + 4 hi + k, i = 32 ti + 4 a
     const int k = lane & 3, a = l32 >> 2;
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
+    for (int ti = 0; ti < WT; ++ti)
 #pragma unroll
-      for (int tj = 0; tj < 2; ++tj)
+      for (int tj = 0; tj < WT; ++tj)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int r = 32 * tj + 8 * q + 4 * hi + k, ch = 4 * ti + (a >> 1);
-          *reinterpret_cast<lds_u32x2*>(W + r * 128 + ((ch ^ swz_p(r)) * 16) + (a & 1) * 8) =
+          *reinterpret_cast<lds_u32x2*>(W + r * SB + ((ch ^ swz<SB>(r)) * 16) + (a & 1) * 8) =
               quad_transpose(out[ti][tj][q], k);
         }
-    store_rows(Ct + (int64_t)(bj * BT + wn * 64) * g.ldc + bi * BT + wm * 64);
+    store_rows(Ct + (int64_t)(bj * BT + wn * WC) * g.ldc + bi * BT + wm * WC);
   }
 }
 
-template <int MODE, bool SC>
-__global__ __launch_bounds__(NT, 2) void ns_blk_kernel(BlkArgs g) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * SLOT];
+template <int MODE, bool SC, int BT>
+__global__ __launch_bounds__(NT, 2) void ns_blk_kernel(NsProduct g) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[8 * BT * BK];
   const int nbi = g.M / BT, nbj = g.N / BT;
   const int per_tile = MODE == kApply ? nbi * nbj : nbi * (nbi + 1) / 2;
   const int64_t total = g.ntiles * per_tile;
@@ -274,30 +282,47 @@ __global__ __launch_bounds__(NT, 2) void ns_blk_kernel(BlkArgs g) {
   const int64_t tile = item / per_tile;
   const int p = (int)(item - tile * per_tile);
   if constexpr (MODE == kApply) {
-    blk_item<MODE, SC, false>(g, (lds_u8*)lds, tile, p / nbj, p % nbj);
+    blk_item<MODE, SC, false, BT>(g, (lds_u8*)lds, tile, p / nbj, p % nbj);
   } else {
     int bi = 0;
     while ((bi + 1) * (bi + 2) / 2 <= p) ++bi;
     const int bj = p - bi * (bi + 1) / 2;
-    if (bi == bj) blk_item<MODE, SC, true>(g, (lds_u8*)lds, tile, bi, bj);
-    else blk_item<MODE, SC, false>(g, (lds_u8*)lds, tile, bi, bj);
+    if (bi == bj) blk_item<MODE, SC, true, BT>(g, (lds_u8*)lds, tile, bi, bj);
+    else blk_item<MODE, SC, false, BT>(g, (lds_u8*)lds, tile, bi, bj);
   }
 }
 
-}  // namespace
-
-void ns_blk_product(int mode, const BlkArgs& g, hipStream_t s) {
+template <int BT>
+void launch(int mode, const NsProduct& g, hipStream_t s) {
   const int64_t nbi = g.M / BT, nbj = g.N / BT;
   const int64_t items = g.ntiles * (mode == kApply ? nbi * nbj : nbi * (nbi + 1) / 2);
   const dim3 grid((unsigned)xcd_grid(items)), block(NT);
   const bool sc = g.inv != nullptr;
   if (mode == kGramA) {
-    if (sc) hipLaunchKernelGGL((ns_blk_kernel<kGramA, true>), grid, block, 0, s, g);
-    else hipLaunchKernelGGL((ns_blk_kernel<kGramA, false>), grid, block, 0, s, g);
+    if (sc) hipLaunchKernelGGL((ns_blk_kernel<kGramA, true, BT>), grid, block, 0, s, g);
+    else hipLaunchKernelGGL((ns_blk_kernel<kGramA, false, BT>), grid, block, 0, s, g);
   } else if (mode == kGramB) {
-    hipLaunchKernelGGL((ns_blk_kernel<kGramB, false>), grid, block, 0, s, g);
+    hipLaunchKernelGGL((ns_blk_kernel<kGramB, false, BT>), grid, block, 0, s, g);
   } else {
-    if (sc) hipLaunchKernelGGL((ns_blk_kernel<kApply, true>), grid, block, 0, s, g);
-    else hipLaunchKernelGGL((ns_blk_kernel<kApply, false>), grid, block, 0, s, g);
+    if (sc) hipLaunchKernelGGL((ns_blk_kernel<kApply, true, BT>), grid, block, 0, s, g);
+    else hipLaunchKernelGGL((ns_blk_kernel<kApply, false, BT>), grid, block, 0, s, g);
   }
+}
+
+}  // namespace
+
+// 64 x 64 blocks where 128 x 128 ones would leave much of the chip idle: a
+// workgroup alone on its CU is bound by its own operand stream (about 55 GB/s
+// of it), which a smaller block shortens. One 1024 x 1024 matrix 7.7 / 7.9 /
+// 8.1 against 12.4 / 13.5 / 12.7 us for the three products (36 and 64 blocks of
+// 128), GramA of one 1024 x 3072 24 against 34 us, of 4 1024 x 1024 (144 blocks)
+// 12.3 against 13.5; Apply of those (256 blocks) 15.6 against 14.8, all three of
+// one 2560 x 2560 (210 and 400) 40 / 39 / 68 against 30 / 31 / 44. Gram products
+// of 256 rows with K = 256 stay short enough for 64 x 64 (10 of 16 blocks
+// computed instead of 3 of 4): 512 of them 29.5 against 34.7 us.
+void ns_blk_product(int mode, const NsProduct& g, hipStream_t s) {
+  const int64_t nbi = g.M / 128, nbj = g.N / 128;
+  const int64_t items = g.ntiles * (mode == kApply ? nbi * nbj : nbi * (nbi + 1) / 2);
+  if (items <= num_cus() * 5 / 8 || (mode != kApply && g.K <= 256)) launch<64>(mode, g, s);
+  else launch<128>(mode, g, s);
 }

@@ -174,14 +174,16 @@ struct BaUntile {
 // between x and y. round_once: the third product
 // rounds bf16(B X + a X) once (the 2-D form) instead of bf16(bf16(B X) + a X).
 // fused_ba: the second and third products run as one kernel (ns5_ba.hip;
-// mp == np == 512), wsB unused. Returns 0, or HIMUON_EINVAL (nothing
-// launched) when cnt is too large for the fused kernel.
+// mp == np == 512), wsB unused, where that is faster. `pick`: each product on
+// the faster of the block sizes (ns_product), else on 256 x 256 blocks.
+// Returns 0, or HIMUON_EINVAL (nothing launched) when cnt is too large for
+// the fused kernel.
 bool ns5_stream_supported(int mp, int np);
 // untile (fused_ba only; steps >= 2): the last iteration applies the untile
 // with WD/LR instead of storing its result.
 int ns5_stream_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int mp, int np, int steps,
-                    float a, float b, float c, bool round_once, bool fused_ba, uint16_t* wsA, uint16_t* wsB,
-                    hipStream_t s, const BaUntile* untile = nullptr);
+                    float a, float b, float c, bool round_once, bool fused_ba, bool pick, uint16_t* wsA,
+                   uint16_t* wsB, hipStream_t s, const BaUntile* untile = nullptr);
 
 // Fused B = bf16(c A A^T + b A), Y = bf16(bf16(B X) + a X) (ns5_ba.hip) on
 // `cnt` 512 x 512 tiles: A from the first product, X -> Y (Y != X). xinv
@@ -196,16 +198,42 @@ bool ns5_ba_supported(int mp, int np);
 bool ns5_ba_run(const uint16_t* A, const uint16_t* X, uint16_t* Y, const float* xinv, int64_t cnt, float a,
                 float b, float c, bool round_once, hipStream_t s, const BaUntile* untile = nullptr);
 
-// One NS product over `ntiles` batch entries on the 256-block stream kernels
-// (M, N, K multiples of 256; row pitches in elements, batch strides):
-//   mode 0: C = bf16(P P^T)                      P: M x K, C: M x M
-//   mode 1: C = bf16(alpha P P^T + beta R)       R = P, K = M
-//   mode 2: C = bf16(bf16(P Q) + beta R)         P: M x K (K = M), Q, R, C: M x N
+// One NS product over `ntiles` batch entries (row pitches in elements, batch
+// strides):
+//   kGramA: C = bf16(P P^T)                      P: M x K, Q = P, C: M x M
+//   kGramB: C = bf16(alpha P P^T + beta R)       R = P, K = M
+//   kApply: C = bf16(bf16(P Q) + beta R)         P: M x K (K = M), Q, R, C: M x N
 //           (bf16(P Q + beta R) with round_once)
-void ns_stream_product(int mode, const uint16_t* P, int64_t p_bs, int ldp, const uint16_t* Q, int64_t q_bs,
-                       int ldq, const uint16_t* R, int64_t r_bs, int ldr, uint16_t* C, int64_t c_bs, int ldc,
-                       int M, int N, int K, int64_t ntiles, float alpha, float beta, bool round_once,
-                       hipStream_t s);
+// inv non-null (kGramA, kApply): X (P and Q of kGramA, Q and R of kApply) is
+// the raw tile, and X0 = bf16(X inv[tile]) is used in its place.
+enum { kGramA = 0, kGramB = 1, kApply = 2 };
+struct NsProduct {
+  const uint16_t* P; int64_t p_bs; int ldp;    // rows i (output rows), k-contiguous
+  const uint16_t* Q; int64_t q_bs; int ldq;    // Gram: rows j, k-contiguous; Apply: X [k][j]
+  const uint16_t* R; int64_t r_bs; int ldr;    // epilogue operand [i][j] (A or X)
+  uint16_t* C; int64_t c_bs; int ldc;          // output [i][j]
+  int M, N, K;
+  int64_t ntiles;
+  float alpha, beta;
+  int round_once;
+  const float* inv;
+};
+// On 256 x 256 blocks (ns5_stream.hip; M, N, K multiples of 256), on 64 x 64
+// or 128 x 128 blocks (ns5_blk.hip; multiples of 128), and on whichever is
+// faster for the shape (ns5.hip). All give the same bits.
+void ns_stream_product(int mode, const NsProduct& g, hipStream_t s);
+void ns_blk_product(int mode, const NsProduct& g, hipStream_t s);
+void ns_product(int mode, const NsProduct& g, hipStream_t s);
+
+// CUs of the current device, queried per launch (a host-side attribute lookup;
+// nothing is cached in the library).
+inline int num_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+    n = 256;
+  return n;
+}
 
 // Fused LDS-resident path (ns5_lds.hip): mp == 128, np = 128 or 256. Runs
 // `steps` >= 1 iterations of `cnt` tiles in one launch; reads X from x and
@@ -241,19 +269,3 @@ bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype);
 void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
                   int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
                   bool round_once, const float* sa, hipStream_t s);
-// One NS product over a batch (modes, strides and rounding as
-// ns_stream_product) on 128 x 128 output blocks (ns5_blk.hip): M, N, K
-// multiples of 128. inv non-null (modes 0 and 2): X is the raw tile, X0 =
-// bf16(X inv[tile]).
-struct BlkArgs {
-  const uint16_t* P; int64_t p_bs; int ldp;
-  const uint16_t* Q; int64_t q_bs; int ldq;
-  const uint16_t* R; int64_t r_bs; int ldr;
-  uint16_t* C; int64_t c_bs; int ldc;
-  int M, N, K;
-  int64_t ntiles;
-  float alpha, beta;
-  int round_once;
-  const float* inv;
-};
-void ns_blk_product(int mode, const BlkArgs& g, hipStream_t s);

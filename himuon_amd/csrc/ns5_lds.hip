@@ -443,14 +443,6 @@ __global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* 
   step_io<M, NT, DT, PDT, true, false, 8>(params, n_params, X, tile_begin + tt, 0, tile_h, tile_w, sa, 0);
 }
 
-int num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  return n;
-}
-
 }  // namespace
 
 bool lds_step_supported(int tile_h, int tile_w, int dtype, int param_dtype) {

@@ -47,25 +47,13 @@ constexpr int BK = 32;                // K per stream unit
 constexpr int SLOT = 32768;           // bytes per ring slot
 constexpr int HALF = SLOT / 2;        // Q panel offset within a slot
 
-enum { kGramA = 0, kGramB = 1, kApply = 2 };
-
 // Ring slots; units in flight ahead of the MFMAs = slots - 1. GramB and
 // Apply stream their epilogue operand R as four units behind the K loop
 // and take 5 slots; GramA has no R, and 4 slots are 1-3 % faster there.
 template <int MODE>
 constexpr int kSlots = MODE == kGramA ? 4 : 5;
 
-struct StArgs {
-  const uint16_t* P; int64_t p_bs; int ldp;    // rows i (output rows), k-contiguous
-  const uint16_t* Q; int64_t q_bs; int ldq;    // Gram: rows j, k-contiguous; Apply: X [k][j]
-  const uint16_t* R; int64_t r_bs; int ldr;    // epilogue operand [i][j] (A or X)
-  uint16_t* C; int64_t c_bs; int ldc;          // output [i][j]
-  int M, N, K;
-  int64_t ntiles;
-  float alpha, beta;                           // GramB: c, b; Apply: beta = a
-  int round_once;                              // Apply: bf16(B X + a X), one rounding
-  const float* inv;                            // SC kernels: X0 = bf16(X inv[tile]) on load
-};
+using StArgs = NsProduct;
 
 // Chunk swizzles (16-byte chunk index XOR a function of the row):
 //  P/Q row panels, 64-byte rows: spreads 8 (or 16) consecutive rows of one
@@ -574,16 +562,6 @@ __global__ __launch_bounds__(64 * NW, 1) void ns_st_kernel(StArgs g) {
   }
 }
 
-// CUs of the current device, queried per launch (a host-side attribute
-// lookup; nothing is cached in the library).
-int num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  return n;
-}
-
 template <int MODE, bool SC = false>
 void launch(const StArgs& a, int64_t items, hipStream_t s) {
   const int64_t per_xcd = (items + 7) / 8;
@@ -602,47 +580,46 @@ void launch(const StArgs& a, int64_t items, hipStream_t s) {
 
 bool ns5_stream_supported(int mp, int np) { return mp % BT == 0 && np % BT == 0; }
 
-void ns_stream_product(int mode, const uint16_t* P, int64_t p_bs, int ldp, const uint16_t* Q, int64_t q_bs,
-                       int ldq, const uint16_t* R, int64_t r_bs, int ldr, uint16_t* C, int64_t c_bs, int ldc,
-                       int M, int N, int K, int64_t ntiles, float alpha, float beta, bool round_once,
-                       hipStream_t s) {
-  const StArgs g{P, p_bs, ldp, Q, q_bs, ldq, R, r_bs, ldr, C, c_bs, ldc, M, N, K, ntiles, alpha, beta,
-                 round_once ? 1 : 0, nullptr};
-  const int nb = M / BT;
-  if (mode == kApply)
-    launch<kApply>(g, ntiles * nb * (N / BT), s);
-  else if (mode == kGramB)
-    launch<kGramB>(g, ntiles * (nb * (nb + 1) / 2), s);
-  else
-    launch<kGramA>(g, ntiles * (nb * (nb + 1) / 2), s);
+void ns_stream_product(int mode, const NsProduct& g, hipStream_t s) {
+  const int nb = g.M / BT;
+  const int64_t gram = g.ntiles * (nb * (nb + 1) / 2), apply = g.ntiles * nb * (g.N / BT);
+  if (mode == kApply) {
+    if (g.inv) launch<kApply, true>(g, apply, s);
+    else launch<kApply>(g, apply, s);
+  } else if (mode == kGramB) {
+    launch<kGramB>(g, gram, s);
+  } else {
+    if (g.inv) launch<kGramA, true>(g, gram, s);
+    else launch<kGramA>(g, gram, s);
+  }
 }
 
 // One sub-batch of `cnt` tiles, `steps` >= 1 iterations, ping-ponging X
 // between x and y; the first iteration's kernels scale the raw x on load
 // (X0 is never written); A and B live in the workspace.
 int ns5_stream_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int mp, int np, int steps,
-                   float a, float b, float c, bool round_once, bool fused_ba, uint16_t* wsA, uint16_t* wsB,
-                   hipStream_t s, const BaUntile* untile) {
+                   float a, float b, float c, bool round_once, bool fused_ba, bool pick, uint16_t* wsA,
+                   uint16_t* wsB, hipStream_t s, const BaUntile* untile) {
   if (fused_ba && cnt > kBaMaxTiles) return HIMUON_EINVAL;
   if (untile && (!fused_ba || steps < 2)) return HIMUON_EINVAL;
+  const auto product = pick ? ns_product : ns_stream_product;
+  // The fused kernel takes 27 us for up to 16 tiles (4 work items per tile, a
+  // chain of two products per item), the two products on 64 x 64 blocks 16-20;
+  // at 32 tiles 29.5 against 28-32 us, at 48 and more the fused one is ahead.
+  const bool few = pick && cnt <= num_cus() / 16;
   const int64_t sq = (int64_t)mp * mp, rect = (int64_t)mp * np;
-  const int nb = mp / BT;
-  const int64_t gram_items = cnt * (nb * (nb + 1) / 2);
-  const int64_t apply_items = cnt * nb * (np / BT);
   uint16_t* cur = x;
   uint16_t* nxt = y;
   for (int it = 0; it < steps; ++it) {
     const float* xinv = it == 0 ? inv : nullptr;
-    const StArgs ga{cur, rect, np, cur, rect, np, nullptr, 0, 0, wsA, sq, mp, mp, mp, np, cnt, 1.0f, 0.0f, 0, xinv};
-    if (xinv)
-      launch<kGramA, true>(ga, gram_items, s);
-    else
-      launch<kGramA>(ga, gram_items, s);
-    if (fused_ba) {  // B stays on chip: ns5_ba.hip
+    const bool apply_params = untile && it + 1 == steps;
+    product(kGramA, NsProduct{cur, rect, np, cur, rect, np, nullptr, 0, 0, wsA, sq, mp, mp, mp, np, cnt, 1.0f, 0.0f, 0,
+                              xinv}, s);
+    if (fused_ba && (!few || apply_params)) {  // B stays on chip: ns5_ba.hip
       // the untile fused into the last iteration; its per-tile records go to
       // wsB, which the fused path does not use otherwise (cnt mp^2 bf16)
       BaUntile u{};
-      if (untile && it + 1 == steps) {
+      if (apply_params) {
         u = *untile;
         u.rec = reinterpret_cast<int32_t*>(wsB);
       }
@@ -651,14 +628,10 @@ int ns5_stream_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int 
       std::swap(cur, nxt);
       continue;
     }
-    const StArgs gb{wsA, sq, mp, wsA, sq, mp, wsA, sq, mp, wsB, sq, mp, mp, mp, mp, cnt, c, b, 0, nullptr};
-    launch<kGramB>(gb, gram_items, s);
-    const StArgs ap{wsB, sq, mp, cur, rect, np, cur, rect, np, nxt, rect, np, mp, np, mp, cnt, 1.0f, a,
-                    round_once ? 1 : 0, xinv};
-    if (xinv)
-      launch<kApply, true>(ap, apply_items, s);
-    else
-      launch<kApply>(ap, apply_items, s);
+    product(kGramB, NsProduct{wsA, sq, mp, wsA, sq, mp, wsA, sq, mp, wsB, sq, mp, mp, mp, mp, cnt, c, b, 0, nullptr},
+            s);
+    product(kApply, NsProduct{wsB, sq, mp, cur, rect, np, cur, rect, np, nxt, rect, np, mp, np, mp, cnt, 1.0f, a,
+                              round_once ? 1 : 0, xinv}, s);
     std::swap(cur, nxt);
   }
   return 0;

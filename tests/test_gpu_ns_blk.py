@@ -1,10 +1,11 @@
-"""The three NS products on 128 x 128 blocks (ns5_blk.hip) at the edges of
-their range: two K units only, one block, odd block counts, row counts that are
+"""The three NS products on 64 x 64 and 128 x 128 blocks (ns5_blk.hip) at the
+edges of their range: two K units only, one block, odd block counts, row counts that are
 no multiple of 256, more blocks than fit the chip at once. Each against float64
 within a bound from the roundings it makes (torch's own bf16 products split the
 contraction for some of these shapes, so equal bits are not the measure here):
 half a bf16 ulp (at most 2^-8, eight significant bits) of every rounded value, and K 2^-24 of the sum of the
-absolute products for the fp32 accumulation."""
+absolute products for the fp32 accumulation. And the choice of the block size
+(ns_product): whatever it picks gives the bits of the 256 x 256 blocks."""
 
 from __future__ import annotations
 
@@ -15,12 +16,13 @@ pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
     from himuon_amd import _native as nat
+    from himuon_amd.engine import newton_schulz
 
 DEV = "cuda"
 
 
 @pytest.mark.parametrize("batch,M,N", [(1, 128, 128), (5, 128, 1152), (3, 640, 128), (2, 896, 2432), (1, 1024, 256),
-                                       (40, 384, 384)])
+                                       (180, 384, 384), (1, 64 * 11 * 2, 128)])
 @pytest.mark.parametrize("round_once", [False, True])
 def test_blk_products(batch, M, N, round_once):
     g = torch.Generator().manual_seed(M + N)
@@ -51,3 +53,12 @@ def test_blk_products(batch, M, N, round_once):
     e = e if round_once else e + ulp * (s.abs() + e)
     r = s + nat.NS_A * x
     close(Y, r, ulp * (r.abs() + e) + e + 2 * acc * (s.abs() + nat.NS_A * x.abs()))
+
+
+@pytest.mark.parametrize("shape", [(3, 512, 512), (20, 512, 512), (40, 512, 512), (1024, 1024), (9, 1024, 1280),
+                                   (70, 256, 512), (300, 256, 768), (16, 512, 1024)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_block_size_choice_gives_the_256_blocks_bits(shape):
+    G = (torch.randn(*shape, generator=torch.Generator().manual_seed(5)) * 1e-3).to(DEV)
+    for steps in (1, 2):
+        assert torch.equal(newton_schulz(G, steps=steps), newton_schulz(G, steps=steps, family="stream3"))
