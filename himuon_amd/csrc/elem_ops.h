@@ -48,8 +48,7 @@ HM_DEV void wdlr_elems(void* base, int64_t o, const float (&y)[8], int valid, fl
 
 // Untile store of 8 consecutive update values y (fp32, already scaled by the
 // parameter's upd_scale) at element offset o of descriptor P's `update`;
-// `full`: all 8 in range and 16-byte aligned, else the first `valid` one at a
-// time. APPLY: `update` is the parameter itself (ld_upd its row stride) and
+// `full`: all 8 in range, else the first `valid` one at a time. APPLY: `update` is the parameter itself (ld_upd its row stride) and
 // the weight decay and learning rate of its group are applied in place
 // instead of storing the update (himuon_untile_apply):
 //     p = rd(fma(alpha_g, rd(u), rd(p * s_g))),  u = upd_scale * NS (fp32)

@@ -186,7 +186,16 @@ HM_DEV UParam uparam_get(int recv, float sav) {
 // pointers: as flat accesses (what a pointer read from a record becomes) they
 // would also count in lgkmcnt, and every LDS wait of the epilogue would then
 // wait for the parameter loads and stores in flight.
-typedef __attribute__((address_space(1))) u32x4_t g_u32x4;
+// (With the element's alignment only, as load8.)
+template <int DT>
+struct GVec {
+  typedef __attribute__((address_space(1))) u32x4_any type;
+};
+template <>
+struct GVec<HIMUON_DTYPE_F32> {
+  typedef uint32_t vec __attribute__((ext_vector_type(4), aligned(4)));
+  typedef __attribute__((address_space(1))) vec type;
+};
 typedef __attribute__((address_space(1))) uint16_t g_u16;
 typedef __attribute__((address_space(1))) float g_f32;
 
@@ -195,7 +204,8 @@ typedef __attribute__((address_space(1))) float g_f32;
 // row i + 8 n, columns j .. j + 7 (bf16); u = upd_scale X' (fp32), and
 // p = rd(fma(alpha, rd(u), rd(p s))) for every element inside the tile and the
 // parameter. Whole 8-element vectors load their parameter values first (all
-// 4 rows, 2 at a time for fp32 parameters); others go one element at a time.
+// 4 rows, 2 at a time for fp32 parameters); a vector cut by an edge goes one
+// element at a time.
 // u = upd_scale X' for the 8 bf16 values of x.
 HM_DEV void ba_updates(const u32x4_t x, float sc, float (&y)[8]) {
 #pragma unroll
@@ -222,7 +232,7 @@ HM_DEV void ba_unpack(const u32x4_t (&raw)[DT == HIMUON_DTYPE_F32 ? 2 : 1], floa
 
 // 8 parameter values stored as store8<DT> stores them.
 template <int DT>
-HM_DEV void ba_store(g_u32x4* dst, const float (&p)[8]) {
+HM_DEV void ba_store(typename GVec<DT>::type* dst, const float (&p)[8]) {
   if constexpr (DT == HIMUON_DTYPE_F32) {
     __builtin_nontemporal_store(
         u32x4_t{__float_as_uint(p[0]), __float_as_uint(p[1]), __float_as_uint(p[2]), __float_as_uint(p[3])}, dst);
@@ -249,6 +259,7 @@ HM_DEV bool ba_untile_block(const UParam& up, const BaUntile& u, MakeRows&& make
   static_assert(DT == HIMUON_DTYPE_F32 || DT == HIMUON_DTYPE_BF16, "fp32 or bf16 parameters");
   constexpr bool F32 = DT == HIMUON_DTYPE_F32;
   constexpr int ES = F32 ? 4 : 2, NQ = F32 ? 2 : 1;
+  typedef typename GVec<DT>::type gvec;
   u32x4_t rows[4];
   if constexpr (!EARLY) make_rows(rows);
   const int64_t pc = up.c0 + j;
@@ -258,9 +269,8 @@ HM_DEV bool ba_untile_block(const UParam& up, const BaUntile& u, MakeRows&& make
   const int64_t ou0 = (up.r0 + i) * up.ld + pc;  // row i's first element
   // The common case, decided per wave (no divergent branch, so the compiler
   // counts the loads in flight exactly instead of waiting for all of them):
-  // every lane's 4 rows are whole, 16-byte aligned 8-element vectors.
-  const bool all_full = col_full && i + 24 < u.tile_h && up.r0 + i + 24 < up.h &&
-                        aligned16<DT>(up.base, ou0) && ((up.ld * ES) & 15) == 0;
+  // every lane's 4 rows are whole 8-element vectors.
+  const bool all_full = col_full && i + 24 < u.tile_h && up.r0 + i + 24 < up.h;
   if (__all(all_full)) {
     constexpr int NB = F32 ? 2 : 4;  // rows whose loads are in flight together
 #pragma unroll
@@ -268,7 +278,7 @@ HM_DEV bool ba_untile_block(const UParam& up, const BaUntile& u, MakeRows&& make
       u32x4_t raw[NB][NQ];
 #pragma unroll
       for (int k = 0; k < NB; ++k) {
-        const g_u32x4* src = (const g_u32x4*)(base + (ou0 + 8 * (n0 + k) * up.ld) * ES);
+        const gvec* src = (const gvec*)(base + (ou0 + 8 * (n0 + k) * up.ld) * ES);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) raw[k][q] = __builtin_nontemporal_load(src + q);
       }
@@ -279,13 +289,14 @@ HM_DEV bool ba_untile_block(const UParam& up, const BaUntile& u, MakeRows&& make
         ba_updates(rows[n0 + k], up.sc, y);
         ba_unpack<DT>(raw[k], p);
         wdlr8<DT>(p, y, up.s, up.alpha);
-        ba_store<DT>((g_u32x4*)(base + (ou0 + 8 * (n0 + k) * up.ld) * ES), p);
+        ba_store<DT>((gvec*)(base + (ou0 + 8 * (n0 + k) * up.ld) * ES), p);
       }
     }
     return true;
   }
-  // Edge tiles, ragged or unaligned parameters: element by element inside
-  // the tile and the parameter, as wdlr_elems<DT> (static indices).
+  // Edge tiles: whole vectors where a lane has them, the rest element by
+  // element inside the tile and the parameter, as wdlr_elems<DT> (static
+  // indices).
   if constexpr (EARLY) make_rows(rows);
   const int valid = col_ok ? (int)min<int64_t>(min(8, u.tile_w - j), up.w - pc) : 0;
 #pragma unroll
@@ -297,6 +308,17 @@ HM_DEV bool ba_untile_block(const UParam& up, const BaUntile& u, MakeRows&& make
     const int64_t ou = pr * up.ld + pc;
     float y[8];
     ba_updates(rows[n], up.sc, y);
+    if (nv == 8) {
+      u32x4_t raw[NQ];
+      float p[8];
+      gvec* const q8 = (gvec*)(base + ou * ES);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) raw[q] = __builtin_nontemporal_load(q8 + q);
+      ba_unpack<DT>(raw, p);
+      wdlr8<DT>(p, y, up.s, up.alpha);
+      ba_store<DT>(q8, p);
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       if (e < nv) {

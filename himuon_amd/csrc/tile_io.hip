@@ -83,8 +83,7 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(
         const int i = q * rows + v / vpr, j0 = (v % vpr) * 8;
         const int64_t pr = (int64_t)r * geo.tile_h + i, pc = (int64_t)c * geo.tile_w + j0;
         const int64_t og = pr * P.ld_grad + pc, om = pr * P.ld_mom + pc;
-        fast[k] = v < per_item && i < geo.tile_h && pr < P.h && j0 + 8 <= geo.tile_w && pc + 8 <= P.w &&
-                  aligned16<DT>(P.grad, og) && (!has_mom || aligned16<DT>(P.momentum, om));
+        fast[k] = v < per_item && i < geo.tile_h && pr < P.h && j0 + 8 <= geo.tile_w && pc + 8 <= P.w;
         if (fast[k]) {
           load8<DT>(P.grad, og, g[k]);
           if (has_mom) load8<DT>(P.momentum, om, m[k]);
@@ -169,8 +168,7 @@ __global__ __launch_bounds__(kThreads) void gather_trans_kernel(
     const bool row_ok = tr < geo.tile_h && pr < P.h;
     const int64_t og = pr * P.ld_grad + pc, om = pr * P.ld_mom + pc;
     float x[8];
-    const bool fast = row_ok && tc + 8 <= geo.tile_w && pc + 8 <= P.w &&
-                      aligned16<DT>(P.grad, og) && (!has_mom || aligned16<DT>(P.momentum, om));
+    const bool fast = row_ok && tc + 8 <= geo.tile_w && pc + 8 <= P.w;
     if (fast) {
       float g[8], m[8];
       load8<DT>(P.grad, og, g);
@@ -216,6 +214,33 @@ __global__ __launch_bounds__(kThreads) void tile_scale_kernel(const float* __res
   float s = 0.f;
   for (int q = 0; q < per_tile; ++q) s += partials[t * per_tile + q];
   inv[t] = 1.0f / (sqrtf(s) + eps);
+}
+
+// The same for tiles of many partials (whole matrices: one per 64 x 64 block or
+// 32-row slab), one wave per tile: 64 partials per load, added in the same
+// order from the lanes that hold them. One thread walking a 3072 x 1024
+// matrix's 768 took 48 us, latency-bound; this takes 10 us.
+__global__ __launch_bounds__(kThreads) void tile_scale_wave_kernel(const float* __restrict__ partials, int per_tile,
+                                                                  int64_t n_tiles, float eps,
+                                                                  float* __restrict__ inv) {
+  const int64_t t = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  if (t >= n_tiles) return;
+  const int lane = threadIdx.x & 63;
+  const float* const p = partials + t * per_tile;
+  float s = 0.f;
+  float v = lane < per_tile ? p[lane] : 0.f;
+  for (int q0 = 0; q0 < per_tile; q0 += 64) {
+    const float next = q0 + 64 + lane < per_tile ? p[q0 + 64 + lane] : 0.f;
+    const int n = min(64, per_tile - q0);
+    if (n == 64) {
+#pragma unroll
+      for (int i = 0; i < 64; ++i) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
+    } else {
+      for (int i = 0; i < n; ++i) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
+    }
+    v = next;
+  }
+  if (lane == 0) inv[t] = 1.0f / (sqrtf(s) + eps);
 }
 
 // ---------------------------------------------------------------------------
@@ -264,7 +289,7 @@ __global__ __launch_bounds__(kThreads) void untile_rows_kernel(
           y[2 * e2 + 1] = sc * __uint_as_float(w[e2] & 0xffff0000u);
         }
         const int64_t ou = pr * P.ld_upd + pc;
-        const bool full = j0 + 8 <= geo.tile_w && pc + 8 <= P.w && aligned16<DT>(P.update, ou);
+        const bool full = j0 + 8 <= geo.tile_w && pc + 8 <= P.w;
         const int valid = (int)min<int64_t>(min(8, geo.tile_w - j0), P.w - pc);
         put8<APPLY, DT>(P, ou, y, full, valid, sa);
       }
@@ -318,18 +343,10 @@ __global__ __launch_bounds__(kThreads) void untile_trans_kernel(
       y[2 * k + 1] = sc * __uint_as_float(w[k] & 0xffff0000u);
     }
     const int64_t ou = pr * P.ld_upd + pc;
-    const bool full = tc + 8 <= geo.tile_w && pc + 8 <= P.w && aligned16<DT>(P.update, ou);
+    const bool full = tc + 8 <= geo.tile_w && pc + 8 <= P.w;
     const int valid = (int)min<int64_t>(min(8, geo.tile_w - tc), P.w - pc);
     put8<APPLY, DT>(P, ou, y, full, valid, sa);
   }
-}
-
-int num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  return n;
 }
 
 bool geo_ok(int tile_h, int tile_w, int mp, int np) {
@@ -385,9 +402,16 @@ extern "C" int himuon_tile_scale(const float* partials, int partials_per_tile, i
                                  float eps, float* inv, void* stream) {
   if (!partials || !inv || partials_per_tile <= 0 || n_tiles < 0) return HIMUON_EINVAL;
   if (n_tiles == 0) return 0;
-  const dim3 grid((unsigned)((n_tiles + kThreads - 1) / kThreads)), block(kThreads);
-  hipLaunchKernelGGL(tile_scale_kernel, grid, block, 0, static_cast<hipStream_t>(stream),
-                     partials, partials_per_tile, n_tiles, eps, inv);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 block(kThreads);
+  // up to 16 partials (512 x 512 tiles) a thread per tile is as fast and takes
+  // fewer waves (4.7 us for 13,860 tiles)
+  if (partials_per_tile > 16)
+    hipLaunchKernelGGL(tile_scale_wave_kernel, dim3((unsigned)((n_tiles + kThreads / 64 - 1) / (kThreads / 64))), block,
+                       0, s, partials, partials_per_tile, n_tiles, eps, inv);
+  else
+    hipLaunchKernelGGL(tile_scale_kernel, dim3((unsigned)((n_tiles + kThreads - 1) / kThreads)), block, 0, s, partials,
+                       partials_per_tile, n_tiles, eps, inv);
   return (int)hipGetLastError();
 }
 

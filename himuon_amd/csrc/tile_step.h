@@ -83,14 +83,13 @@ HM_DEV float step_io(const HimuonParamDesc* __restrict__ params, int n_params, l
         const int64_t pr = (int64_t)U.r * tile_h + i, pc = (int64_t)U.c * tile_w + j0;
         const int64_t ou = pr * U.P->ld_upd + pc;
         uok[k] = i < tile_h && j0 < tile_w && pr < U.P->h && pc < U.P->w;
-        ufull[k] = uok[k] && j0 + 8 <= tile_w && pc + 8 <= U.P->w && aligned16<PDT>(U.P->update, ou);
+        ufull[k] = uok[k] && j0 + 8 <= tile_w && pc + 8 <= U.P->w;
         if (ufull[k]) load8<PDT>(U.P->update, ou, pv[k]);
       }
       if constexpr (GAT) {
         const int64_t pr = (int64_t)G.r * tile_h + i, pc = (int64_t)G.c * tile_w + j0;
         const int64_t og = pr * G.P->ld_grad + pc, om = pr * G.P->ld_mom + pc;
-        fast[k] = i < tile_h && pr < G.P->h && j0 + 8 <= tile_w && pc + 8 <= G.P->w &&
-                  aligned16<DT>(G.P->grad, og) && (!has_mom || aligned16<DT>(G.P->momentum, om));
+        fast[k] = i < tile_h && pr < G.P->h && j0 + 8 <= tile_w && pc + 8 <= G.P->w;
         if (fast[k]) {
           load8<DT>(G.P->grad, og, g[k]);
           if (has_mom) load8<DT>(G.P->momentum, om, m[k]);
