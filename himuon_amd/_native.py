@@ -170,6 +170,11 @@ _SIGNATURES = {
         [c_void_p, c_int, c_int64, c_int, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double),
          ctypes.POINTER(ctypes.c_double), c_int, c_void_p, c_void_p],
     ),
+    "himuon_adamw_apply": (
+        c_int,
+        [c_void_p, c_int, c_int64, c_int, c_int, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double),
+         ctypes.POINTER(ctypes.c_double), c_int, c_void_p, c_void_p, c_void_p],
+    ),
 }
 
 _lib = None
@@ -554,20 +559,32 @@ def adamw_chunk_elems() -> int:
     return int(load().himuon_adamw_chunk_elems())
 
 
-def adamw_step(desc_table, n_descs, n_chunks, dtype, beta1s, beta2s, epss, bias):
+def adamw_step(desc_table, n_descs, n_chunks, dtype, beta1s, beta2s, epss, bias, param_dtype=None, scale_alpha=None):
     """One AdamW fallback step over a descriptor table (himuon.py:359-372):
     per-group betas/eps are host Python floats; ``bias`` is fp32 device
-    scratch of 2 * n_descs elements."""
+    scratch of 2 * n_descs elements. With ``param_dtype`` the descriptors'
+    update pointers are parameters, and the WD/LR of the device table
+    ``scale_alpha`` is applied to them (himuon_adamw_apply)."""
     n = len(beta1s)
     b1 = (ctypes.c_double * n)(*beta1s)
     b2 = (ctypes.c_double * n)(*beta2s)
     ep = (ctypes.c_double * n)(*epss)
-    _check(
-        load().himuon_adamw_step(
-            desc_table.data_ptr(), n_descs, n_chunks, DTYPE_CODES[dtype], b1, b2, ep, n, bias.data_ptr(), _stream()
-        ),
-        "himuon_adamw_step",
-    )
+    if param_dtype is None:
+        _check(
+            load().himuon_adamw_step(
+                desc_table.data_ptr(), n_descs, n_chunks, DTYPE_CODES[dtype], b1, b2, ep, n, bias.data_ptr(),
+                _stream()
+            ),
+            "himuon_adamw_step",
+        )
+    else:
+        _check(
+            load().himuon_adamw_apply(
+                desc_table.data_ptr(), n_descs, n_chunks, DTYPE_CODES[dtype], DTYPE_CODES[param_dtype], b1, b2, ep, n,
+                bias.data_ptr(), scale_alpha.data_ptr(), _stream()
+            ),
+            "himuon_adamw_apply",
+        )
 
 
 def adamw_desc_table(descs: list[AdamwDesc], device) -> torch.Tensor:

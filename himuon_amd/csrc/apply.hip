@@ -20,7 +20,7 @@
 // into chunks of 8192 elements per parameter; a persistent grid walks the
 // chunks, each thread issuing the loads of its four 8-element vectors before
 // using them.
-#include "common.h"
+#include "elem_ops.h"
 
 namespace {
 
@@ -54,15 +54,6 @@ HM_DEV int find_desc(const HimuonApplyDesc* __restrict__ d, int n, int64_t q) {
     if (d[mid].chunk0 <= q) lo = mid; else hi = mid - 1;
   }
   return lo;
-}
-
-// p1 + alpha * round_p(u), stored in the parameter dtype PD (see above).
-template <int PD, int UD>
-HM_DEV float add_update(float alpha, float u, float p1) {
-  if constexpr (PD == HIMUON_DTYPE_F16 && UD == HIMUON_DTYPE_F32)
-    return fma_f16_once(alpha, round_to<PD>(u), p1);
-  else
-    return __builtin_fmaf(alpha, round_to<PD>(u), p1);
 }
 
 template <int PD, int UD>

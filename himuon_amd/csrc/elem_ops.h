@@ -46,6 +46,18 @@ HM_DEV void wdlr_elems(void* base, int64_t o, const float (&y)[8], int valid, fl
   }
 }
 
+// The add of an update u (dtype UD) into a parameter (dtype PD) already
+// multiplied by 1 - lr wd: p1 + alpha round_p(u), stored in the parameter
+// dtype; for fp16 parameters with fp32 updates rounded once, as torch's
+// mixed-dtype add does.
+template <int PD, int UD>
+HM_DEV float add_update(float alpha, float u, float p1) {
+  if constexpr (PD == HIMUON_DTYPE_F16 && UD == HIMUON_DTYPE_F32)
+    return fma_f16_once(alpha, round_to<PD>(u), p1);
+  else
+    return __builtin_fmaf(alpha, round_to<PD>(u), p1);
+}
+
 // Untile store of 8 consecutive update values y (fp32, already scaled by the
 // parameter's upd_scale) at element offset o of descriptor P's `update`;
 // `full`: all 8 in range, else the first `valid` one at a time. APPLY: `update` is the parameter itself (ld_upd its row stride) and

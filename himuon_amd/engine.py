@@ -348,30 +348,50 @@ class AdamwTables:
     """Device descriptor tables for the AdamW fallback step of a list of
     (grad, moment1, moment2, update, step, group_idx), one table (and one
     launch pair) per grad dtype, built once: every pointer must stay put, as
-    the graph path requires of grads anyway. Entries the kernel cannot take
+    the graph path requires of grads anyway. ``params`` (one per entry, or
+    None): entries with a parameter the kernel takes have their WD/LR applied to
+    it in the same pass and use no update tensor (None may be given); the table
+    is then per (grad dtype, parameter dtype). Entries the kernel cannot take
     (non-contiguous, misaligned, mixed or other dtypes, more than
     ADAMW_MAX_GROUPS groups) are returned in ``fallback`` for the reference's
     torch ops."""
 
-    def __init__(self, entries):
+    @staticmethod
+    def _plain(t, n: int) -> bool:
+        return t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0 and t.numel() == n
+
+    @classmethod
+    def _takes(cls, entry) -> bool:
+        """Whether the kernel takes the entry's grad, moments and step."""
+        g, m, v, _u, st, gi = entry
+        return (
+            all(cls._plain(t, g.numel()) and t.dtype == g.dtype for t in (g, m, v)) and g.dtype in nat.DTYPE_CODES
+            and st.is_cuda and st.dtype == torch.float32 and st.numel() == 1 and g.numel() > 0
+            and gi < nat.ADAMW_MAX_GROUPS
+        )
+
+    @classmethod
+    def applies(cls, entry, p) -> bool:
+        """Whether the kernel also applies the entry's WD/LR to parameter p."""
+        return (p is not None and cls._takes(entry) and cls._plain(p, entry[0].numel())
+                and p.dtype in nat.DTYPE_CODES)
+
+    def __init__(self, entries, params=None):
         chunk = nat.adamw_chunk_elems()
-        by_dtype: dict[torch.dtype, list] = {}
+        by_dtype: dict[tuple, list] = {}
         self.fallback = []
-        for e in entries:
+        self.applied = []  # per entry: run() updates the parameter
+        for e, p in zip(entries, params or [None] * len(entries)):
             g, m, v, u, st, gi = e
-            ts = (g, m, v, u)
-            ok = (
-                all(t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0 and t.dtype == g.dtype
-                    and t.numel() == g.numel() for t in ts)
-                and g.dtype in nat.DTYPE_CODES and st.is_cuda and st.dtype == torch.float32 and st.numel() == 1
-                and g.numel() > 0 and gi < nat.ADAMW_MAX_GROUPS
-            )
-            if ok:
-                by_dtype.setdefault(g.dtype, []).append(e)
+            self.applied.append(self.applies(e, p))
+            if self.applied[-1]:
+                by_dtype.setdefault((g.dtype, p.dtype), []).append((g, m, v, p, st, gi))
+            elif self._takes(e) and self._plain(u, g.numel()) and u.dtype == g.dtype:
+                by_dtype.setdefault((g.dtype, None), []).append(e)
             else:
                 self.fallback.append(e)
-        self.launches = []  # (table, n_descs, n_chunks, dtype, bias scratch)
-        for dt, lst in by_dtype.items():
+        self.launches = []  # (table, n_descs, n_chunks, dtype, bias scratch, parameter dtype or None)
+        for (dt, pdt), lst in by_dtype.items():
             descs, c0 = [], 0
             for g, m, v, u, st, gi in lst:
                 d = nat.AdamwDesc()
@@ -381,11 +401,12 @@ class AdamwTables:
                 c0 += -(-g.numel() // chunk)
             dev = lst[0][0].device
             bias = torch.zeros(2 * len(descs), device=dev, dtype=torch.float32)
-            self.launches.append((nat.adamw_desc_table(descs, dev), len(descs), c0, dt, bias))
+            self.launches.append((nat.adamw_desc_table(descs, dev), len(descs), c0, dt, bias, pdt))
 
-    def run(self, beta1s: list[float], beta2s: list[float], epss: list[float]) -> None:
-        for table, n, n_chunks, dt, bias in self.launches:
-            nat.adamw_step(table, n, n_chunks, dt, beta1s, beta2s, epss, bias)
+    def run(self, beta1s: list[float], beta2s: list[float], epss: list[float],
+            scale_alpha: "torch.Tensor | None" = None) -> None:
+        for table, n, n_chunks, dt, bias, pdt in self.launches:
+            nat.adamw_step(table, n, n_chunks, dt, beta1s, beta2s, epss, bias, pdt, scale_alpha)
 
 
 class _NsPlan:

@@ -73,6 +73,9 @@ class HiMuon(Optimizer):
     # fused-untile buckets of 512 x 512 tiles: the untile with WD/LR runs
     # inside the last NS iteration (himuon_ns5_untile_apply)
     _fuse_ns_untile: bool = True
+    # The AdamW groups' WD/LR runs inside their step (himuon_adamw_apply) for
+    # the parameters it takes; False keeps update tensors and the separate pass.
+    _fuse_adamw: bool = True
     # NS kernel family of every tile group (a key of _native.NS_FAMILIES):
     # "auto", the per-geometry choice; the others are comparison runs, which
     # also keep 128 x 128 buckets off the one-launch LDS step for "block128".
@@ -348,9 +351,10 @@ class HiMuon(Optimizer):
 
     def _prepare_adamw(self):
         """State (as the reference creates it: fp32 device step, zero moments in
-        the grad dtype), persistent update buffers and the device tables of the
-        fused AdamW step for every AdamW-group parameter with a grad. Runs
-        outside graph capture; returns the list of (param, group_idx)."""
+        the grad dtype) and the device tables of the fused AdamW step for every
+        AdamW-group parameter with a grad; persistent update buffers for those
+        whose WD/LR the step cannot apply itself. Runs outside graph capture;
+        returns the list of (param, group_idx)."""
         params = []
         for group_idx, group in enumerate(self.param_groups):
             if group["use_muon"]:
@@ -364,43 +368,51 @@ class HiMuon(Optimizer):
                     st["step"] = torch.zeros((), device=g.device)
                     st["moment1"] = torch.zeros_like(g)
                     st["moment2"] = torch.zeros_like(g)
-                u = self._adamw_updates.get(p)
-                if u is None or u.shape != g.shape or u.dtype != g.dtype or u.device != g.device:
-                    u = torch.empty_like(g, memory_format=torch.contiguous_format)
-                    self._adamw_updates[p] = u
                 params.append((p, group_idx))
         sig = tuple(
-            (id(p), p.grad.data_ptr(), p.grad.dtype, self.state[p]["moment1"].data_ptr(),
-             self._adamw_updates[p].data_ptr(), gi)
+            (id(p), self._local(p).data_ptr(), p.grad.data_ptr(), p.grad.dtype, self.state[p]["moment1"].data_ptr(), gi)
             for p, gi in params
-        )
+        ) + (self._fuse_adamw,)
         if sig != self._adamw_sig:
             self._adamw_sig = sig
-            entries = [
-                (p.grad, self.state[p]["moment1"], self.state[p]["moment2"], self._adamw_updates[p],
-                 self.state[p]["step"], gi)
-                for p, gi in params
-            ]
-            self._adamw_tables = AdamwTables(entries) if entries else None
+            entries, fuse = [], []
+            for p, gi in params:
+                g, st, u = p.grad, self.state[p], self._adamw_updates.get(p)
+                e = (g, st["moment1"], st["moment2"], u, st["step"], gi)
+                fuse.append(p.data if self._fuse_adamw and not self._is_dtensor(p) else None)
+                if AdamwTables.applies(e, fuse[-1]):
+                    self._adamw_updates.pop(p, None)
+                elif u is None or u.shape != g.shape or u.dtype != g.dtype or u.device != g.device:
+                    u = torch.empty_like(g, memory_format=torch.contiguous_format)
+                    self._adamw_updates[p] = u
+                    e = e[:3] + (u,) + e[4:]
+                entries.append(e)
+            self._adamw_tables = AdamwTables(entries, fuse) if entries else None
         return params
 
     def _step_adamw_groups(self):
         """AdamW fallback groups (himuon.py:1013/1034 -> 878-888): one fused
-        HIP pass per grad dtype (himuon_adamw_step) computes step, moments and
-        the update of every parameter; the update then takes the same WD/LR
-        path as the reference's (deferred to after replay in graph mode)."""
+        HIP pass per dtype pair (himuon_adamw_apply) computes step, moments and
+        update of every parameter and applies the WD/LR of the device table.
+        Parameters it cannot take get their update from himuon_adamw_step or
+        the reference's torch ops, and then the reference's WD/LR path (deferred
+        to after replay in graph mode)."""
         params = self._prepare_adamw()
         if not params:
             return
         tables = self._adamw_tables
-        fallback = {e[0].data_ptr() for e in tables.fallback} if tables is not None else set()
-        if tables is not None and tables.launches:
+        fallback = {e[0].data_ptr() for e in tables.fallback}
+        if tables.launches:
             b1 = [float(g["adamw_betas"][0]) for g in self.param_groups]
             b2 = [float(g["adamw_betas"][1]) for g in self.param_groups]
             ep = [float(g["adamw_eps"]) for g in self.param_groups]
-            tables.run(b1, b2, ep)
-        for p, gi in params:
+            tables.run(b1, b2, ep, self._lrwd)
+        for (p, gi), applied in zip(params, tables.applied):
             group = self.param_groups[gi]
+            if applied:
+                if self._in_graph_region:
+                    self._pending_updates.append((p, None, gi))
+                continue
             if p.grad.data_ptr() in fallback:
                 update = self._compute_adamw_step(p, p.grad, group["adamw_betas"], group["adamw_eps"])
             else:

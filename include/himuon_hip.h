@@ -454,6 +454,20 @@ int himuon_adamw_step(const HimuonAdamwDesc* descs_dev, int n_descs,
                       const double* beta2_by_group, const double* eps_by_group,
                       int n_groups, float* bias_dev, void* stream);
 
+/*
+ * himuon_adamw_step with the weight decay and learning rate applied in the
+ * same pass: each descriptor's `update` is the parameter itself (contiguous,
+ * param_dtype), and instead of storing the update,
+ *     p = round_p(fma(alpha[g], round_p(update), round_p(float(p) * scale[g])))
+ * with (scale, alpha) of the descriptor's group read from the device table of
+ * himuon_write_scale_alpha when the kernel runs: the parameters end as
+ * himuon_adamw_step followed by himuon_apply_updates leaves them, bit for bit.
+ */
+int himuon_adamw_apply(const HimuonAdamwDesc* descs_dev, int n_descs,
+                      int64_t n_chunks, int dtype, int param_dtype, const double* beta1_by_group,
+                      const double* beta2_by_group, const double* eps_by_group,
+                      int n_groups, float* bias_dev, const float* scale_alpha_dev, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,92 @@
+"""himuon_adamw_apply: the AdamW step with its WD/LR in the same pass leaves
+moments, step counters and parameters bit-identical to himuon_adamw_step
+followed by himuon_apply_updates, for every dtype pair, sizes around the
+8-element vectors and the chunks, and two groups; and at the optimizer level
+over steps with a changing learning rate, eager and captured."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from himuon_amd import _native as nat
+    from himuon_amd.engine import AdamwTables, ApplyTables
+    from himuon_amd.optimizers.himuon import HiMuon
+
+DEV = "cuda"
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
+BITS = {2: torch.int16, 4: torch.int32}
+SCALE, ALPHA = [1 - 0.02 * 0.1, 1.0], [-0.02, -0.003]
+
+
+@pytest.mark.parametrize("gdt", DTYPES)
+@pytest.mark.parametrize("pdt", DTYPES)
+def test_adamw_apply_equals_step_then_apply(gdt, pdt):
+    gen = torch.Generator().manual_seed(2)
+    sizes = [1, 7, 8, 4095, 4096, 4097, 20001]
+    sa = torch.zeros(2 * nat.APPLY_MAX_GROUPS, device=DEV)
+    nat.write_scale_alpha(sa, SCALE, ALPHA)
+    sides = []
+    data = [[torch.randn(n, generator=gen) * s for s in (1e-3, 1e-4, 1e-6, 0.02)] for n in sizes]
+    for _ in range(2):
+        entries, params = [], []
+        for i, (g, m, v, p) in enumerate(data):
+            g, m, v = (t.to(gdt).to(DEV) for t in (g, m, v.abs()))
+            entries.append((g, m, v, torch.empty_like(g), torch.full((), float(i), device=DEV), i % 2))
+            params.append(p.to(pdt).to(DEV))
+        sides.append((entries, params))
+    (e0, p0), (e1, p1) = sides
+    b, eps = [0.95, 0.9], [1e-8, 1e-6]
+    for _ in range(3):
+        AdamwTables(e0).run(b, b, eps)
+        ApplyTables([(p, e[3], e[5]) for p, e in zip(p0, e0)]).run(SCALE, ALPHA)
+        fused = AdamwTables(e1, p1)
+        assert all(fused.applied) and not fused.fallback
+        fused.run(b, b, eps, sa)
+    for a, c, p, q in zip(e0, e1, p0, p1):
+        for k in (1, 2, 4):
+            assert torch.equal(a[k], c[k])
+        # (bits: fp16 second moments underflow to zero here, so some updates are infinite or NaN)
+        assert torch.equal(p.view(BITS[p.element_size()]), q.view(BITS[q.element_size()]))
+
+
+@pytest.mark.parametrize("cuda_graph", [False, True])
+def test_optimizer_with_and_without(cuda_graph):
+    gen = torch.Generator().manual_seed(3)
+    vals = [torch.randn(*s, generator=gen) * 0.02 for s in ((999, 64), (64,), (256, 320), (33, 5))]
+    runs = []
+    for fuse in (True, False):
+        ps = [torch.nn.Parameter(v.to(torch.bfloat16).to(DEV)) for v in vals]
+        for p in ps:
+            p.grad = torch.zeros_like(p)
+        opt = HiMuon([{"params": [ps[2]], "use_muon": True},
+                      {"params": [ps[0], ps[3]], "use_muon": False, "lr": 2e-3, "weight_decay": 0.1},
+                      {"params": [ps[1]], "use_muon": False, "lr": 1e-3, "weight_decay": 0.0}],
+                     lr=0.02, tile_size=128, cuda_graph=cuda_graph, cuda_graph_warmup=1)
+        opt._fuse_adamw, opt._fuse_untile = fuse, True
+        gg = torch.Generator().manual_seed(4)
+        for k in range(5):
+            for p in ps:
+                p.grad.copy_((torch.randn(p.shape, generator=gg) * 1e-3).to(p.dtype))
+            opt.param_groups[1]["lr"] = 2e-3 / (k + 1)
+            opt.step()
+        if fuse:
+            assert not opt._adamw_updates
+        runs.append(ps)
+    # (eager, unfused: torch's own adds, the same arithmetic where the dtypes agree)
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
+
+
+def test_adamw_apply_argument_errors():
+    import ctypes
+
+    one = (ctypes.c_double * 1)(0.95)
+    lib = nat.load()
+    assert lib.himuon_adamw_apply(8, 1, 4, 0, 1, one, one, one, 1, 8, None, None) == -22
+    assert lib.himuon_adamw_apply(8, 1, 4, 0, 3, one, one, one, 1, 8, 16, None) == -22
+    assert lib.himuon_adamw_apply(None, 1, 4, 0, 1, one, one, one, 1, 8, 16, None) == -22
+    assert lib.himuon_adamw_apply(8, 1, 4, 0, 1, one, one, one, 33, 8, 16, None) == -22
