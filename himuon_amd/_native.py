@@ -139,6 +139,10 @@ _SIGNATURES = {
                                 c_float, c_float, c_float, c_int, c_void_p, c_void_p]),
     "himuon_reg_step": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float,
                                 c_float, c_float, c_float, c_int, c_void_p, c_void_p]),
+    "himuon_ns_direct_supported": (c_int, [c_int, c_int, c_int]),
+    "himuon_ns_direct": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_float, c_float, c_float,
+                                 c_float, c_int, c_void_p]),
+    "himuon_write_desc": (c_int, [ctypes.POINTER(ParamDesc), c_void_p, c_void_p]),
     "himuon_ns5_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_float,
                                    c_float, c_int, c_void_p]),
     "himuon_untile": (
@@ -480,6 +484,26 @@ def reg_step(desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, p
     """lds_step for 256 x 256 NS tiles."""
     _tile_step("himuon_reg_step", desc_table, n_params, tile_begin, n_tiles, tile_h, tile_w, dtype, param_dtype,
                steps, scale_alpha, round_once, coeffs, eps)
+
+
+def ns_direct_supported(M: int, N: int, dtype) -> bool:
+    return bool(load().himuon_ns_direct_supported(M, N, dtype_code(dtype)))
+
+
+def ns_direct(g, out, batch, M, N, steps, round_once=False, coeffs=(NS_A, NS_B, NS_C), eps=NS_EPS):
+    """newton_schulz of `batch` contiguous M x N matrices from g into out in one
+    launch (the shapes of ns_direct_supported)."""
+    a, b, c = coeffs
+    _check(
+        load().himuon_ns_direct(g.data_ptr(), out.data_ptr(), batch, M, N, dtype_code(g.dtype), steps, a, b, c, eps,
+                                NS_ROUND_ONCE if round_once else 0, _stream()),
+        "himuon_ns_direct",
+    )
+
+
+def write_desc(desc: ParamDesc, desc_table) -> None:
+    """desc into the first slot of a device table (a kernel on the current stream)."""
+    _check(load().himuon_write_desc(ctypes.byref(desc), desc_table.data_ptr(), _stream()), "himuon_write_desc")
 
 
 def untile(desc_table, n_params, n_tiles, tile_h, tile_w, mp, np_, dtype, tiles):

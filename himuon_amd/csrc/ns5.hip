@@ -234,6 +234,24 @@ extern "C" int himuon_reg_step(const HimuonParamDesc* params_dev, int n_params, 
   return (int)hipGetLastError();
 }
 
+extern "C" int himuon_ns_direct_supported(int M, int N, int dtype) {
+  const bool rows = (M > 64 && N <= 128) || (M > 128 && N <= 256);
+  return rows && M <= N && (dtype == HIMUON_DTYPE_F32 || dtype == HIMUON_DTYPE_BF16 || dtype == HIMUON_DTYPE_F16);
+}
+
+extern "C" int himuon_ns_direct(const void* g, void* out, int64_t batch, int M, int N, int dtype, int steps, float a,
+                                float b, float c, float eps, int flags, void* stream) {
+  if (!g || !out || batch < 0 || batch > 0x7fffffff || steps < 0 || (flags & ~HIMUON_NS_ROUND_ONCE) ||
+      !himuon_ns_direct_supported(M, N, dtype))
+    return HIMUON_EINVAL;
+  if (batch == 0) return 0;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool ro = (flags & HIMUON_NS_ROUND_ONCE) != 0;
+  if (N <= 128) ns_direct_lds_run(g, out, batch, M, N, dtype, steps, a, b, c, eps, ro, s);
+  else ns_direct_reg_run(g, out, batch, M, N, dtype, steps, a, b, c, eps, ro, s);
+  return (int)hipGetLastError();
+}
+
 extern "C" int himuon_ns5_noalloc(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp,
                                   int np, int steps, float a, float b, float c, int flags, void* stream) {
   if (!x || !y || x == y || !inv || n_tiles < 0 || steps < 0 || mp <= 0 || np <= 0 || mp > np ||

@@ -269,3 +269,10 @@ bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype);
 void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
                   int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
                   bool round_once, const float* sa, hipStream_t s);
+// newton_schulz of cnt contiguous rows x cols matrices (64 < rows <= cols <=
+// 128 / 128 < rows <= cols <= 256, cnt < 2^31) in one launch (ns5_lds.hip,
+// ns5_reg.hip).
+void ns_direct_lds_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
+                       float b, float c, float eps, bool round_once, hipStream_t s);
+void ns_direct_reg_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
+                       float b, float c, float eps, bool round_once, hipStream_t s);

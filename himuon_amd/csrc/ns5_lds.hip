@@ -443,7 +443,53 @@ __global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* 
   step_io<M, NT, DT, PDT, true, false, 8>(params, n_params, X, tile_begin + tt, 0, tile_h, tile_w, sa, 0);
 }
 
+// newton_schulz of a contiguous batch of plain matrices on 128 x 128 NS tiles in
+// one launch: cast, normaliser, iterations and the cast back with the tile in
+// LDS, each element read and written once. 512 matrices of 128 x 128 in bf16:
+// 39 us for the call, against 75 for copy, gather, normaliser, NS,
+// untile and copy.
+template <int DT>
+__global__ __launch_bounds__(NT, 3) void ns_direct_lds_kernel(const void* __restrict__ g, void* __restrict__ out,
+                                                              int64_t ntiles, int rows, int cols, int steps, float ca,
+                                                              float cb, float cc, float eps, int round_once) {
+  constexpr int XCH = M / 8;
+  __shared__ __attribute__((aligned(16))) uint8_t sx_raw[M * M * 2];
+  __shared__ __attribute__((aligned(16))) uint8_t sa_raw[tri_bytes(4)];
+  __shared__ float red[NT / 64];
+  __shared__ float s_inv;
+  lds_u8* const X = (lds_u8*)sx_raw;
+  const int64_t t = blockIdx.x;
+  if (t >= ntiles) return;
+  const float sum = block_sum<NT>(direct_load<M, NT, DT, 8>(g, X, t, rows, cols, 0), red);
+  if (threadIdx.x == 0) s_inv = 1.0f / (sqrtf(0.f + sum) + eps);
+  __syncthreads();
+  const float inv = s_inv;
+  const int ts = opaque_lane((int)threadIdx.x);
+#pragma unroll
+  for (int k = 0; k < M * XCH / NT; ++k) {
+    const int v = k * NT + ts;
+    lds_u32x4* const px = reinterpret_cast<lds_u32x4*>(X + lds_pos(v / XCH, v % XCH, XCH));
+    *px = scale8(*px, inv);
+  }
+  __syncthreads();
+  ns_iterations<1, 4>(X, (lds_u8*)sa_raw, threadIdx.x & 63, steps, ca, cb, cc, round_once);
+  direct_store<M, NT, DT>(out, X, t, rows, cols, 0);
+}
+
 }  // namespace
+
+void ns_direct_lds_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
+                       float b, float c, float eps, bool round_once, hipStream_t s) {
+  const auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)cnt), dim3(NT), 0, s, g, out, cnt, rows, cols, steps, a, b, c, eps,
+                       round_once ? 1 : 0);
+  };
+  switch (dtype) {
+    case HIMUON_DTYPE_F32: run(ns_direct_lds_kernel<HIMUON_DTYPE_F32>); break;
+    case HIMUON_DTYPE_BF16: run(ns_direct_lds_kernel<HIMUON_DTYPE_BF16>); break;
+    default: run(ns_direct_lds_kernel<HIMUON_DTYPE_F16>); break;
+  }
+}
 
 bool lds_step_supported(int tile_h, int tile_w, int dtype, int param_dtype) {
   return tile_h > 0 && tile_h <= tile_w && tile_w <= M &&

@@ -304,6 +304,19 @@ __global__ __launch_bounds__(NT, 1) void ns5_reg_kernel(const uint16_t* x, uint1
   }
 }
 
+// The normaliser of a tile from every wave's sum of squares of the two slabs it
+// passed over (red[s][wave], published): slab 2 s + g is waves 4 g .. + 3 of
+// pass s; the slabs in order, as tile_scale adds the gather's partials.
+HM_DEV float tile_inv(const float (&red)[2][NT / 64], float eps) {
+  float sum = 0.f;
+  for (int q = 0; q < 4; ++q) {
+    float p = 0.f;
+    for (int i = 0; i < 4; ++i) p += red[q >> 1][4 * (q & 1) + i];
+    sum += p;
+  }
+  return 1.0f / (sqrtf(sum) + eps);
+}
+
 // The whole optimizer step of a bucket of 256 x 256 NS tiles in one launch
 // (tiles not transposed), as lds_step_kernel does it for 128 x 128: momentum
 // and gather into LDS, the normaliser, the iterations, the untile with WD/LR.
@@ -335,16 +348,7 @@ __global__ __launch_bounds__(NT, 1) void reg_step_kernel(const HimuonParamDesc* 
     if ((threadIdx.x & 63) == 0) red[s][threadIdx.x >> 6] = w;
   }
   __syncthreads();  // the tile and the waves' sums are in
-  if (threadIdx.x == 0) {
-    // slab 2 s + g: waves 4 g .. + 3 of pass s; slabs in order, as tile_scale adds them
-    float sum = 0.f;
-    for (int q = 0; q < 4; ++q) {
-      float p = 0.f;
-      for (int i = 0; i < 4; ++i) p += red[q >> 1][4 * (q & 1) + i];
-      sum += p;
-    }
-    s_inv = 1.0f / (sqrtf(sum) + eps);
-  }
+  if (threadIdx.x == 0) s_inv = tile_inv(red, eps);
   __syncthreads();
   ns_iterations(L, s_inv, steps, ca, cb, cc, round_once);
 #pragma unroll 1
@@ -352,7 +356,45 @@ __global__ __launch_bounds__(NT, 1) void reg_step_kernel(const HimuonParamDesc* 
     step_io<T, NT, DT, PDT, true, false, UNT_BATCH>(params, n_params, L, tile_begin + tt, 0, tile_h, tile_w, sa, s);
 }
 
+// newton_schulz of a contiguous batch of plain matrices on 256 x 256 NS tiles in
+// one launch, as ns_direct_lds_kernel (ns5_lds.hip) for 128 x 128.
+template <int DT>
+__global__ __launch_bounds__(NT, 1) void ns_direct_reg_kernel(const void* __restrict__ g, void* __restrict__ out,
+                                                              int64_t ntiles, int rows, int cols, int steps, float ca,
+                                                              float cb, float cc, float eps, int round_once) {
+  __shared__ __attribute__((aligned(16))) uint8_t raw[LDS_BYTES];
+  __shared__ float red[2][NT / 64];
+  __shared__ float s_inv;
+  lds_u8* const L = (lds_u8*)raw;
+  const int64_t t = blockIdx.x;
+  if (t >= ntiles) return;
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) {
+    const float w = wave_sum(direct_load<T, NT, DT, 8>(g, L, t, rows, cols, s));
+    if ((threadIdx.x & 63) == 0) red[s][threadIdx.x >> 6] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) s_inv = tile_inv(red, eps);
+  __syncthreads();
+  ns_iterations(L, s_inv, steps, ca, cb, cc, round_once);
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) direct_store<T, NT, DT>(out, L, t, rows, cols, s);
+}
+
 }  // namespace
+
+void ns_direct_reg_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
+                       float b, float c, float eps, bool round_once, hipStream_t s) {
+  const auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)cnt), dim3(NT), 0, s, g, out, cnt, rows, cols, steps, a, b, c, eps,
+                       round_once ? 1 : 0);
+  };
+  switch (dtype) {
+    case HIMUON_DTYPE_F32: run(ns_direct_reg_kernel<HIMUON_DTYPE_F32>); break;
+    case HIMUON_DTYPE_BF16: run(ns_direct_reg_kernel<HIMUON_DTYPE_BF16>); break;
+    default: run(ns_direct_reg_kernel<HIMUON_DTYPE_F16>); break;
+  }
+}
 
 bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype) {
   return tile_h > T / 2 && tile_h <= tile_w && tile_w <= T &&

@@ -349,6 +349,12 @@ __global__ __launch_bounds__(kThreads) void untile_trans_kernel(
   }
 }
 
+// One descriptor into a device table, passed as a launch argument: ordered on
+// the stream before the launches that read it, no host buffer to keep.
+__global__ __launch_bounds__(64) void write_desc_kernel(HimuonParamDesc d, HimuonParamDesc* __restrict__ out) {
+  if (threadIdx.x == 0) *out = d;
+}
+
 bool geo_ok(int tile_h, int tile_w, int mp, int np) {
   const int m = tile_h <= tile_w ? tile_h : tile_w;
   const int n = tile_h <= tile_w ? tile_w : tile_h;
@@ -364,6 +370,12 @@ bool geo_ok(int tile_h, int tile_w, int mp, int np) {
 extern "C" int himuon_gather_partials_per_tile(int tile_h, int tile_w, int mp, int np) {
   if (!geo_ok(tile_h, tile_w, mp, np)) return HIMUON_EINVAL;
   return tile_h > tile_w ? (mp / kBlk) * (np / kBlk) : mp / slab_rows(mp, np);
+}
+
+extern "C" int himuon_write_desc(const HimuonParamDesc* desc, HimuonParamDesc* desc_dev, void* stream) {
+  if (!desc || !desc_dev) return HIMUON_EINVAL;
+  hipLaunchKernelGGL(write_desc_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), *desc, desc_dev);
+  return (int)hipGetLastError();
 }
 
 extern "C" int himuon_momentum_gather(const HimuonParamDesc* params_dev, int n_params,

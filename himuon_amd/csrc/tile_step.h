@@ -158,3 +158,74 @@ HM_DEV float step_io(const HimuonParamDesc* __restrict__ params, int n_params, l
   }
   return ssq;
 }
+
+// newton_schulz on a contiguous batch of rows x cols matrices (rows <= cols <=
+// N), matrix t: slab s0 of it as bf16 into X, zero padded to N x N; returns
+// this thread's sum of squares of it.
+template <int N, int NT, int DT, int BATCH>
+HM_DEV float direct_load(const void* __restrict__ g, lds_u8* X, int64_t t, int rows, int cols, int s0) {
+#pragma clang fp contract(off)
+  using Geo = StepGeo<N, NT>;
+  static_assert(8 % BATCH == 0, "a batch stays inside a slab");
+  const int tq = opaque_lane((int)threadIdx.x);
+  const int64_t base = t * (int64_t)rows * cols;
+  float ssq = 0.f;
+#pragma unroll 1
+  for (int b0 = 8 * s0; b0 < 8 * s0 + 8; b0 += BATCH) {
+    float x[BATCH][8];
+    bool full[BATCH];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int v = Geo::vec(b0 + k, tq), i = v / Geo::VPR, j0 = (v % Geo::VPR) * 8;
+      full[k] = i < rows && j0 + 8 <= cols;
+      if (full[k]) load8<DT>(g, base + (int64_t)i * cols + j0, x[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int v = Geo::vec(b0 + k, tq), i = v / Geo::VPR, j0 = (v % Geo::VPR) * 8;
+      if (!full[k]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          x[k][e] = i < rows && j0 + e < cols ? load_elem<DT>(g, base + (int64_t)i * cols + j0 + e) : 0.f;
+      }
+      uint32_t h[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        h[e] = f32_to_bf16(x[k][e]);
+        const float f = bf16_to_f32(h[e]);
+        ssq = fmaf(f, f, ssq);
+      }
+      *reinterpret_cast<lds_u32x4*>(X + lds_pos(i, v % Geo::VPR, N / 8)) =
+          u32x4_t{pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
+    }
+  }
+  return ssq;
+}
+
+// Slab s0 of X to matrix t of the contiguous output batch.
+template <int N, int NT, int DT>
+HM_DEV void direct_store(void* __restrict__ out, const lds_u8* X, int64_t t, int rows, int cols, int s0) {
+  using Geo = StepGeo<N, NT>;
+  const int tq = opaque_lane((int)threadIdx.x);
+  const int64_t base = t * (int64_t)rows * cols;
+#pragma unroll
+  for (int k = 8 * s0; k < 8 * s0 + 8; ++k) {
+    const int v = Geo::vec(k, tq), i = v / Geo::VPR, j0 = (v % Geo::VPR) * 8;
+    if (i >= rows || j0 >= cols) continue;
+    const u32x4_t w = *reinterpret_cast<lds_cu32x4*>(X + lds_pos(i, v % Geo::VPR, N / 8));
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[2 * e] = bf16_to_f32(w[e] & 0xffffu);
+      y[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+    }
+    const int64_t o = base + (int64_t)i * cols + j0;
+    if (j0 + 8 <= cols) {
+      store8<DT>(out, o, y);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (j0 + e < cols) store_elem<DT>(out, o + e, y[e]);
+    }
+  }
+}

@@ -411,13 +411,14 @@ class AdamwTables:
 
 class _NsPlan:
     """Device state of ``newton_schulz`` for one (batch shape, dtype, device,
-    rounding form, kernel family): a tile group over its own input and output
-    buffers, the sub-batch and the NS workspace, built once, and per step
-    count a hipGraph of its launches (gather, normaliser, NS, untile),
-    captured on first use. A call copies the input into ``xin``, replays the
-    graph and copies the result out of ``out``: it neither allocates device
-    state (beyond the returned tensor) nor rewrites the descriptor table, and
-    costs one replay instead of a dozen or more host launches."""
+    rounding form, kernel family): a tile group, the sub-batch and the NS
+    workspace, built once, and per step count a hipGraph of its launches
+    (gather, normaliser, NS, untile), captured on first use. The launches read
+    and write what the one descriptor of the group's device table points at:
+    ``xin`` and ``out`` until run() writes the call's own input and result
+    there, which then are gathered from and untiled into without a copy. A call
+    neither allocates device state (beyond the returned tensor) nor
+    synchronises, and costs two launches from the host instead of a dozen."""
 
     def __init__(self, n: int, M: int, N: int, dtype: torch.dtype, device, round_once: bool, family: str):
         self.xin = torch.empty((n * M, N), device=device, dtype=dtype)
@@ -426,6 +427,8 @@ class _NsPlan:
             mus=[0.0], nesterovs=[False], device=device, dtype=dtype, round_once=round_once, ns_family=family,
         )
         self.out = self.grp.updates[0]
+        d = self.desc = nat.ParamDesc()
+        d.h, d.w, d.ld_grad, d.ld_upd, d.R, d.C, d.upd_scale = n * M, N, N, N, n, 1, 1.0
         self.sub_batch = self.grp.default_sub_batch()
         self.ws = torch.empty(max(1, self.grp.workspace_bytes(self.sub_batch)), device=device, dtype=torch.uint8)
         self.grp.tiles  # allocate the tile buffers now, not inside a capture
@@ -440,20 +443,30 @@ class _NsPlan:
         g.ns(0, g.n_tiles, steps, self.ws, self.sub_batch)
         g.untile(steps)
 
-    def run(self, steps: int) -> torch.Tensor:
+    def run(self, G: torch.Tensor, steps: int) -> torch.Tensor:
+        """newton_schulz of G (the plan's shape and dtype) as a new tensor."""
+        if not G.is_contiguous():
+            self.xin.view(G.shape).copy_(G)
+            G = self.xin.view(G.shape)
+        out = torch.empty(G.shape, device=G.device, dtype=G.dtype)
+        graph = None
         if torch.cuda.is_current_stream_capturing():
-            # inside the caller's capture: record the launches there
-            self.pinned = True
-            self._launches(steps)
-            return self.out
-        graph = self.graphs.get(steps)
+            self.pinned = True  # inside the caller's capture: record the launches there
+        else:
+            graph = self.graphs.get(steps)
+            if graph is None:
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph):
+                    self._launches(steps)
+                self.graphs[steps] = graph
+        # stream-ordered: after the launches of an earlier call, before this one's
+        self.desc.grad, self.desc.update = G.data_ptr(), out.data_ptr()
+        nat.write_desc(self.desc, self.grp.desc)
         if graph is None:
-            graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
-                self._launches(steps)
-            self.graphs[steps] = graph
-        graph.replay()
-        return self.out
+            self._launches(steps)
+        else:
+            graph.replay()
+        return out
 
 
 _NS_PLANS: "dict[tuple, _NsPlan]" = {}
@@ -463,7 +476,9 @@ _NS_PLANS_MAX = 8
 def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torch.Tensor:
     """Batched NS5 of ``G`` (..., M, N) on the HIP path; same shape and dtype.
 
-    The batch is viewed as one (B*M, N) matrix cut into M x N tiles, so the
+    Matrices of 65 .. 128 by up to 128 and 129 .. 256 by up to 256 (not
+    tall) run in one launch (himuon_ns_direct). Otherwise the batch is
+    viewed as one (B*M, N) matrix cut into M x N tiles, so the
     gather/untile kernels handle the cast, the transpose-if-tall and the
     padding (himuon.py:263-284, test_kernels.py:176-198). A 2-D ``G`` takes
     the reference's 2-D rounding of the third product (torch.addmm,
@@ -480,6 +495,12 @@ def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torc
     n = G.numel() // (M * N) if M * N else 0
     if n == 0:
         return torch.empty_like(G)
+    g = G.detach().to(dtype)
+    if family == "auto" and nat.ns_direct_supported(M, N, dtype) and n < 1 << 31:
+        g = g.contiguous()
+        out = torch.empty(G.shape, device=G.device, dtype=dtype)
+        nat.ns_direct(g, out, n, M, N, steps, round_once=G.ndim == 2)
+        return out.to(G.dtype)
     key = (n, M, N, dtype, G.device, G.ndim == 2, family)
     plan = _NS_PLANS.pop(key, None)
     if plan is None:
@@ -489,5 +510,4 @@ def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torc
                 _NS_PLANS.pop(old)
         plan = _NsPlan(n, M, N, dtype, G.device, G.ndim == 2, family)
     _NS_PLANS[key] = plan  # most recently used last
-    plan.xin.view(G.shape).copy_(G)
-    return plan.run(steps).view(G.shape).to(G.dtype, copy=True)
+    return plan.run(g, steps).to(G.dtype)

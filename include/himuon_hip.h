@@ -291,6 +291,25 @@ int himuon_reg_step(const HimuonParamDesc* params_dev, int n_params,
                     const float* scale_alpha_dev, void* stream);
 
 /*
+ * newton_schulz (himuon.py:232-284) of `batch` contiguous M x N matrices of
+ * dtype (HIMUON_DTYPE_F32 / BF16 / F16) from g into out (same shape and dtype,
+ * contiguous, any element alignment; out may be g itself) in one launch: cast to bf16, normaliser, `steps` iterations, cast back, with
+ * the values of himuon_momentum_gather (no momentum) + himuon_tile_scale +
+ * himuon_ns5_ex + himuon_untile bit for bit. flags: HIMUON_NS_ROUND_ONCE only.
+ * Supported (else HIMUON_EINVAL) for 64 < M <= N <= 128 and 128 < M <= N <= 256.
+ */
+int himuon_ns_direct_supported(int M, int N, int dtype);
+int himuon_ns_direct(const void* g, void* out, int64_t batch, int M, int N, int dtype, int steps, float a, float b,
+                     float c, float eps, int flags, void* stream);
+
+/*
+ * Write one descriptor (a HOST struct, copied into the launch arguments) into a
+ * device descriptor table, as a kernel on `stream`.
+ */
+int himuon_write_desc(const HimuonParamDesc* desc, HimuonParamDesc* desc_dev, void* stream);
+
+
+/*
  * himuon_ns5_ex without a workspace argument, for callers that cannot
  * allocate (code under hipGraph capture, tight serving loops, harnesses that
  * forbid hipMalloc). No counterpart in the reference. It allocates nothing:
