@@ -24,19 +24,33 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int BM = 128;  // edges are multiples of this
+constexpr int kScaleRows = 768;  // padded rows from which X0 is written first
 
-// Y = bf16(X * inv[t]) (steps == 0) or a plain copy (inv == nullptr).
-__global__ __launch_bounds__(kThreads) void ns_scale_copy_kernel(const uint16_t* __restrict__ X,
-                                                                uint16_t* __restrict__ Y,
-                                                                const float* __restrict__ inv,
-                                                                int64_t per_tile, int64_t ntiles) {
-  const int64_t nvec = ntiles * per_tile / 8;
-  for (int64_t v = (int64_t)blockIdx.x * kThreads + threadIdx.x; v < nvec;
-       v += (int64_t)gridDim.x * kThreads) {
-    u32x4_t q = reinterpret_cast<const u32x4_t*>(X)[v];
-    if (inv) q = scale8(q, inv[(v * 8) / per_tile]);
-    reinterpret_cast<u32x4_t*>(Y)[v] = q;
-  }
+// X = bf16(X inv[t]) in place: the result of steps == 0, and X0 of matrices
+// whose products would otherwise scale each value many times (ns5_impl). A
+// workgroup covers kScaleVec 16-byte vectors per thread of one tile.
+constexpr int kScaleVec = 8;
+__global__ __launch_bounds__(kThreads) void ns_scale_kernel(uint16_t* __restrict__ X, const float* __restrict__ inv,
+                                                            int64_t vec_per_tile, int64_t wgs_per_tile) {
+  const int64_t t = blockIdx.x / wgs_per_tile;
+  const int64_t v0 = (blockIdx.x - t * wgs_per_tile) * (kThreads * kScaleVec) + threadIdx.x;
+  u32x4_t* const x = reinterpret_cast<u32x4_t*>(X) + t * vec_per_tile;
+  const float s = inv[t];
+  u32x4_t v[kScaleVec];
+#pragma unroll
+  for (int k = 0; k < kScaleVec; ++k)
+    if (v0 + k * kThreads < vec_per_tile) v[k] = x[v0 + k * kThreads];
+#pragma unroll
+  for (int k = 0; k < kScaleVec; ++k)
+    if (v0 + k * kThreads < vec_per_tile) x[v0 + k * kThreads] = scale8(v[k], s);
+}
+
+void ns_scale(uint16_t* x, const float* inv, int64_t n_tiles, int64_t rect, hipStream_t s) {
+  const int64_t vpt = rect / 8, wgs = (vpt + kThreads * kScaleVec - 1) / (kThreads * kScaleVec);
+  const int64_t most = ((int64_t)1 << 30) / wgs;  // tiles per launch
+  for (int64_t t = 0; t < n_tiles; t += most)
+    hipLaunchKernelGGL(ns_scale_kernel, dim3((unsigned)(std::min(most, n_tiles - t) * wgs)), dim3(kThreads), 0, s,
+                       x + t * rect, inv + t, vpt, wgs);
 }
 
 }  // namespace
@@ -70,10 +84,7 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   const int64_t sq = (int64_t)mp * mp, rect = (int64_t)mp * np;
 
   if (steps == 0) {  // X0 = bf16(x * inv), in place (the result of an even step count is in x)
-    const int64_t nvec = n_tiles * rect / 8;
-    const unsigned grid = (unsigned)std::min<int64_t>((nvec + kThreads - 1) / kThreads, 65536);
-    hipLaunchKernelGGL(ns_scale_copy_kernel, dim3(grid), dim3(kThreads), 0, s, x, x, inv, rect,
-                       n_tiles);
+    ns_scale(x, inv, n_tiles, rect, s);
     return (int)hipGetLastError();
   }
 
@@ -96,9 +107,19 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   const bool ba = ns5_ba_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
   const bool reg = ns5_reg_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
 
+  // Matrices of many blocks: the products of the first iteration would scale
+  // every X value once per block that reads it (9 times in GramA and 8 in Apply
+  // at 1024 rows), beside MFMAs that leave no time for it; X0 is written in its
+  // place once instead. Five iterations of 56 matrices of 1024 x 3072 3.78-3.83
+  // against 3.91-3.95 ms, of 12 of 896 x 2432 0.66-0.67 against 0.68-0.69, of 60
+  // of 768 x 768 0.92-0.93 against 0.93-0.94; from 512 rows on, 400 of 512 x 768
+  // would be slower (2.65 against 2.56-2.60 ms).
+  const bool scale_first = !few_rows && family == HIMUON_NS_FAMILY_AUTO && mp >= kScaleRows;
   for (int64_t s0 = 0; s0 < n_tiles; s0 += sb) {
     const int64_t cnt = std::min<int64_t>(sb, n_tiles - s0);
     const int64_t o = s0 * rect;
+    if (scale_first) ns_scale(x + o, inv + s0, cnt, rect, s);
+    const float* const first_inv = scale_first ? nullptr : inv + s0;
     if (few_rows) {
       if (!ns5_small_run(x + o, y + o, inv + s0, cnt, rows, np, steps, a, b, c, round_once, s)) return HIMUON_EINVAL;
     } else if (lds) {
@@ -111,13 +132,13 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
         u = *untile;
         u.tile0 += s0;
       }
-      const int rc = ns5_stream_run(x + o, y + o, inv + s0, cnt, mp, np, steps, a, b, c, round_once, ba,
+      const int rc = ns5_stream_run(x + o, y + o, first_inv, cnt, mp, np, steps, a, b, c, round_once, ba,
                                     family == HIMUON_NS_FAMILY_AUTO, wsA, wsB, s, untile ? &u : nullptr);
       if (rc) return rc;
     } else {
       const uint16_t* cur = x + o;
       uint16_t* nxt = y + o;
-      const float* cur_inv = inv + s0;
+      const float* cur_inv = first_inv;
       for (int it = 0; it < steps; ++it) {
         ns_blk_product(kGramA, NsProduct{cur, rect, np, cur, rect, np, nullptr, 0, 0, wsA, sq, mp, mp, mp, np, cnt, 1.f, 0.f,
                                   0, cur_inv}, s);
