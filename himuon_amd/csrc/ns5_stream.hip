@@ -13,11 +13,11 @@
 // issues loads. (The code also takes 4 waves in 2x2 of 128x128 each, one
 // per SIMD; that layout measured slower.)
 //
-// Operand stream. K advances in units of 32. Each unit of P (and Q) goes
-// straight from global memory into a 32 KiB slot of a 5-slot LDS ring
+// Operand stream. K advances in units of 32 (GramA: 64). Each unit of P (and Q)
+// goes straight from global memory into a 32 KiB slot of a 5-slot LDS ring
 // (global_load_lds_dwordx4, 1 KiB per wave instruction); loads run 4 units
-// ahead of the MFMAs, so up to 128 KiB per CU are in flight (GramA: 4 slots,
-// 3 units ahead). The epilogue
+// ahead of the MFMAs, so up to 128 KiB per CU are in flight (GramA: two 64 KiB
+// slots, one unit ahead). The epilogue
 // operand R (A for GramB, X for Apply) is streamed behind the last K unit as
 // four more 32 KiB units (64 rows x 256 columns each), so it lands while the
 // last MFMAs run. A direct load writes lane l's 16 bytes at 16 l of the wave's
@@ -26,11 +26,11 @@
 //
 // MFMA operands are swapped (A operand = rows j, B operand = rows i), so lane
 // l holds C[row l%32][4 consecutive columns]. The epilogue converts in
-// registers, then first issues the workgroup's next item's first 4 K units
-// into ring slots 0..3, so that their latency, and the drain of this item's
+// registers, then first issues the workgroup's next item's first 4 K units (GramA:
+// one) into all ring slots but the last, so that their latency, and the drain of this item's
 // stores (vmcnt retires loads and stores in issue order), overlap this
 // epilogue instead of stalling the next item's start. It then stages each
-// wave's 128x128 bf16 result through its 8 KiB quarter of ring slot 4, in 4
+// wave's 128x64 bf16 result through its 4 KiB of the last ring slot, in 4
 // rounds of 32 rows, and writes it with 16-byte row-contiguous stores (256
 // bytes per row). Off-diagonal Gram blocks also write the mirrored block: a
 // 4x4 transpose across each lane quad (two DPP exchanges) restages the
@@ -43,25 +43,38 @@ namespace {
 typedef __attribute__((address_space(3))) u32x4_t lds_u32x4;
 
 constexpr int BT = 256;               // output block edge
-constexpr int BK = 32;                // K per stream unit
-constexpr int SLOT = 32768;           // bytes per ring slot
-constexpr int HALF = SLOT / 2;        // Q panel offset within a slot
+constexpr int STAGE_BYTES = 32768;    // the epilogue's staging area, in the last slot
+
+// K per stream unit; bytes per ring slot (a P and a Q panel of that many
+// columns); the Q panel's offset in a slot
+template <int MODE>
+constexpr int kBK = MODE == kGramA ? 64 : 32;
+template <int MODE>
+constexpr int kSlot = 2 * BT * kBK<MODE> * 2;
+template <int MODE>
+constexpr int kHalf = kSlot<MODE> / 2;
 
 // Ring slots; units in flight ahead of the MFMAs = slots - 1. GramB and
-// Apply stream their epilogue operand R as four units behind the K loop
-// and take 5 slots; GramA has no R, and 4 slots are 1-3 % faster there.
+// Apply stream their epilogue operand R as four 32 KiB units behind the K loop
+// and take 5 slots. GramA has no R and takes units of 64, whose rows are whole
+// 128-byte lines (a row of 32 is half of one, and each line was fetched twice):
+// 4,096 tiles of 512 x 512 back to back 0.953-0.956 ms against 0.980-0.986 with
+// four slots of 32, the Qwen3-4B step at tile 512 68.32-68.38 against
+// 68.57-68.66 ms. (A staging area behind both slots, so that two units of the
+// next item are in flight before this item's stores: 68.37-68.38 ms.)
 template <int MODE>
-constexpr int kSlots = MODE == kGramA ? 4 : 5;
+constexpr int kSlots = MODE == kGramA ? 2 : 5;
 
 using StArgs = NsProduct;
 
 // Chunk swizzles (16-byte chunk index XOR a function of the row):
-//  P/Q row panels, 64-byte rows: spreads 8 (or 16) consecutive rows of one
-//  chunk over distinct bank groups for 32- and 64-bank layouts;
+//  P/Q row panels, 128-byte (swz_p64) or 64-byte rows: spreads 8 (or 16)
+//  consecutive rows of one chunk over distinct bank groups;
 //  X panel of Apply, 512-byte rows: the transposing reads of 4 rows x 32
 //  bytes hit distinct bank groups;
 //  R units and the output staging, 512/256-byte rows: consecutive rows of
 //  one chunk land in distinct bank groups.
+HM_DEV int swz_p64(int r) { return (r >> 1) & 7; }
 HM_DEV int swz_p(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 HM_DEV int swz_x(int r) { return 10 * (r & 1) + 4 * ((r >> 1) & 1); }
 HM_DEV int swz_c(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
@@ -79,7 +92,7 @@ template <int L, int NR, int RL, int DI>
 HM_DEV void wait_unit(int nk, int w, int sp) {
   constexpr auto rmin = [](int a, int b) { return a < b ? a : b; };
   const int rem = nk - 1 - w;
-  if (w < DI && sp > 0) {  // nk >= 8, so rem >= DI here; sp is 16, 32 or 64
+  if (w < DI && sp > 0) {  // nk >= 2 DI, so rem >= DI here; sp is 16, 32 or 64
     if (sp > 32)
       wait_vm<63>();
     else if (sp == 16)
@@ -117,11 +130,12 @@ HM_DEV ItemSrc item_src(const StArgs& g, const ItemPos& it, int lane, int wave) 
   // Row panel (256 rows x 64 B): wave instruction n = NW i + wave fills rows
   // 16 n .. 16 n + 15; lane l lands at row 16 n + l/4, position l%4 and
   // fetches chunk (l%4) ^ swz_p(row) (row & 15 = l/4).
-  const int prl = lane >> 2;
-  const int pch = (lane & 3) ^ swz_p(prl);
+  constexpr int BK = kBK<MODE>, RPI = 512 / BK;  // rows per instruction
+  const int prl = RPI * wave + lane / (BK / 8);
+  const int pch = (lane & (BK / 8 - 1)) ^ (BK == 64 ? swz_p64(prl) : swz_p(prl & 15));
   ItemSrc s;
-  s.p = g.P + it.tile * g.p_bs + (int64_t)(it.bi * BT + 16 * wave + prl) * g.ldp + pch * 8;
-  s.pstep = 16 * NW * (int64_t)g.ldp;
+  s.p = g.P + it.tile * g.p_bs + (int64_t)(it.bi * BT + prl) * g.ldp + pch * 8;
+  s.pstep = RPI * NW * (int64_t)g.ldp;
   if constexpr (MODE == kApply) {
     // X panel (32 k-rows x 512 B): instruction n fills k-rows 2n, 2n + 1;
     // lane l lands at row 2n + l/32, position l%32, fetching chunk
@@ -132,24 +146,25 @@ HM_DEV ItemSrc item_src(const StArgs& g, const ItemPos& it, int lane, int wave) 
     s.qstep = 2 * NW * (int64_t)g.ldq;
     s.qunit = BK * (int64_t)g.ldq;
   } else {
-    s.q = g.Q + it.tile * g.q_bs + (int64_t)(it.bj * BT + 16 * wave + prl) * g.ldq + pch * 8;
-    s.qstep = 16 * NW * (int64_t)g.ldq;
+    s.q = g.Q + it.tile * g.q_bs + (int64_t)(it.bj * BT + prl) * g.ldq + pch * 8;
+    s.qstep = RPI * NW * (int64_t)g.ldq;
     s.qunit = BK;
   }
   return s;
 }
 
 // K unit v of an item into ring slot `slot` (wdst = the wave's 1 KiB part).
-template <int NW>
+template <int MODE, int NW>
 HM_DEV void issue_k(const ItemSrc& s, uint32_t wdst, int v, int slot, bool diag) {
-  const uint32_t d = wdst + slot * SLOT;
+  constexpr int BK = kBK<MODE>, PI = BK / 2 / NW;
+  const uint32_t d = wdst + slot * kSlot<MODE>;
 #pragma unroll
-  for (int i = 0; i < 16 / NW; ++i)
+  for (int i = 0; i < PI; ++i)
     dma16(s.p + i * s.pstep + v * BK, d + i * NW * 1024);
   if (!diag) {
 #pragma unroll
-    for (int i = 0; i < 16 / NW; ++i)
-      dma16(s.q + i * s.qstep + v * s.qunit, d + HALF + i * NW * 1024);
+    for (int i = 0; i < PI; ++i)
+      dma16(s.q + i * s.qstep + v * s.qunit, d + kHalf<MODE> + i * NW * 1024);
   }
 }
 
@@ -181,7 +196,9 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   constexpr int WN = NW / 2;                      // waves along the block's columns
   constexpr int WC = BT / WN;                     // columns per wave (128 or 64)
   constexpr int TJ = WC / 32;                     // MFMA tiles along a wave's columns
-  constexpr int L = (DIAG ? 16 : 32) / NW;        // K-unit loads per wave
+  constexpr int BK = kBK<MODE>, SLOT = kSlot<MODE>, HALF = kHalf<MODE>;
+  constexpr int KSU = BK / 16;                    // MFMA k-steps per unit
+  constexpr int L = (DIAG ? 1 : 2) * (BK / 2) / NW;  // K-unit loads per wave
   constexpr int RL = 32 / NW;                     // R-unit loads per wave
   constexpr int NSLOT = kSlots<MODE>;             // ring slots
   constexpr int DIST = NSLOT - 1;                 // units in flight ahead of the MFMAs
@@ -213,7 +230,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   auto issue = [&](int v) {
     const int slot = v % NSLOT;
     if (v < nk) {
-      issue_k<NW>(src, wdst, v, slot, DIAG);
+      issue_k<MODE, NW>(src, wdst, v, slot, DIAG);
     } else if constexpr (NR > 0) {
       const uint32_t d = wdst + slot * SLOT;
       const int q = v - nk;
@@ -232,8 +249,8 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   // reads of the X panel (ds_read_b64_tr_b16: within 16 lanes, lane 4a+b
   // receives element b of the 8-byte rows addressed by lanes a, a+4, a+8,
   // a+12), giving lane l column j = wn*WC + 32 t + l%32, k = 16 ks + 8 hi + 0..7.
-  const int sp = swz_p(l32 & 15);
-  const int prow = (wm * 128 + l32) * 64, qrow = (wn * WC + l32) * 64;
+  const int sp = BK == 64 ? swz_p64(l32) : swz_p(l32 & 15);
+  const int prow = (wm * 128 + l32) * (2 * BK), qrow = (wn * WC + l32) * (2 * BK);
   const int r16 = lane & 15, te = r16 >> 2;
   const int tr_s = swz_x(te);
   const int tr_row = 8 * hi + te;
@@ -245,7 +262,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
     const int pos = ((2 * ks + hi) ^ sp) * 16;
     if (which & 1) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) fb[t] = *reinterpret_cast<lds_cu32x4*>(s + prow + t * 2048 + pos);
+      for (int t = 0; t < 4; ++t) fb[t] = *reinterpret_cast<lds_cu32x4*>(s + prow + t * (64 * BK) + pos);
     }
     if (!(which & 2)) return;
     // Apply: the lane's read base is made opaque per call, so the addresses
@@ -263,7 +280,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
         fa[t] = u32x4_t{l2[0], l2[1], u2[0], u2[1]};
       } else {
         const lds_u8* qs = DIAG ? s : s + HALF;
-        fa[t] = *reinterpret_cast<lds_cu32x4*>(qs + qrow + t * 2048 + pos);
+        fa[t] = *reinterpret_cast<lds_cu32x4*>(qs + qrow + t * (64 * BK) + pos);
       }
     }
   };
@@ -292,7 +309,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
       asm volatile("" ::: "memory");  // the reads below follow the vmcnt wait
       lds_u8* const d = lds + (v % NSLOT) * SLOT + wave * 1024 + 16 * lane;
 #pragma unroll
-      for (int i = 0; i < 16 / NW; ++i) {
+      for (int i = 0; i < BK / 2 / NW; ++i) {
         lds_u32x4* const p = reinterpret_cast<lds_u32x4*>(d + i * NW * 1024);
         *p = scale8_rne(*p, xs);
         if constexpr (!DIAG) {
@@ -335,7 +352,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   wait_unit<L, NR, RL, DIST>(nk, 0, pre_st);
   scale_unit(0);
   lds_barrier();  // unit 0 is in; every wave is past the previous epilogue's staging
-  issue(DIST);
+  if (DIST < U) issue(DIST);
   u32x4_t fa0[TJ], fb0[4], fa1[TJ], fb1[4];
   // At most one half-unit of fragment reads is in flight at any time (8 or 12
   // LDS operations: lgkmcnt counts to 15). Unit u: the first-half fragments
@@ -350,7 +367,28 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   // After the barrier, the DMA issue of unit u + 1 + DIST and the first-half
   // fragment reads of unit u + 1 go between the rows of unit u's second-half
   // MFMAs, so that they issue while the MFMA pipe is busy.
+  // (64-wide units: two more k-steps between the first and the last.)
+  auto middle = [&](int u) {
+    if constexpr (KSU > 2) {
+#pragma unroll
+      for (int ks = 2; ks < KSU; ks += 2) {
+        mma(fa0, fb0);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkm<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        frags(u, ks, fa0, fb0);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(fa1, fb1);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkm<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        frags(u, ks + 1, fa1, fb1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
   auto unit = [&](int u) {
+    middle(u);
     mma(fa0, fb0);
     __builtin_amdgcn_sched_barrier(0);
     wait_lgkm<0>();  // second-half fragments of unit u
@@ -386,6 +424,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   } else {
     for (int u = 0; u + 1 < nk; ++u) unit(u);
   }
+  middle(nk - 1);
   mma(fa0, fb0);
   __builtin_amdgcn_sched_barrier(0);
   wait_lgkm<0>();
@@ -442,7 +481,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   if (more) {
     const ItemSrc ns = item_src<MODE, NW>(g, nx, lane, wave);
 #pragma unroll
-    for (int v = 0; v < DIST; ++v) issue_k<NW>(ns, wdst, v, v, nx.diag);
+    for (int v = 0; v < DIST; ++v) issue_k<MODE, NW>(ns, wdst, v, v, nx.diag);
   }
 
   // Output stores are non-temporal: the block is not read again by this
@@ -456,7 +495,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
   // Row swizzle: 256-byte rows chunk ^ swz_c(row); 128-byte rows (two per
   // 256-byte bank line) chunk ^ ((row >> 1) & 7).
   constexpr int RB = WC * 2, CPR = WC / 8, RPI = 64 / CPR;
-  lds_u8* const W = lds + DIST * SLOT + wave * (SLOT / NW);
+  lds_u8* const W = lds + DIST * SLOT + wave * (STAGE_BYTES / NW);
   auto swz_s = [](int r) { return CPR == 16 ? swz_c(r) : ((r >> 1) & 7); };
   uint16_t* Ct = g.C + tile * g.c_bs;
   uint16_t* const cdst = Ct + (int64_t)(bi * BT + wm * 128) * g.ldc + bj * BT + wn * WC;
@@ -486,7 +525,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
     // k = l32%4) holds C^T[jt][it..it+3], jt = 32 tj + 8 q + 4 hi + k,
     // it = 32 ti + 4 a (wave-local): 256-byte rows. A round stages MR rows
     // (32 for NW = 4: all q of one tj; 16 for NW = 8: a pair of q).
-    constexpr int MR = (SLOT / NW) / 256, QR = MR / 8;
+    constexpr int MR = (STAGE_BYTES / NW) / 256, QR = MR / 8;
     uint16_t* const mdst = Ct + (int64_t)(bj * BT + wn * WC) * g.ldc + bi * BT + wm * 128;
     const int k = lane & 3, a = l32 >> 2;
     const int srow = lane >> 4, sch = lane & 15;
@@ -520,7 +559,7 @@ __device__ __forceinline__ int st_item(const StArgs& g, lds_u8* lds, const ItemP
 // 0: K from the arguments). NW: waves per workgroup (4 or 8).
 template <int MODE, int NKC, int NW, bool SC>
 __global__ __launch_bounds__(64 * NW, 1) void ns_st_kernel(StArgs g) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kSlots<MODE> * SLOT];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kSlots<MODE> * kSlot<MODE>];
   const int nbi = g.M / BT, nbj = g.N / BT;
   const int per_tile = (MODE == kApply) ? nbi * nbj : nbi * (nbi + 1) / 2;
   const int64_t total = g.ntiles * per_tile;
@@ -570,8 +609,9 @@ void launch(const StArgs& a, int64_t items, hipStream_t s) {
   // 8 waves (two per SIMD): 4.5 % faster than 4 at K = 512 and about 10 %
   // at K = 256 and 1024 on MI355X, so only that layout is launched.
   constexpr int kNW = 8;
-  if (a.K == 16 * BK)
-    hipLaunchKernelGGL((ns_st_kernel<MODE, 16, kNW, SC>), grid, dim3(64 * kNW), 0, s, a);
+  constexpr int kNKC = 512 / kBK<MODE>;
+  if (a.K == 512)
+    hipLaunchKernelGGL((ns_st_kernel<MODE, kNKC, kNW, SC>), grid, dim3(64 * kNW), 0, s, a);
   else
     hipLaunchKernelGGL((ns_st_kernel<MODE, 0, kNW, SC>), grid, dim3(64 * kNW), 0, s, a);
 }
