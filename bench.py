@@ -90,9 +90,9 @@ KERNEL_TRAFFIC = {
 }
 KERNEL_SOURCES = {
     "ns_ba_kernel": ["ns5_ba.hip", "ns5_kernels.h", "common.h"],
-    "ns5_lds_kernel": ["ns5_lds.hip", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
-    "lds_step_kernel": ["ns5_lds.hip", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
-    "ns5_reg_kernel": ["ns5_reg.hip", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
+    "ns5_lds_kernel": ["ns5_lds.hip", "ns_reg.h", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
+    "lds_step_kernel": ["ns5_lds.hip", "ns_reg.h", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
+    "ns5_reg_kernel": ["ns5_reg.hip", "ns_reg.h", "tile_step.h", "lds_tiles.h", "ns5_kernels.h", "common.h", "elem_ops.h"],
     "ns_st_kernel": ["ns5_stream.hip", "ns5_kernels.h", "common.h"],
 }
 

@@ -42,7 +42,7 @@
 // of one chunk and 4 consecutive rows of 2 chunks hit distinct bank groups.
 // np = 128: 52 KiB per workgroup, three workgroups per CU; np = 256: 84 KiB,
 // np = 512: 148 KiB, one per CU (eight waves).
-#include "lds_tiles.h"
+#include "ns_reg.h"
 #include "tile_step.h"
 
 namespace {
@@ -391,7 +391,7 @@ __global__ __launch_bounds__(NTQ, NQ == 1 ? 3 : 1) void ns5_lds_kernel(const uin
 // grad, the momentum buffer (read and written) and the parameter (read and
 // written) once each; no NS tile buffer exists. One tile per workgroup: the
 // workgroups that start as others finish fall out of step with each other, so
-// a CU's three workgroups are mostly in different phases (memory or NS). That
+// a CU's workgroups are mostly in different phases (memory or NS). That
 // measured faster than persistent workgroups that walk several tiles, even
 // with one tile's untile and the next one's gather merged into one pass.
 //
@@ -401,43 +401,36 @@ __global__ __launch_bounds__(NTQ, NQ == 1 ? 3 : 1) void ns5_lds_kernel(const uin
 // 8-element vectors t, t + 256, ..., t + 1792 of the 128 x 128 tile, each in
 // element order; then the same wave and block reductions, and the same
 // 1 / (sqrt(s) + eps)).
+// The iterations keep X in registers (ns_reg.h), so a workgroup takes 32 KiB of
+// LDS and 128 VGPRs and four fit a CU, one more to cover the memory passes
+// with: 8 Llama-3-8B layers (106,496 tiles, fp32) 8.43-8.45 ms against
+// 8.58-8.59 with X and A / B in 52 KiB of LDS and three workgroups (3 workgroups
+// with X in registers: 8.64-8.67 against 8.48-8.51). The NS launches without the
+// memory passes gain nothing from it (2,048 tiles 123-124 against 122 us, 512
+// 42-43 against 40) and keep the LDS form.
 // (The untile issues all 8 of a thread's parameter loads before using any,
 // 8 VGPRs each; the gather 4 grad and momentum pairs, 16 VGPRs each: 8 would
 // spill.)
 template <int DT, int PDT>
-__global__ __launch_bounds__(NT, 3) void lds_step_kernel(const HimuonParamDesc* __restrict__ params, int n_params,
+__global__ __launch_bounds__(NT, 4) void lds_step_kernel(const HimuonParamDesc* __restrict__ params, int n_params,
                                                          int64_t tile_begin, int64_t ntiles, int tile_h,
                                                          int tile_w, int steps, float ca, float cb, float cc,
                                                          float eps, int round_once,
                                                          const float* __restrict__ sa) {
-  constexpr int XCH = M / 8;
   __shared__ __attribute__((aligned(16))) uint8_t sx_raw[M * M * 2];
-  __shared__ __attribute__((aligned(16))) uint8_t sa_raw[tri_bytes(4)];
   __shared__ float red[NT / 64];
   __shared__ float s_inv;
   lds_u8* const X = (lds_u8*)sx_raw;
-  lds_u8* const A = (lds_u8*)sa_raw;
-  const int lane = threadIdx.x & 63;
 
   const int64_t tt = blockIdx.x;  // the grid has one workgroup per tile
   if (tt >= ntiles) return;
   const float ssq =
       step_io<M, NT, DT, PDT, false, true, 4>(params, n_params, X, 0, tile_begin + tt, tile_h, tile_w, sa, 0);
-  // ---- normaliser (the gather's block sum, then tile_scale), X0 in place ----------
+  // ---- normaliser (the gather's block sum, then tile_scale) ---------------------------
   const float sum = block_sum<NT>(ssq, red);
   if (threadIdx.x == 0) s_inv = 1.0f / (sqrtf(0.f + sum) + eps);
   __syncthreads();
-  const float inv = s_inv;
-  const int ts = opaque_lane((int)threadIdx.x);
-#pragma unroll
-  for (int k = 0; k < M * XCH / NT; ++k) {
-    const int v = k * NT + ts;
-    lds_u32x4* const px = reinterpret_cast<lds_u32x4*>(X + lds_pos(v / XCH, v % XCH, XCH));
-    *px = scale8(*px, inv);
-  }
-  __syncthreads();
-
-  ns_iterations<1, 4>(X, A, lane, steps, ca, cb, cc, round_once);
+  ns_reg::reg_iterations<M>(X, s_inv, steps, ca, cb, cc, round_once);
 
   // ---- untile with WD/LR ----------------------------------------------------------
   step_io<M, NT, DT, PDT, true, false, 8>(params, n_params, X, tile_begin + tt, 0, tile_h, tile_w, sa, 0);
