@@ -323,6 +323,7 @@ void launch(int mode, const NsProduct& g, hipStream_t s) {
 void ns_blk_product(int mode, const NsProduct& g, hipStream_t s) {
   const int64_t nbi = g.M / 128, nbj = g.N / 128;
   const int64_t items = g.ntiles * (mode == kApply ? nbi * nbj : nbi * (nbi + 1) / 2);
-  if (items <= num_cus() * 5 / 8 || (mode != kApply && g.K <= 256)) launch<64>(mode, g, s);
+  const bool short_gram = mode != kApply && g.K <= 256 && items < (1 << 21);  // a grid holds 2^24 workgroups
+  if (items <= num_cus() * 5 / 8 || short_gram) launch<64>(mode, g, s);
   else launch<128>(mode, g, s);
 }

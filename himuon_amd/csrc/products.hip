@@ -20,18 +20,31 @@
 //                 keeps 11), each partial product exact in fp32.
 // Output dtypes: fp32, bf16, fp16 (round to nearest even from fp32).
 //
-// The bf16-in / bf16-out products keep their own kernels (ns5.hip,
+// The bf16-in / bf16-out products keep their own kernels (ns5_blk.hip,
 // ns5_stream.hip), bit-identical to torch; these kernels serve every other
-// dtype pair. Block tile 128 x 128 x 64, four waves of 64 x 64 (2 x 2 MFMA
-// 32x32 tiles), operands double-buffered in LDS, as ns5.hip's 128-block
-// kernels; the Gram products compute the lower blocks and store each block
+// dtype pair. Block tile 64 x 64 x 64, four waves of one MFMA 32x32 tile each;
+// operands are converted as they are staged through registers into a double
+// buffer in LDS; the Gram products compute the lower blocks and store each block
 // and its mirror.
+//
+// What bounds them: each K unit's loads, conversions and barrier in turn, so
+// what counts is how many workgroups share a CU. 64 x 64 blocks were faster than
+// 128 x 128 at every size (us, fp32 XXT / ba_plus_cAA / bmm_add): 8 of 512 x 1024
+// 27 / 19 / 42 against 49 / 39 / 54 (59 / 49 / 55 with the mirrored block stored
+// element by element and twice the instructions per conversion), 64 of 1024 x
+// 2048 950 / 548 / 2370 against 1031 / 692 / 3121; fp16 8 of 512 x 1024 21 / 19 /
+// 25 against 47 / 50 / 46.
+#include <algorithm>
+
 #include "ns5_kernels.h"
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int BM = 128, BN = 128, BK = 64;
+constexpr int BT = 64;       // output block edge
+constexpr int BK = 64;       // K per unit
+constexpr int R = BT / 32;   // loader rows per thread
+constexpr int kAlign = 128;  // operand dimensions
 constexpr int kLd = BK + 8;  // padded LDS row pitch (16-bit elements)
 
 enum InType { kInF32 = HIMUON_DTYPE_F32, kInBf16 = HIMUON_DTYPE_BF16, kInF16 = HIMUON_DTYPE_F16,
@@ -70,8 +83,8 @@ HM_DEV Oct load_oct(const void* base, int64_t idx) {
     float x[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float h0 = round_bf16(x[2 * k]), h1 = round_bf16(x[2 * k + 1]);
-      o.hi[k] = pk_bf16(h0, h1);
+      o.hi[k] = pk_bf16(x[2 * k], x[2 * k + 1]);
+      const float h0 = __uint_as_float(o.hi[k] << 16), h1 = __uint_as_float(o.hi[k] & 0xffff0000u);
       // (an infinite or NaN hi carries the value alone)
       o.lo[k] = pk_bf16(__builtin_isfinite(h0) ? x[2 * k] - h0 : 0.f, __builtin_isfinite(h1) ? x[2 * k + 1] - h1 : 0.f);
     }
@@ -111,22 +124,38 @@ HM_DEV void store_out(void* base, int64_t idx, float v, int out_dtype) {
 
 constexpr int planes(int in) { return in == kInF32 ? 2 : 1; }
 
+// 4 consecutive outputs, at any element alignment.
+HM_DEV void store_out4(void* base, int64_t idx, const float (&v)[4], int out_dtype) {
+  if (out_dtype == HIMUON_DTYPE_F32) {
+    *reinterpret_cast<f32x4_any*>(static_cast<float*>(base) + idx) = f32x4_any{v[0], v[1], v[2], v[3]};
+  } else {
+    typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+    u32x2_any w;
+    if (out_dtype == HIMUON_DTYPE_BF16)
+      w = u32x2_any{pack2(f32_to_bf16(v[0]), f32_to_bf16(v[1])), pack2(f32_to_bf16(v[2]), f32_to_bf16(v[3]))};
+    else
+      w = u32x2_any{pack2(f32_to_f16(v[0]), f32_to_f16(v[1])), pack2(f32_to_f16(v[2]), f32_to_f16(v[3]))};
+    *reinterpret_cast<u32x2_any*>(static_cast<uint16_t*>(base) + idx) = w;
+  }
+}
+
 // C = alpha S S^T (+ beta S when add_s; K == M) for each batch entry; S:
-// M x K, C: M x M. Lower 128 x 128 blocks only, each stored at (bi, bj) and
-// mirrored.
+// M x K, C: M x M. Lower BT x BT blocks only, each stored at (bi, bj) and
+// mirrored (a lane holds 4 consecutive rows of a column: 4 consecutive
+// elements of the mirrored row).
 template <int IN>
 __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restrict__ S, void* __restrict__ C,
-                                                             int M, int K, int64_t ntiles, float alpha, float beta,
-                                                             int add_s, int out_dtype) {
+                                                             int M, int K, int64_t first, int64_t count,
+                                                             float alpha, float beta, int add_s, int out_dtype) {
   constexpr int NP = planes(IN);
-  __shared__ __attribute__((aligned(16))) uint16_t sI[2][NP][BM * kLd];
-  __shared__ __attribute__((aligned(16))) uint16_t sJ[2][NP][BN * kLd];
+  __shared__ __attribute__((aligned(16))) uint16_t sI[2][NP][BT * kLd];
+  __shared__ __attribute__((aligned(16))) uint16_t sJ[2][NP][BT * kLd];
 
-  const int nb = M / BM;
+  const int nb = M / BT;
   const int npairs = nb * (nb + 1) / 2;
-  const int64_t total = ntiles * npairs;
-  const int64_t item = xcd_item(total);
-  if (item >= total) return;
+  const int64_t local = xcd_item(count);
+  if (local >= count) return;
+  const int64_t item = first + local;
   const int64_t tile = item / npairs;
   const int p = (int)(item % npairs);
   int bi = 0;
@@ -138,18 +167,18 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
   const int wm = wave >> 1, wn = wave & 1;
   const int lrow = tid >> 3, lkv = (tid & 7) * 8;  // loader: rows lrow + 32q, k offset lkv
 
-  Oct ra[4], rb[4];
+  Oct ra[R], rb[R];
   auto gload = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < R; ++q) {
       const int row = lrow + 32 * q;
-      ra[q] = load_oct<IN>(S, s0 + (int64_t)(bi * BM + row) * K + k0 + lkv);
-      rb[q] = load_oct<IN>(S, s0 + (int64_t)(bj * BN + row) * K + k0 + lkv);
+      ra[q] = load_oct<IN>(S, s0 + (int64_t)(bi * BT + row) * K + k0 + lkv);
+      rb[q] = load_oct<IN>(S, s0 + (int64_t)(bj * BT + row) * K + k0 + lkv);
     }
   };
   auto lstore = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < R; ++q) {
       const int row = lrow + 32 * q;
       *reinterpret_cast<u32x4_t*>(&sI[buf][0][row * kLd + lkv]) = ra[q].hi;
       *reinterpret_cast<u32x4_t*>(&sJ[buf][0][row * kLd + lkv]) = rb[q].hi;
@@ -160,13 +189,9 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
     }
   };
 
-  f32x16_t acc[2][2];
+  f32x16_t acc;
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 
   const int nk = K / BK;
   gload(0);
@@ -178,24 +203,17 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
 #pragma unroll
     for (int ks = 0; ks < BK / 16; ++ks) {
       const int kk = ks * 16 + (lane >> 5) * 8;
-      u32x4_t a[NP][2], b[NP][2];
+      u32x4_t a[NP], b[NP];
 #pragma unroll
-      for (int pl = 0; pl < NP; ++pl)
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) {
-          a[pl][mi] = *reinterpret_cast<const u32x4_t*>(&sI[cur][pl][(wm * 64 + mi * 32 + (lane & 31)) * kLd + kk]);
-          b[pl][mi] = *reinterpret_cast<const u32x4_t*>(&sJ[cur][pl][(wn * 64 + mi * 32 + (lane & 31)) * kLd + kk]);
-        }
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
-          if constexpr (NP == 2) {
-            acc[mi][ni] = mfma_in<IN>(a[1][mi], b[0][ni], acc[mi][ni]);
-            acc[mi][ni] = mfma_in<IN>(a[0][mi], b[1][ni], acc[mi][ni]);
-          }
-          acc[mi][ni] = mfma_in<IN>(a[0][mi], b[0][ni], acc[mi][ni]);
-        }
+      for (int pl = 0; pl < NP; ++pl) {
+        a[pl] = *reinterpret_cast<const u32x4_t*>(&sI[cur][pl][(wm * 32 + (lane & 31)) * kLd + kk]);
+        b[pl] = *reinterpret_cast<const u32x4_t*>(&sJ[cur][pl][(wn * 32 + (lane & 31)) * kLd + kk]);
+      }
+      if constexpr (NP == 2) {
+        acc = mfma_in<IN>(a[1], b[0], acc);
+        acc = mfma_in<IN>(a[0], b[1], acc);
+      }
+      acc = mfma_in<IN>(a[0], b[0], acc);
     }
     if (kt + 1 < nk) lstore(cur ^ 1);
     __syncthreads();
@@ -206,18 +224,24 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
   const int64_t c0 = tile * (int64_t)M * M;
   const bool offdiag = bi > bj;
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int q = 0; q < 4; ++q) {
+    const int i0 = bi * BT + wm * 32 + 8 * q + 4 * (lane >> 5);
+    const int j = bj * BT + wn * 32 + (lane & 31);
+    float v[4];
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
+    for (int e = 0; e < 4; ++e) {
+      v[e] = alpha * acc[4 * q + e];
+      if (add_s) v[e] = fmaf(beta, load_elem_in<IN>(S, s0 + (int64_t)(i0 + e) * K + j), v[e]);
+      if (offdiag || i0 + e >= j) store_out(C, c0 + (int64_t)(i0 + e) * M + j, v[e], out_dtype);
+    }
+    if (offdiag || i0 > j) {  // all 4 below the diagonal
+      store_out4(C, c0 + (int64_t)j * M + i0, v, out_dtype);
+    } else {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = bi * BM + wm * 64 + mi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int j = bj * BN + wn * 64 + ni * 32 + (lane & 31);
-        float v = alpha * acc[mi][ni][r];
-        if (add_s) v = fmaf(beta, load_elem_in<IN>(S, s0 + (int64_t)i * K + j), v);
-        if (offdiag || i >= j) store_out(C, c0 + (int64_t)i * M + j, v, out_dtype);
-        if (offdiag || i > j) store_out(C, c0 + (int64_t)j * M + i, v, out_dtype);
-      }
+      for (int e = 0; e < 4; ++e)
+        if (i0 + e > j) store_out(C, c0 + (int64_t)j * M + i0 + e, v[e], out_dtype);
+    }
+  }
 }
 
 // C = out(Bm X) + gamma X for each batch entry (Bm X rounded to the output
@@ -227,17 +251,17 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
 template <int IN>
 __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __restrict__ Bm,
                                                               const void* __restrict__ X, void* __restrict__ C,
-                                                              int M, int N, int64_t ntiles, float gamma,
-                                                              int out_dtype) {
+                                                              int M, int N, int64_t first, int64_t count,
+                                                              float gamma, int out_dtype) {
   constexpr int NP = planes(IN);
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][NP][BM * kLd];
-  __shared__ __attribute__((aligned(16))) uint16_t sX[2][NP][(BK / 8) * BN * 8];
+  __shared__ __attribute__((aligned(16))) uint16_t sA[2][NP][BT * kLd];
+  __shared__ __attribute__((aligned(16))) uint16_t sX[2][NP][(BK / 8) * BT * 8];
 
-  const int nbi = M / BM, nbj = N / BN;
+  const int nbi = M / BT, nbj = N / BT;
   const int blocks = nbi * nbj;
-  const int64_t total = ntiles * blocks;
-  const int64_t item = xcd_item(total);
-  if (item >= total) return;
+  const int64_t local = xcd_item(count);
+  if (local >= count) return;
+  const int64_t item = first + local;
   const int64_t tile = item / blocks;
   const int blk = (int)(item % blocks);
   const int bi = blk / nbj, bj = blk % nbj;
@@ -246,47 +270,40 @@ __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __rest
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int lrow = tid >> 3, lkv = (tid & 7) * 8;  // Bm loader
-  const int xkq = tid >> 4, xjo = (tid & 15) * 8;  // X loader: rows 4 xkq .. + 3, columns xjo .. + 7
+  const int xk = tid / (BT / 8) * R, xjo = tid % (BT / 8) * 8;  // X loader: rows xk .. + R - 1, columns xjo .. + 7
 
-  Oct ra[4], rx[4];
+  Oct ra[R], rx[R];
   auto gload = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < R; ++q) {
       const int row = lrow + 32 * q;
-      ra[q] = load_oct<IN>(Bm, b0 + (int64_t)(bi * BM + row) * M + k0 + lkv);
+      ra[q] = load_oct<IN>(Bm, b0 + (int64_t)(bi * BT + row) * M + k0 + lkv);
     }
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) rx[rr] = load_oct<IN>(X, x0 + (int64_t)(k0 + 4 * xkq + rr) * N + bj * BN + xjo);
+    for (int rr = 0; rr < R; ++rr) rx[rr] = load_oct<IN>(X, x0 + (int64_t)(k0 + xk + rr) * N + bj * BT + xjo);
   };
   auto lstore = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < R; ++q) {
       const int row = lrow + 32 * q;
       *reinterpret_cast<u32x4_t*>(&sA[buf][0][row * kLd + lkv]) = ra[q].hi;
       if constexpr (NP == 2) *reinterpret_cast<u32x4_t*>(&sA[buf][NP - 1][row * kLd + lkv]) = ra[q].lo;
     }
 #pragma unroll
     for (int pl = 0; pl < NP; ++pl) {
-      uint16_t* base = &sX[buf][pl][(xkq >> 1) * BN * 8 + (xkq & 1) * 4];
+      uint16_t* base = &sX[buf][pl][(xk >> 3) * BT * 8 + (xk & 7)];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int w = e >> 1, h = e & 1;
-        auto v = [&](int rr) { return pl == 0 ? rx[rr].hi[w] : rx[rr].lo[w]; };
-        u32x2_t d;
-        d[0] = pack2(half16(v(0), h), half16(v(1), h));
-        d[1] = pack2(half16(v(2), h), half16(v(3), h));
-        *reinterpret_cast<u32x2_t*>(base + (xjo + e) * 8) = d;
+        auto v = [&](int rr) { return half16(pl == 0 ? rx[rr].hi[w] : rx[rr].lo[w], h); };
+        *reinterpret_cast<uint32_t*>(base + (xjo + e) * 8) = pack2(v(0), v(1));
       }
     }
   };
 
-  f32x16_t acc[2][2];
+  f32x16_t acc;
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 
   const int nk = M / BK;
   gload(0);
@@ -299,41 +316,30 @@ __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __rest
     for (int ks = 0; ks < BK / 16; ++ks) {
       const int kk = ks * 16 + (lane >> 5) * 8;
       const int koct = ks * 2 + (lane >> 5);
-      u32x4_t av[NP][2], bv[NP][2];
+      u32x4_t av[NP], bv[NP];
 #pragma unroll
-      for (int pl = 0; pl < NP; ++pl)
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) {
-          av[pl][mi] = *reinterpret_cast<const u32x4_t*>(&sA[cur][pl][(wm * 64 + mi * 32 + (lane & 31)) * kLd + kk]);
-          bv[pl][mi] = *reinterpret_cast<const u32x4_t*>(&sX[cur][pl][(koct * BN + wn * 64 + mi * 32 + (lane & 31)) * 8]);
-        }
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
-          if constexpr (NP == 2) {
-            acc[mi][ni] = mfma_in<IN>(av[1][mi], bv[0][ni], acc[mi][ni]);
-            acc[mi][ni] = mfma_in<IN>(av[0][mi], bv[1][ni], acc[mi][ni]);
-          }
-          acc[mi][ni] = mfma_in<IN>(av[0][mi], bv[0][ni], acc[mi][ni]);
-        }
+      for (int pl = 0; pl < NP; ++pl) {
+        av[pl] = *reinterpret_cast<const u32x4_t*>(&sA[cur][pl][(wm * 32 + (lane & 31)) * kLd + kk]);
+        bv[pl] = *reinterpret_cast<const u32x4_t*>(&sX[cur][pl][(koct * BT + wn * 32 + (lane & 31)) * 8]);
+      }
+      if constexpr (NP == 2) {
+        acc = mfma_in<IN>(av[1], bv[0], acc);
+        acc = mfma_in<IN>(av[0], bv[1], acc);
+      }
+      acc = mfma_in<IN>(av[0], bv[0], acc);
     }
     if (kt + 1 < nk) lstore(cur ^ 1);
     __syncthreads();
   }
 
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = bi * BM + wm * 64 + mi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int j = bj * BN + wn * 64 + ni * 32 + (lane & 31);
-        const int64_t e = x0 + (int64_t)i * N + j;
-        const float bx = round_out(acc[mi][ni][r], out_dtype);
-        store_out(C, e, bx + gamma * load_elem_in<IN>(X, e), out_dtype);
-      }
+  for (int r = 0; r < 16; ++r) {
+    const int i = bi * BT + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+    const int j = bj * BT + wn * 32 + (lane & 31);
+    const int64_t e = x0 + (int64_t)i * N + j;
+    const float bx = round_out(acc[r], out_dtype);
+    store_out(C, e, bx + gamma * load_elem_in<IN>(X, e), out_dtype);
+  }
 }
 
 bool dtype_in_ok(int d) {
@@ -341,39 +347,49 @@ bool dtype_in_ok(int d) {
 }
 bool dtype_out_ok(int d) { return d == HIMUON_DTYPE_F32 || d == HIMUON_DTYPE_BF16 || d == HIMUON_DTYPE_F16; }
 
+// Launches of at most 2^23 work items: a grid holds fewer than 2^32 threads,
+// which a result near the size of the memory exceeds in 64 x 64 blocks.
+constexpr int64_t kLaunchItems = int64_t(1) << 23;
+
 template <int IN>
-void launch_gram(const void* s, void* c, int M, int K, int64_t items, int64_t batch, float alpha, float beta,
-                 int add_s, int od, hipStream_t st) {
-  hipLaunchKernelGGL(prod_gram_kernel<IN>, dim3((unsigned)xcd_grid(items)), dim3(kThreads), 0, st, s, c, M, K,
-                     batch, alpha, beta, add_s, od);
+void launch_gram(const void* s, void* c, int M, int K, int64_t batch, float alpha, float beta, int add_s, int od,
+                 hipStream_t st) {
+  const int64_t nb = M / BT, items = batch * (nb * (nb + 1) / 2);
+  for (int64_t first = 0; first < items; first += kLaunchItems) {
+    const int64_t count = std::min(kLaunchItems, items - first);
+    hipLaunchKernelGGL(prod_gram_kernel<IN>, dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, s, c, M, K, first,
+                       count, alpha, beta, add_s, od);
+  }
 }
 
 template <int IN>
-void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t items, int64_t batch, float gamma,
-                  int od, hipStream_t st) {
-  hipLaunchKernelGGL(prod_apply_kernel<IN>, dim3((unsigned)xcd_grid(items)), dim3(kThreads), 0, st, b, x, c, M, N,
-                     batch, gamma, od);
+void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int od,
+                  hipStream_t st) {
+  const int64_t items = batch * (M / BT) * (N / BT);
+  for (int64_t first = 0; first < items; first += kLaunchItems) {
+    const int64_t count = std::min(kLaunchItems, items - first);
+    hipLaunchKernelGGL(prod_apply_kernel<IN>, dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, b, x, c, M, N,
+                       first, count, gamma, od);
+  }
 }
 
-// Work items (one 128 x 128 output block each) a launch takes: the grid is
-// at most 2^31 workgroups.
+// 128 x 128 output blocks a call takes.
 constexpr int64_t kMaxItems = (int64_t(1) << 31) - 8;
 
 int gram(const void* s, void* c, int M, int K, int64_t batch, float alpha, float beta, int add_s, int id, int od,
          void* stream) {
-  if (!s || !c || s == c || batch < 0 || M <= 0 || K <= 0 || M % BM || K % BK || !dtype_in_ok(id) ||
+  if (!s || !c || s == c || batch < 0 || M <= 0 || K <= 0 || M % kAlign || K % BK || !dtype_in_ok(id) ||
       !dtype_out_ok(od) || (add_s && K != M))
     return HIMUON_EINVAL;
   if (batch == 0) return 0;
-  const int nb = M / BM;
+  const int64_t nb = M / kAlign;
   if (batch > kMaxItems / (nb * (nb + 1) / 2)) return HIMUON_EINVAL;
-  const int64_t items = batch * (nb * (nb + 1) / 2);
   const hipStream_t st = static_cast<hipStream_t>(stream);
   switch (id) {
-    case HIMUON_DTYPE_F32: launch_gram<kInF32>(s, c, M, K, items, batch, alpha, beta, add_s, od, st); break;
-    case HIMUON_DTYPE_BF16: launch_gram<kInBf16>(s, c, M, K, items, batch, alpha, beta, add_s, od, st); break;
-    case HIMUON_DTYPE_F16: launch_gram<kInF16>(s, c, M, K, items, batch, alpha, beta, add_s, od, st); break;
-    default: launch_gram<kInE5m2>(s, c, M, K, items, batch, alpha, beta, add_s, od, st); break;
+    case HIMUON_DTYPE_F32: launch_gram<kInF32>(s, c, M, K, batch, alpha, beta, add_s, od, st); break;
+    case HIMUON_DTYPE_BF16: launch_gram<kInBf16>(s, c, M, K, batch, alpha, beta, add_s, od, st); break;
+    case HIMUON_DTYPE_F16: launch_gram<kInF16>(s, c, M, K, batch, alpha, beta, add_s, od, st); break;
+    default: launch_gram<kInE5m2>(s, c, M, K, batch, alpha, beta, add_s, od, st); break;
   }
   return (int)hipGetLastError();
 }
@@ -392,19 +408,18 @@ extern "C" int himuon_ba_plus_caa_typed(const void* a, void* out, int64_t batch,
 
 extern "C" int himuon_bmm_add_typed(const void* b, const void* x, void* out, int64_t batch, int M, int N, float a,
                                     int in_dtype, int out_dtype, void* stream) {
-  if (!b || !x || !out || out == x || out == b || batch < 0 || M <= 0 || N <= 0 || M % BM || N % BN ||
+  if (!b || !x || !out || out == x || out == b || batch < 0 || M <= 0 || N <= 0 || M % kAlign || N % kAlign ||
       !dtype_in_ok(in_dtype) || !dtype_out_ok(out_dtype))
     return HIMUON_EINVAL;
   if (batch == 0) return 0;
-  const int64_t blocks = (int64_t)(M / BM) * (N / BN);
+  const int64_t blocks = (int64_t)(M / kAlign) * (N / kAlign);
   if (batch > kMaxItems / blocks) return HIMUON_EINVAL;
-  const int64_t items = batch * blocks;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   switch (in_dtype) {
-    case HIMUON_DTYPE_F32: launch_apply<kInF32>(b, x, out, M, N, items, batch, a, out_dtype, st); break;
-    case HIMUON_DTYPE_BF16: launch_apply<kInBf16>(b, x, out, M, N, items, batch, a, out_dtype, st); break;
-    case HIMUON_DTYPE_F16: launch_apply<kInF16>(b, x, out, M, N, items, batch, a, out_dtype, st); break;
-    default: launch_apply<kInE5m2>(b, x, out, M, N, items, batch, a, out_dtype, st); break;
+    case HIMUON_DTYPE_F32: launch_apply<kInF32>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    case HIMUON_DTYPE_BF16: launch_apply<kInBf16>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    case HIMUON_DTYPE_F16: launch_apply<kInF16>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    default: launch_apply<kInE5m2>(b, x, out, M, N, batch, a, out_dtype, st); break;
   }
   return (int)hipGetLastError();
 }

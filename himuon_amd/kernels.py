@@ -24,7 +24,8 @@ Drop-in for ``tang0389/himuon`` ``src/himuon/triton_kernels``
   no counterpart.
 
 Dimensions that are not multiples of 128 are zero padded (exact for all three
-products) into scratch tensors and sliced back. There is no CPU path: non-HIP
+products) into scratch tensors and sliced back; an ``out`` of the kernels' own
+shape is written directly. There is no CPU path: non-HIP
 tensors raise, as the reference's stubs do without a GPU
 (triton_kernels/__init__.py:8-19).
 """
@@ -69,6 +70,21 @@ def _padded(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
     return out
 
 
+def _result(out: torch.Tensor, shape: tuple, *operands: torch.Tensor) -> "torch.Tensor | None":
+    """`out` itself where the kernel can write it: the unpadded shape on the
+    operands' device, contiguous and 16-byte aligned, in a storage of its own
+    (the kernels read their operands while they store). None: a scratch tensor
+    is written and copied to it, which also keeps copy_'s own checks for tensors
+    that require a gradient and for inference tensors."""
+    own = out.untyped_storage().data_ptr()
+    if (tuple(out.shape) == shape and out.is_contiguous() and out.data_ptr() % 16 == 0 and not out.requires_grad
+            and not out.is_inference() and not out.is_neg()
+            and all(t.device == out.device and t.untyped_storage().data_ptr() != own for t in operands)):
+        torch.autograd.graph.increment_version(out)  # as the copy would
+        return out
+    return None
+
+
 def _r(n: int) -> int:
     return nat.round_up(n, nat.NS_ALIGN)
 
@@ -92,12 +108,15 @@ def XXT(A: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     B = a3.shape[0]
     mp, kp = _r(M), _r(K)
     x = _padded(a3, mp, kp)
-    o = torch.empty((B, mp, mp), device=A.device, dtype=out.dtype)
+    o3 = _as3d(out)
+    res = _result(o3, (B, mp, mp), A)
+    o = torch.empty((B, mp, mp), device=A.device, dtype=out.dtype) if res is None else res
     if _native_bf16(A, out):
         nat.xxt(x, o, B, mp, kp)
     else:
         nat.xxt_typed(x, o, B, mp, kp)
-    _as3d(out).copy_(o[:, :M, :M])
+    if res is None:
+        o3.copy_(o[:, :M, :M])
     return out
 
 
@@ -114,12 +133,15 @@ def ba_plus_cAA(A: torch.Tensor, alpha: float, beta: float, out: torch.Tensor) -
     B = a3.shape[0]
     mp = _r(M)
     x = _padded(a3, mp, mp)
-    o = torch.empty((B, mp, mp), device=A.device, dtype=out.dtype)
+    o3 = _as3d(out)
+    res = _result(o3, (B, mp, mp), A)
+    o = torch.empty((B, mp, mp), device=A.device, dtype=out.dtype) if res is None else res
     if _native_bf16(A, out):
         nat.ba_plus_caa(x, o, B, mp, float(alpha), float(beta))
     else:
         nat.ba_plus_caa_typed(x, o, B, mp, float(alpha), float(beta))
-    _as3d(out).copy_(o[:, :M, :M])
+    if res is None:
+        o3.copy_(o[:, :M, :M])
     return out
 
 
@@ -142,12 +164,14 @@ def fused_bmm_add(B: torch.Tensor, X: torch.Tensor, a: float, out: torch.Tensor 
     mp, npd = _r(M), _r(N)
     b = _padded(B, mp, mp)
     x = _padded(X, mp, npd)
-    o = torch.empty((Batch, mp, npd), device=X.device, dtype=out.dtype)
+    res = _result(out, (Batch, mp, npd), B, X)
+    o = torch.empty((Batch, mp, npd), device=X.device, dtype=out.dtype) if res is None else res
     if _native_bf16(B, X, out):
         nat.bmm_add(b, x, o, Batch, mp, npd, float(a))
     else:
         nat.bmm_add_typed(b, x, o, Batch, mp, npd, float(a))
-    out.copy_(o[:, :M, :N])
+    if res is None:
+        out.copy_(o[:, :M, :N])
     return out
 
 
