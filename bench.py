@@ -45,7 +45,7 @@ NS_KERNELS = {
     "fused": "ns5 stage: ns_st_kernel<0> (X X^T) + ns_ba_kernel (c A A^T + b A, then B X + a X with B kept in LDS) per iteration",
     "stream": "ns5 stage: ns_st_kernel<0> (X X^T), <1> (c A A^T + b A), <2> (B X + a X) per iteration",
     "lds": "ns5 stage: ns5_lds_kernel (128-row tiles) or ns5_reg_kernel (256x256): all 5 iterations of a tile on chip",
-    "small": "ns5 stage: ns_gram_kernel x2 + ns_apply_kernel per iteration",
+    "small": "ns5 stage: ns_blk_kernel (X X^T, c A A^T + b A, B X + a X) per iteration",
     "few_rows": "ns5 stage: ns5_small_kernel (all 5 iterations of a tile's 16, 32 or 64 rows resident in LDS)",
 }
 
@@ -82,11 +82,11 @@ PEAK_HBM_GBS = 8000.0
 # (config, kernel) with the sha256 (first 16 hex digits) of the kernel's
 # source files: a figure measured on other sources is not reported.
 KERNEL_TRAFFIC = {
-    # 4096 tiles: FETCH_SIZE 2,389,747 KiB x 1.99968, WRITE_SIZE 2,097,152 KiB x 1.0
-    ("qwen3-4b", "ns_ba_kernel"): (7.0409e+09, "3a8e3e6cc89a4157"),
+    # 4096 tiles: FETCH_SIZE 2,392,451 KiB x 1.99966, WRITE_SIZE 2,097,152 KiB x 1.0
+    ("qwen3-4b", "ns_ba_kernel"): (7.0464e+09, "38713ea5ca84f4fa"),
     # 65,536 tiles of 128 x 128, the whole step (fp32 grads, momentum and params):
-    # FETCH_SIZE 6,291,820 KiB x 1.99966, WRITE_SIZE 8,388,635 KiB x 1.0
-    ("llama3-8b-t128", "lds_step_kernel"): (2.1473e+10, "d874cb37e2f82c2e"),
+    # FETCH_SIZE 6,291,902 KiB x 1.99967, WRITE_SIZE 8,388,760 KiB x 1.0
+    ("llama3-8b-t128", "lds_step_kernel"): (2.1474e+10, "eea0b2d025b0ad3f"),
 }
 KERNEL_SOURCES = {
     "ns_ba_kernel": ["ns5_ba.hip", "ns5_kernels.h", "common.h"],
@@ -259,7 +259,7 @@ def time_dominant_kernel(opt, reps: int) -> dict:
     steps = g["steps"]
     ms = _event_loop(lambda: nat.ns5(x, y, inv, n, m, nn, steps, opt._workspace, n, round_once=grp.round_once),
                      reps, prep=grp.gather)
-    name = {"lds": "ns5_lds_kernel" if m == 128 else "ns5_reg_kernel", "stream": "ns_st_kernel", "small": "ns_gram_kernel/ns_apply_kernel"}[fam]
+    name = {"lds": "ns5_lds_kernel" if m == 128 else "ns5_reg_kernel", "stream": "ns_st_kernel", "small": "ns_blk_kernel"}[fam]
     return {"kernel": name, "family": fam, "launch_tiles": n, "launch_ms": ms,
             "flops_per_launch": float(ns_flops(grp.m, grp.n)) * n}
 
