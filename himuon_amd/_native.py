@@ -262,9 +262,9 @@ def ns5_workspace_bytes(sub_batch: int, mp: int, np_: int) -> int:
 
 
 # himuon_ns5_ex flags (include/himuon_hip.h). Kernel families: AUTO picks per
-# geometry (what the optimizer runs); BLOCK128 runs the 128x128-block kernels
-# everywhere and STREAM3 the three streamed products where AUTO fuses two
-# (comparison runs, named explicitly by the caller). ROUND_ONCE: the
+# geometry (what the optimizer runs); BLOCK128 runs the 64x64- and 128x128-block
+# kernels everywhere and STREAM3 the three streamed 256-block products where
+# both edges are multiples of 256 (comparison runs, named explicitly by the caller). ROUND_ONCE: the
 # reference's 2-D third product, bf16(B X + a X).
 NS_FAMILY_AUTO = 0
 NS_FAMILY_BLOCK128 = 1

@@ -139,13 +139,14 @@ size_t himuon_ns5_workspace_bytes(int64_t sub_batch, int mp, int np);
  * x, y: (n_tiles, mp, np) bf16; X ping-pongs between them, so the result is
  * in x when `steps` is even and in y when it is odd (the other buffer's
  * contents are unspecified afterwards; x and y must not alias). X0 is formed
- * by the first iteration's kernels as they read x, not by a separate pass.
+ * by the first iteration's kernels as they read x, or, for three products of
+ * mp >= 768, written over x by one pass before them.
  * Tiles with mp == 128 and np in {128, 256, 512} run all iterations
- * of a tile inside one workgroup's LDS; 512 x 512 tiles run the first
- * product on a persistent 256x256-block kernel and the other two fused
- * (himuon_ba_bmm_add's kernel); other tiles whose mp and np are multiples of
- * 256 run the three products on persistent 256x256-block kernels; other
- * geometries on 128x128-block kernels. Tiles are processed in sub-batches of `sub_batch`;
+ * of a tile inside one workgroup's LDS, 256 x 256 tiles with X in registers; more
+ * than 16 512 x 512 tiles run the first product on a persistent 256x256-block
+ * kernel and the other two fused (himuon_ba_bmm_add's kernel); other
+ * geometries run three products, each on the faster of 64x64, 128x128 and
+ * (edges that are multiples of 256) 256x256 blocks. Tiles are processed in sub-batches of `sub_batch`;
  * the workspace must hold himuon_ns5_workspace_bytes(sub_batch, mp, np)
  * bytes whenever steps > 0.
  */
@@ -164,9 +165,9 @@ int himuon_ns5(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles,
  *  - kernel family (bits HIMUON_NS_FAMILY_MASK; no reference counterpart,
  *    for comparison tests and benchmarks): HIMUON_NS_FAMILY_AUTO picks per
  *    geometry as himuon_ns5 does; HIMUON_NS_FAMILY_BLOCK128 runs the
- *    128x128-block kernels for every geometry; HIMUON_NS_FAMILY_STREAM3 runs
- *    the three products as three streamed 256-block kernels where AUTO fuses
- *    the second and third (512 x 512 tiles). Results are identical.
+ *    64x64- and 128x128-block kernels for every geometry; HIMUON_NS_FAMILY_STREAM3
+ *    runs the three products as three streamed 256-block kernels wherever both
+ *    edges are multiples of 256. Results are identical.
  *  - HIMUON_NS_ROWS(m), m = 1 .. 64: the tiles' NS operands have only m
  *    nonzero rows (the reference's small-M shapes, e.g. 16 x 1024;
  *    himuon.py:261-284). With mp == 128, family AUTO then iterates only the
