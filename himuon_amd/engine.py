@@ -495,7 +495,7 @@ def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torc
     n = G.numel() // (M * N) if M * N else 0
     if n == 0:
         return torch.empty_like(G)
-    g = G.detach().to(dtype)
+    g = G.detach().to(dtype).resolve_neg()  # the launches read its memory
     if family == "auto" and nat.ns_direct_supported(M, N, dtype) and n < 1 << 31:
         g = g.contiguous()
         out = torch.empty(G.shape, device=G.device, dtype=dtype)

@@ -61,6 +61,8 @@ def test_input_layouts(shape):
         assert torch.equal(newton_schulz(x), ref)
     d = newton_schulz(G.double())
     assert d.dtype == torch.float64 and torch.equal(d, ref.double())
+    neg = torch._neg_view(-G)  # contiguous, its memory holds -G
+    assert neg.is_neg() and neg.is_contiguous() and torch.equal(newton_schulz(neg), ref)
     p = G.clone().requires_grad_()
     assert torch.equal(newton_schulz(p), ref)
     nan = G.clone()
