@@ -300,26 +300,31 @@ extern "C" int himuon_ns5(uint16_t* x, uint16_t* y, const float* inv, int64_t n_
 
 // ---------------------------------------------------------------------------
 // One product on the faster block size. Rounds of 256 x 256 blocks (one per
-// CU) cost the same whether full or not, so r = blocks / CUs of them cost
+// CU) cost about the same whether full or not, so r = blocks / CUs of them cost
 // ceil(r); 64 x 64 and 128 x 128 blocks (two workgroups per CU) fill the chip
 // at any count at a lower rate, about 1.25 r for Apply and 1.3 r for a Gram
-// product; a Gram product on 128 x 128 blocks computes fewer elements (36 of 64
-// blocks against 10 of 16 at 1024), which makes it the faster one at any count
-// when M and K are large enough for its operand stream. Measured (us, smaller
-// blocks / 256 x 256): Apply of 28 1024 x 1024 (448 blocks) 76 / 66, of 7 1024 x
-// 2560 (280) 52 / 63, of one 1024 x 3072 (48) 15 / 30; GramA of 28 1024 x 1024
-// 43-48 / 63, of 56 1024 x 3072 229-235 / 264-302, of 4 4096 x 4096 326 / 340,
-// of one 1024 x 3072 24 / 75, of 128 512 x 512 (r = 1.5) 32 / 34, of 256 (r = 3)
-// 58 / 53, of 1,024 272 / 250, of 200 256 x 2048 (r = 0.78) 59 / 47.
+// product; a large Gram product on 128 x 128 blocks computes fewer elements (36 of
+// 64 blocks against 10 of 16 at 1024), and takes 1.26 r. Beyond three rounds the
+// 256 x 256 blocks are ahead, or 3 % behind, for every Gram product. Measured (us, smaller blocks / 256 x 256): Apply of 28 1024 x 1024 (448 blocks) 76 / 66,
+// of 7 1024 x 2560 (280) 52 / 63, of one 1024 x 3072 (48) 15 / 30; GramA of 20
+// 1024 x 1024 (r = 0.78) 40 / 35, of 28 (1.09) 43 / 62, of 50 (1.95) 78 / 69, of 60
+// (2.34) 86 / 94, of 80 (3.13) 133 / 121, of 340 (13.3) 537 / 478 (GramB 41 / 39,
+// 45 / 70, 79 / 80, 92 / 106, 133 / 137, 564 / 529), of 56 1024 x 3072 (2.19) 230 /
+// 245, of 150 610 / 570, of 3 4096 x 4096 (1.59) 240 / 220, of 12 (6.4) 968 / 819,
+// of one 1024 x 3072 24 / 75, of 128 512 x 512 (1.5) 32 / 34, of 256 (3) 58 / 53,
+// of 1,024 272 / 250, of 200 256 x 2048 (0.78) 59 / 47. Gram products of M >= 512
+// and K >= 1024 at any count on smaller blocks: the step of 340 tiles of 1024 x
+// 1024 11.68 ms against 10.97.
 // ---------------------------------------------------------------------------
 void ns_product(int mode, const NsProduct& g, hipStream_t s) {
   bool small = g.M % 256 || g.N % 256 || g.K % 256;
-  if (!small && mode != kApply && g.M >= 512 && g.K >= 1024) small = true;
   if (!small) {
     const int64_t nb = g.M / 256, cus = num_cus();
     const int64_t items = g.ntiles * (mode == kApply ? nb * (g.N / 256) : nb * (nb + 1) / 2);
     const double r = (double)items / cus;
-    small = (mode == kApply ? 1.25 : 1.3) * r < (double)((items + cus - 1) / cus);
+    const bool large = g.M >= 512 && g.K >= 1024 && r > 1.0;
+    const double rate = mode == kApply ? 1.25 : large ? 1.26 : 1.3;
+    small = rate * r < (double)((items + cus - 1) / cus) && (mode == kApply || r <= 3.0);
   }
   if (small) ns_blk_product(mode, g, s);
   else ns_stream_product(mode, g, s);

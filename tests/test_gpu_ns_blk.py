@@ -57,6 +57,7 @@ def test_blk_products(batch, M, N, round_once):
 
 @pytest.mark.parametrize("shape", [(3, 512, 512), (20, 512, 512), (40, 512, 512), (1024, 1024), (9, 1024, 1280),
                                    (70, 256, 512), (300, 256, 768), (16, 512, 1024),
+                                   (28, 1024, 1024), (50, 1024, 1024), (80, 1024, 1024),
                                    (2, 880, 1345), (1, 770, 768), (3, 2100, 700)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_block_size_choice_gives_the_256_blocks_bits(shape):
