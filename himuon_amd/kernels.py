@@ -70,18 +70,27 @@ def _padded(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
     return out
 
 
+def _span(t: torch.Tensor) -> "tuple[int, int]":
+    """First byte and end of the memory that t's elements lie in."""
+    p = t.data_ptr()
+    last = sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
+    return p, p + (last + 1) * t.element_size() if t.numel() else p
+
+
 def _result(out: torch.Tensor, shape: tuple, *operands: torch.Tensor) -> "torch.Tensor | None":
     """`out` itself where the kernel can write it: the unpadded shape on the
-    operands' device, contiguous and 16-byte aligned, in a storage of its own
-    (the kernels read their operands while they store). None: a scratch tensor
-    is written and copied to it, which also keeps copy_'s own checks for tensors
-    that require a gradient and for inference tensors."""
-    own = out.untyped_storage().data_ptr()
+    operands' device, contiguous and 16-byte aligned, in memory that no operand
+    reaches into (the kernels read their operands while they store; addresses
+    are compared, since tensors over one memory need not share a storage: DLPack
+    imports, for one). None: a scratch tensor is written and copied to it, which
+    also keeps copy_'s own checks for tensors that require a gradient and for
+    inference tensors."""
     if (tuple(out.shape) == shape and out.is_contiguous() and out.data_ptr() % 16 == 0 and not out.requires_grad
-            and not out.is_inference() and not out.is_neg()
-            and all(t.device == out.device and t.untyped_storage().data_ptr() != own for t in operands)):
-        torch.autograd.graph.increment_version(out)  # as the copy would
-        return out
+            and not out.is_inference() and not out.is_neg() and all(t.device == out.device for t in operands)):
+        lo, hi = _span(out)
+        if all(e <= lo or hi <= s for s, e in map(_span, operands)):
+            torch.autograd.graph.increment_version(out)  # as the copy would
+            return out
     return None
 
 

@@ -50,6 +50,22 @@ def test_out_in_the_operands_storage(dtype):
         assert torch.equal(call(operand), want)
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("shift", [0, 8, 64 * 128])
+def test_out_over_an_operands_memory_with_a_storage_of_its_own(dtype, shift):
+    shape, n = (2, 128, 128), 2 * 128 * 128
+    g = torch.Generator().manual_seed(5)
+    vals, b = ((torch.randn(shape, generator=g) / 128 ** 0.5).to(dtype).to(DEV) for _ in range(2))
+    for call in (lambda x, o: K.XXT(x, o), lambda x, o: K.ba_plus_cAA(x, 0.5, -1.5, o),
+                 lambda x, o: K.fused_bmm_add(b, x, 2.0, o), lambda x, o: K.fused_bmm_add(x, b, 2.0, o)):
+        want = call(vals, torch.empty_like(vals))
+        buf = torch.zeros(64 + n + shift, device=DEV, dtype=dtype)
+        x, out = buf[64: 64 + n].view(shape), torch.from_dlpack(buf[64 + shift: 64 + shift + n]).view(shape)
+        assert out.untyped_storage().data_ptr() != x.untyped_storage().data_ptr()
+        x.copy_(vals)
+        assert torch.equal(call(x, out), want)
+
+
 def test_out_that_requires_grad_and_inference_out_are_refused_as_before():
     shape, _, call = _calls(1, 128, 128, torch.float32)[0]
     with pytest.raises(RuntimeError):
