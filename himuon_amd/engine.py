@@ -16,6 +16,10 @@ device, allocated once so pointers stay stable for hipGraph capture:
 
 from __future__ import annotations
 
+import ctypes
+import functools
+import threading
+
 import torch
 
 from . import _native as nat
@@ -411,66 +415,110 @@ class AdamwTables:
 
 class _NsPlan:
     """Device state of ``newton_schulz`` for one (batch shape, dtype, device,
-    rounding form, kernel family): a tile group, the sub-batch and the NS
-    workspace, built once, and per step count a hipGraph of its launches
+    rounding form, kernel family): the tile buffers, the NS workspace and a
+    descriptor table of one entry, and per step count a hipGraph of the launches
     (gather, normaliser, NS, untile), captured on first use. The launches read
-    and write what the one descriptor of the group's device table points at:
-    ``xin`` and ``out`` until run() writes the call's own input and result
-    there, which then are gathered from and untiled into without a copy. A call
-    neither allocates device state (beyond the returned tensor) nor
-    synchronises, and costs two launches from the host instead of a dozen."""
+    and write what the descriptor points at, which run() sets to the call's own
+    input and result (a launch that carries the descriptor in its arguments), so
+    neither is copied. A call neither allocates device state (beyond the returned
+    tensor) nor synchronises, and costs two launches from the host instead of a
+    dozen.
+
+    Calls that use one plan must be ordered on one stream, each from its
+    descriptor write to its last launch: a later call's descriptor would
+    otherwise redirect this one's launches. newton_schulz() keeps a plan per
+    stream and per caller's capture, and holds a lock from the one to the other."""
 
     def __init__(self, n: int, M: int, N: int, dtype: torch.dtype, device, round_once: bool, family: str):
-        self.xin = torch.empty((n * M, N), device=device, dtype=dtype)
-        self.grp = TileGroup(
-            params=[self.xin], grads=[self.xin], moms=[None], tile_h=M, tile_w=N, upd_scales=[1.0],
-            mus=[0.0], nesterovs=[False], device=device, dtype=dtype, round_once=round_once, ns_family=family,
-        )
-        self.out = self.grp.updates[0]
-        d = self.desc = nat.ParamDesc()
-        d.h, d.w, d.ld_grad, d.ld_upd, d.R, d.C, d.upd_scale = n * M, N, N, N, n, 1, 1.0
-        self.sub_batch = self.grp.default_sub_batch()
-        self.ws = torch.empty(max(1, self.grp.workspace_bytes(self.sub_batch)), device=device, dtype=torch.uint8)
-        self.grp.tiles  # allocate the tile buffers now, not inside a capture
+        self.n, self.M, self.N, self.dtype = n, M, N, dtype
+        self.round_once, self.family = round_once, family
+        self.m, _, self.mp, self.np, _ = nat.ns_geometry(M, N)
+        self.ppt = nat.gather_partials_per_tile(M, N, self.mp, self.np)
+        self.sub_batch = nat.default_sub_batch(n, self.mp, self.np)
+
+        def buffer(shape, dt):
+            return torch.empty(shape, device=device, dtype=dt)
+
+        # (no host copy here: a plan may be built inside a caller's capture)
+        self.desc = buffer(ctypes.sizeof(nat.ParamDesc), torch.uint8)
+        self.tiles, self.alt = (buffer((n, self.mp, self.np), torch.bfloat16) for _ in range(2))
+        self.partials, self.inv = buffer((n, self.ppt), torch.float32), buffer(n, torch.float32)
+        self.ws = buffer(max(1, nat.ns5_workspace_bytes(self.sub_batch, self.mp, self.np)), torch.uint8)
         self.graphs: "dict[int, torch.cuda.CUDAGraph]" = {}
-        # recorded into a caller's graph: that graph holds these buffers'
-        # addresses, so the plan is never dropped
-        self.pinned = False
+
+    # an input and a result of the plan's own, for _launches() without others
+    @functools.cached_property
+    def xin(self) -> torch.Tensor:
+        return torch.empty((self.n * self.M, self.N), device=self.tiles.device, dtype=self.dtype)
+
+    @functools.cached_property
+    def out(self) -> torch.Tensor:
+        return torch.empty_like(self.xin)
+
+    def _point(self, G: torch.Tensor, out: torch.Tensor) -> None:
+        """The descriptor to G and out, as a launch: ordered after the launches of
+        earlier calls and before this one's."""
+        d = nat.ParamDesc()
+        d.grad, d.update = G.data_ptr(), out.data_ptr()
+        d.h, d.w, d.ld_grad, d.ld_upd, d.R, d.C, d.upd_scale = self.n * self.M, self.N, self.N, self.N, self.n, 1, 1.0
+        nat.write_desc(d, self.desc)
+
+    def _ns(self, steps: int) -> None:
+        """The launches from the input to the result that the descriptor points at."""
+        n, M, N, mp, np_ = self.n, self.M, self.N, self.mp, self.np
+        nat.momentum_gather(self.desc, 1, n, M, N, mp, np_, self.dtype, self.tiles, self.partials)
+        nat.tile_scale(self.partials, self.ppt, n, self.inv)
+        nat.ns5(self.tiles, self.alt, self.inv, n, mp, np_, steps, self.ws, self.sub_batch, family=self.family,
+                round_once=self.round_once, rows=self.m)
+        nat.untile(self.desc, 1, n, M, N, mp, np_, self.dtype, self.tiles if steps % 2 == 0 else self.alt)
 
     def _launches(self, steps: int) -> None:
-        g = self.grp
-        g.gather()
-        g.ns(0, g.n_tiles, steps, self.ws, self.sub_batch)
-        g.untile(steps)
+        """A call's launches, unrecorded, from xin to out."""
+        self._point(self.xin, self.out)
+        self._ns(steps)
 
-    def run(self, G: torch.Tensor, steps: int) -> torch.Tensor:
-        """newton_schulz of G (the plan's shape and dtype) as a new tensor."""
-        if not G.is_contiguous():
-            self.xin.view(G.shape).copy_(G)
-            G = self.xin.view(G.shape)
+    def run(self, G: torch.Tensor, steps: int, capturing: bool) -> torch.Tensor:
+        """newton_schulz of G (the plan's shape and dtype, contiguous) as a new
+        tensor; capturing: inside the caller's capture, which records the launches."""
         out = torch.empty(G.shape, device=G.device, dtype=G.dtype)
         graph = None
-        if torch.cuda.is_current_stream_capturing():
-            self.pinned = True  # inside the caller's capture: record the launches there
-        else:
+        if not capturing:
             graph = self.graphs.get(steps)
             if graph is None:
                 graph = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(graph):
-                    self._launches(steps)
+                    self._ns(steps)
                 self.graphs[steps] = graph
-        # stream-ordered: after the launches of an earlier call, before this one's
-        self.desc.grad, self.desc.update = G.data_ptr(), out.data_ptr()
-        nat.write_desc(self.desc, self.grp.desc)
+        self._point(G, out)
         if graph is None:
-            self._launches(steps)
+            self._ns(steps)
         else:
             graph.replay()
         return out
 
 
+# Plans in order of use, the latest last; a stream's calls keep the shapes they
+# used last, and the least recently used ones of all streams make room beyond
+# the total.
 _NS_PLANS: "dict[tuple, _NsPlan]" = {}
-_NS_PLANS_MAX = 8
+_NS_PLANS_MAX = 8  # per stream
+_NS_PLANS_TOTAL = 32
+_NS_LOCK = threading.RLock()
+
+
+def _ns_plan(stream: int, *spec) -> _NsPlan:
+    """The plan of `spec` (_NsPlan's arguments) for calls on `stream`."""
+    key = (stream, *spec)
+    plan = _NS_PLANS.pop(key, None)
+    if plan is None:
+        own = [k for k in _NS_PLANS if k[0] == stream]
+        if len(own) >= _NS_PLANS_MAX:
+            _NS_PLANS.pop(own[0])
+        elif len(_NS_PLANS) >= _NS_PLANS_TOTAL:
+            _NS_PLANS.pop(next(iter(_NS_PLANS)))
+        plan = _NsPlan(*spec)
+    _NS_PLANS[key] = plan
+    return plan
 
 
 def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torch.Tensor:
@@ -483,9 +531,12 @@ def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torc
     padding (himuon.py:263-284, test_kernels.py:176-198). A 2-D ``G`` takes
     the reference's 2-D rounding of the third product (torch.addmm,
     himuon.py:249-253); a batched one that of fused_bmm_add. The device state
-    for a shape is built on its first call and reused (at most _NS_PLANS_MAX
-    shapes are kept, the least recently used dropped first, except those
-    recorded into a caller's graph); the result is a new tensor.
+    for a shape is built on its first call on a stream and reused by the later
+    ones there (at most _NS_PLANS_MAX shapes per stream, _NS_PLANS_TOTAL in all,
+    the least recently used dropped first); calls on different streams share
+    none, so they may overlap, and calls of several threads on one stream follow
+    each other. A call inside a caller's capture has buffers of its own, in the
+    memory of that graph. The result is a new tensor.
     ``family``: the NS kernel family (comparison runs; "auto" otherwise)."""
     assert G.ndim >= 2
     if not G.is_cuda:
@@ -495,19 +546,13 @@ def newton_schulz(G: torch.Tensor, steps: int = 5, family: str = "auto") -> torc
     n = G.numel() // (M * N) if M * N else 0
     if n == 0:
         return torch.empty_like(G)
-    g = G.detach().to(dtype).resolve_neg()  # the launches read its memory
+    g = G.detach().to(dtype).resolve_neg().contiguous()  # the launches read its memory
     if family == "auto" and nat.ns_direct_supported(M, N, dtype) and n < 1 << 31:
-        g = g.contiguous()
         out = torch.empty(G.shape, device=G.device, dtype=dtype)
         nat.ns_direct(g, out, n, M, N, steps, round_once=G.ndim == 2)
         return out.to(G.dtype)
-    key = (n, M, N, dtype, G.device, G.ndim == 2, family)
-    plan = _NS_PLANS.pop(key, None)
-    if plan is None:
-        if len(_NS_PLANS) >= _NS_PLANS_MAX:
-            old = next((k for k, v in _NS_PLANS.items() if not v.pinned), None)
-            if old is not None:
-                _NS_PLANS.pop(old)
-        plan = _NsPlan(n, M, N, dtype, G.device, G.ndim == 2, family)
-    _NS_PLANS[key] = plan  # most recently used last
-    return plan.run(g, steps).to(G.dtype)
+    spec = (n, M, N, dtype, G.device, G.ndim == 2, family)
+    if torch.cuda.is_current_stream_capturing():
+        return _NsPlan(*spec).run(g, steps, True).to(G.dtype)
+    with _NS_LOCK:
+        return _ns_plan(nat._stream(), *spec).run(g, steps, False).to(G.dtype)
