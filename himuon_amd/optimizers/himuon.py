@@ -74,7 +74,8 @@ class HiMuon(Optimizer):
     # inside the last NS iteration (himuon_ns5_untile_apply)
     _fuse_ns_untile: bool = True
     # The AdamW groups' WD/LR runs inside their step (himuon_adamw_apply) for
-    # the parameters it takes; False keeps update tensors and the separate pass.
+    # the parameters it takes (_adamw_fusable); False keeps update tensors and
+    # the separate pass (same parameters, bit for bit).
     _fuse_adamw: bool = True
     # NS kernel family of every tile group (a key of _native.NS_FAMILIES):
     # "auto", the per-geometry choice; the others are comparison runs, which
@@ -349,12 +350,25 @@ class HiMuon(Optimizer):
             update = self._compute_adamw_step(p, p.grad, group["adamw_betas"], group["adamw_eps"])
             self._apply_wd_and_update(p, update, weight_decay, lr, group_idx)
 
-    def _prepare_adamw(self):
+    def _adamw_fusable(self, p, graph: bool) -> bool:
+        """Whether p's WD/LR may run inside its AdamW step without changing a bit
+        (if the kernel takes p at all: AdamwTables.applies). himuon_adamw_apply
+        does the arithmetic of himuon_apply_updates, the separate pass of a
+        captured step (graph). The separate pass of an eager step is torch's mul_
+        and add_, which agree for fp32 parameters and for bf16 ones with bf16
+        grads. An update of another dtype than its 16-bit parameter keeps its own
+        precision in parts of torch's add (the tail of a tensor, the whole of a
+        small one) where the kernel rounds it to the parameter's, and torch rounds
+        an fp16 add in more than one way."""
+        return (self._fuse_adamw and not self._is_dtensor(p)
+                and (graph or p.dtype == torch.float32 or p.dtype == p.grad.dtype == torch.bfloat16))
+
+    def _prepare_adamw(self, graph: bool):
         """State (as the reference creates it: fp32 device step, zero moments in
         the grad dtype) and the device tables of the fused AdamW step for every
         AdamW-group parameter with a grad; persistent update buffers for those
-        whose WD/LR the step cannot apply itself. Runs outside graph capture;
-        returns the list of (param, group_idx)."""
+        whose WD/LR the step cannot apply itself. graph: for a captured step. Runs
+        outside graph capture; returns the list of (param, group_idx)."""
         params = []
         for group_idx, group in enumerate(self.param_groups):
             if group["use_muon"]:
@@ -372,14 +386,14 @@ class HiMuon(Optimizer):
         sig = tuple(
             (id(p), self._local(p).data_ptr(), p.grad.data_ptr(), p.grad.dtype, self.state[p]["moment1"].data_ptr(), gi)
             for p, gi in params
-        ) + (self._fuse_adamw,)
+        ) + (self._fuse_adamw, graph)
         if sig != self._adamw_sig:
             self._adamw_sig = sig
             entries, fuse = [], []
             for p, gi in params:
                 g, st, u = p.grad, self.state[p], self._adamw_updates.get(p)
                 e = (g, st["moment1"], st["moment2"], u, st["step"], gi)
-                fuse.append(p.data if self._fuse_adamw and not self._is_dtensor(p) else None)
+                fuse.append(p.data if self._adamw_fusable(p, graph) else None)
                 if AdamwTables.applies(e, fuse[-1]):
                     self._adamw_updates.pop(p, None)
                 elif u is None or u.shape != g.shape or u.dtype != g.dtype or u.device != g.device:
@@ -397,7 +411,7 @@ class HiMuon(Optimizer):
         Parameters it cannot take get their update from himuon_adamw_step or
         the reference's torch ops, and then the reference's WD/LR path (deferred
         to after replay in graph mode)."""
-        params = self._prepare_adamw()
+        params = self._prepare_adamw(self._in_graph_region)
         if not params:
             return
         tables = self._adamw_tables
@@ -840,7 +854,7 @@ class HiMuon(Optimizer):
         from the device table step() rewrites before each replay; the
         remaining updates get theirs after replay."""
         self._ensure_device_state()  # allocate everything before capture
-        self._prepare_adamw()
+        self._prepare_adamw(graph=True)
         torch.cuda.synchronize()
         self._pending_updates.clear()
         self._apply_tables = None

@@ -2,7 +2,8 @@
 moments, step counters and parameters bit-identical to himuon_adamw_step
 followed by himuon_apply_updates, for every dtype pair, sizes around the
 8-element vectors and the chunks, and two groups; and at the optimizer level
-over steps with a changing learning rate, eager and captured."""
+over steps with a changing learning rate and over every dtype pair, eager and
+captured."""
 
 from __future__ import annotations
 
@@ -17,6 +18,7 @@ if torch.cuda.is_available():
     from himuon_amd.optimizers.himuon import HiMuon
 
 DEV = "cuda"
+F32, BF16 = torch.float32, torch.bfloat16
 DTYPES = [torch.float32, torch.bfloat16, torch.float16]
 BITS = {2: torch.int16, 4: torch.int32}
 SCALE, ALPHA = [1 - 0.02 * 0.1, 1.0], [-0.02, -0.003]
@@ -79,6 +81,40 @@ def test_optimizer_with_and_without(cuda_graph):
     # (eager, unfused: torch's own adds, the same arithmetic where the dtypes agree)
     for a, b in zip(*runs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("cuda_graph", [False, True], ids=["eager", "captured"])
+@pytest.mark.parametrize("gdt", DTYPES)
+@pytest.mark.parametrize("pdt", DTYPES)
+def test_optimizer_of_mixed_dtypes(pdt, gdt, cuda_graph):
+    """Every pair of parameter and grad dtype, on norms, odd lengths, tails and a
+    length that torch's vectorised add covers: the parameters of the step with
+    and without the WD/LR inside it, which in an eager step is torch's own two
+    ops on an update of the grad's dtype."""
+    gen = torch.Generator().manual_seed(6)
+    shapes = [(1,), (7,), (64,), (1000,), (33, 5), (4097,), (1 << 16,), (999, 64)]
+    vals = [torch.randn(*s, generator=gen) * 0.02 for s in shapes]
+    runs = []
+    for fuse in (True, False):
+        ps = [torch.nn.Parameter(v.to(pdt).to(DEV)) for v in vals]
+        for p in ps:
+            if pdt != gdt:
+                p.grad_dtype = gdt
+            p.grad = torch.zeros(p.shape, dtype=gdt, device=DEV)
+        opt = HiMuon([{"params": ps[::2], "use_muon": False, "lr": 2e-2, "weight_decay": 0.1},
+                      {"params": ps[1::2], "use_muon": False, "lr": 1e-2, "weight_decay": 0.0}],
+                     lr=0.02, tile_size=128, cuda_graph=cuda_graph, cuda_graph_warmup=1)
+        opt._fuse_adamw = fuse
+        gg = torch.Generator().manual_seed(4)
+        for _ in range(4):
+            for p in ps:
+                p.grad.copy_(torch.randn(p.shape, generator=gg).to(gdt))
+            opt.step()
+        fused = fuse and (cuda_graph or pdt == F32 or pdt == gdt == BF16)
+        assert len(opt._adamw_updates) == (0 if fused else len(ps))
+        runs.append(ps)
+    for a, b in zip(*runs):
+        assert torch.equal(a.view(BITS[a.element_size()]), b.view(BITS[b.element_size()])), tuple(a.shape)
 
 
 def test_adamw_apply_argument_errors():
