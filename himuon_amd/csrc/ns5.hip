@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kThreads) void ns_scale_kernel(uint16_t* __restrict
                                                             int64_t vec_per_tile, int64_t wgs_per_tile) {
   const int64_t t = blockIdx.x / wgs_per_tile;
   const int64_t v0 = (blockIdx.x - t * wgs_per_tile) * (kThreads * kScaleVec) + threadIdx.x;
-  u32x4_t* const x = reinterpret_cast<u32x4_t*>(X) + t * vec_per_tile;
+  u32x4_any* const x = reinterpret_cast<u32x4_any*>(X) + t * vec_per_tile;  // (any alignment, as load8)
   const float s = inv[t];
   u32x4_t v[kScaleVec];
 #pragma unroll
@@ -104,7 +104,9 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   const bool few_rows = family == HIMUON_NS_FAMILY_AUTO && ns5_small_supported(rows, mp, np);
   const bool st = ns5_stream_supported(mp, np) && !small;
   const bool lds = ns5_lds_supported(mp, np) && !small;
-  const bool ba = ns5_ba_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
+  // (buffers off 16-byte boundaries: ns_any_product on X0, no fused pair)
+  const bool aligned = dma_aligned(x, y, workspace);
+  const bool ba = ns5_ba_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO && (aligned || untile);
   const bool reg = ns5_reg_supported(mp, np) && family == HIMUON_NS_FAMILY_AUTO;
 
   // Matrices of many blocks: the products of the first iteration would scale
@@ -114,7 +116,8 @@ int ns5_impl(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles, int mp
   // against 3.91-3.95 ms, of 12 of 896 x 2432 0.66-0.67 against 0.68-0.69, of 60
   // of 768 x 768 0.92-0.93 against 0.93-0.94; from 512 rows on, 400 of 512 x 768
   // would be slower (2.65 against 2.56-2.60 ms).
-  const bool scale_first = !few_rows && family == HIMUON_NS_FAMILY_AUTO && mp >= kScaleRows;
+  const bool scale_first = !few_rows && !lds && !reg &&
+                           ((family == HIMUON_NS_FAMILY_AUTO && mp >= kScaleRows) || !aligned);
   for (int64_t s0 = 0; s0 < n_tiles; s0 += sb) {
     const int64_t cnt = std::min<int64_t>(sb, n_tiles - s0);
     const int64_t o = s0 * rect;

@@ -321,6 +321,7 @@ void launch(int mode, const NsProduct& g, hipStream_t s) {
 // of 256 rows with K = 256 stay short enough for 64 x 64 (10 of 16 blocks
 // computed instead of 3 of 4): 512 of them 29.5 against 34.7 us.
 void ns_blk_product(int mode, const NsProduct& g, hipStream_t s) {
+  if (!dma_aligned(g.P, g.Q, g.R)) return ns_any_product(mode, g, s);
   const int64_t nbi = g.M / 128, nbj = g.N / 128;
   const int64_t items = g.ntiles * (mode == kApply ? nbi * nbj : nbi * (nbi + 1) / 2);
   const bool short_gram = mode != kApply && g.K <= 256 && items < (1 << 21);  // a grid holds 2^24 workgroups

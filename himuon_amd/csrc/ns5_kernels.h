@@ -220,10 +220,16 @@ struct NsProduct {
 };
 // On 256 x 256 blocks (ns5_stream.hip; M, N, K multiples of 256), on 64 x 64
 // or 128 x 128 blocks (ns5_blk.hip; multiples of 128), and on whichever is
-// faster for the shape (ns5.hip). All give the same bits.
+// faster for the shape (ns5.hip). Their direct-to-LDS loads read operands on
+// 16-byte boundaries; others (inv null, batches contiguous) go through registers
+// (ns_any_product, products.hip). All give the same bits.
 void ns_stream_product(int mode, const NsProduct& g, hipStream_t s);
 void ns_blk_product(int mode, const NsProduct& g, hipStream_t s);
 void ns_product(int mode, const NsProduct& g, hipStream_t s);
+void ns_any_product(int mode, const NsProduct& g, hipStream_t s);
+inline bool dma_aligned(const void* a, const void* b, const void* c) {
+  return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 15) == 0;
+}
 
 // CUs of the current device, queried per launch (a host-side attribute lookup;
 // nothing is cached in the library).

@@ -621,6 +621,7 @@ void launch(const StArgs& a, int64_t items, hipStream_t s) {
 bool ns5_stream_supported(int mp, int np) { return mp % BT == 0 && np % BT == 0; }
 
 void ns_stream_product(int mode, const NsProduct& g, hipStream_t s) {
+  if (!dma_aligned(g.P, g.Q, g.R)) return ns_any_product(mode, g, s);
   const int nb = g.M / BT;
   const int64_t gram = g.ntiles * (nb * (nb + 1) / 2), apply = g.ntiles * nb * (g.N / BT);
   if (mode == kApply) {

@@ -22,7 +22,8 @@
 //
 // The bf16-in / bf16-out products keep their own kernels (ns5_blk.hip,
 // ns5_stream.hip), bit-identical to torch; these kernels serve every other
-// dtype pair. Block tile 64 x 64 x 64, four waves of one MFMA 32x32 tile each;
+// dtype pair, and bf16 operands off 16-byte boundaries (ns_any_product: the same
+// bits), which those kernels' direct-to-LDS loads do not take. Block tile 64 x 64 x 64, four waves of one MFMA 32x32 tile each;
 // operands are converted as they are staged through registers into a double
 // buffer in LDS; the Gram products compute the lower blocks and store each block
 // and its mirror.
@@ -63,7 +64,8 @@ HM_DEV f32x16_t mfma_in(u32x4_t a, u32x4_t b, f32x16_t c) {
 }
 
 // 8 consecutive input elements as 16-bit MFMA operands: `hi` always, `lo`
-// (the fp32 remainder) for fp32 inputs.
+// (the fp32 remainder) for fp32 inputs. (fp32 and 16-bit operands at any element
+// alignment, as load8.)
 struct Oct {
   u32x4_t hi, lo;
 };
@@ -78,8 +80,8 @@ HM_DEV Oct load_oct(const void* base, int64_t idx) {
   Oct o;
   if constexpr (IN == kInF32) {
     const float* p = static_cast<const float*>(base) + idx;
-    const f32x4_t v0 = *reinterpret_cast<const f32x4_t*>(p);
-    const f32x4_t v1 = *reinterpret_cast<const f32x4_t*>(p + 4);
+    const f32x4_any v0 = *reinterpret_cast<const f32x4_any*>(p);
+    const f32x4_any v1 = *reinterpret_cast<const f32x4_any*>(p + 4);
     float x[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -93,7 +95,7 @@ HM_DEV Oct load_oct(const void* base, int64_t idx) {
     o.hi = u32x4_t{e5m2_pair(w[0], 0), e5m2_pair(w[0], 1), e5m2_pair(w[1], 0), e5m2_pair(w[1], 1)};
     o.lo = u32x4_t{0u, 0u, 0u, 0u};
   } else {
-    o.hi = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(base) + idx);
+    o.hi = *reinterpret_cast<const u32x4_any*>(static_cast<const uint16_t*>(base) + idx);
     o.lo = u32x4_t{0u, 0u, 0u, 0u};
   }
   return o;
@@ -245,14 +247,15 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
 }
 
 // C = out(Bm X) + gamma X for each batch entry (Bm X rounded to the output
-// dtype before the add: fused_bmm_add.py:73-88); Bm: M x M, X and C: M x N.
+// dtype before the add, fused_bmm_add.py:73-88, unless round_once); Bm: M x M, X
+// and C: M x N.
 // X is the MFMA B operand with the contraction along its rows: each 4 x 8
 // block of X is transposed into the k-octet-major LDS layout sX[k/8][j][k%8].
 template <int IN>
 __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __restrict__ Bm,
                                                               const void* __restrict__ X, void* __restrict__ C,
                                                               int M, int N, int64_t first, int64_t count,
-                                                              float gamma, int out_dtype) {
+                                                              float gamma, int round_once, int out_dtype) {
   constexpr int NP = planes(IN);
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][NP][BT * kLd];
   __shared__ __attribute__((aligned(16))) uint16_t sX[2][NP][(BK / 8) * BT * 8];
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __rest
     const int i = bi * BT + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
     const int j = bj * BT + wn * 32 + (lane & 31);
     const int64_t e = x0 + (int64_t)i * N + j;
-    const float bx = round_out(acc[r], out_dtype);
+    const float bx = round_once ? acc[r] : round_out(acc[r], out_dtype);
     store_out(C, e, bx + gamma * load_elem_in<IN>(X, e), out_dtype);
   }
 }
@@ -363,13 +366,13 @@ void launch_gram(const void* s, void* c, int M, int K, int64_t batch, float alph
 }
 
 template <int IN>
-void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int od,
-                  hipStream_t st) {
+void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int round_once,
+                  int od, hipStream_t st) {
   const int64_t items = batch * (M / BT) * (N / BT);
   for (int64_t first = 0; first < items; first += kLaunchItems) {
     const int64_t count = std::min(kLaunchItems, items - first);
     hipLaunchKernelGGL(prod_apply_kernel<IN>, dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, b, x, c, M, N,
-                       first, count, gamma, od);
+                       first, count, gamma, round_once, od);
   }
 }
 
@@ -396,6 +399,13 @@ int gram(const void* s, void* c, int M, int K, int64_t batch, float alpha, float
 
 }  // namespace
 
+void ns_any_product(int mode, const NsProduct& g, hipStream_t s) {
+  if (mode == kApply)
+    launch_apply<kInBf16>(g.P, g.Q, g.C, g.M, g.N, g.ntiles, g.beta, g.round_once, HIMUON_DTYPE_BF16, s);
+  else
+    launch_gram<kInBf16>(g.P, g.C, g.M, g.K, g.ntiles, g.alpha, g.beta, mode == kGramB, HIMUON_DTYPE_BF16, s);
+}
+
 extern "C" int himuon_xxt_typed(const void* x, void* out, int64_t batch, int M, int K, int in_dtype,
                                 int out_dtype, void* stream) {
   return gram(x, out, M, K, batch, 1.f, 0.f, 0, in_dtype, out_dtype, stream);
@@ -416,10 +426,10 @@ extern "C" int himuon_bmm_add_typed(const void* b, const void* x, void* out, int
   if (batch > kMaxItems / blocks) return HIMUON_EINVAL;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   switch (in_dtype) {
-    case HIMUON_DTYPE_F32: launch_apply<kInF32>(b, x, out, M, N, batch, a, out_dtype, st); break;
-    case HIMUON_DTYPE_BF16: launch_apply<kInBf16>(b, x, out, M, N, batch, a, out_dtype, st); break;
-    case HIMUON_DTYPE_F16: launch_apply<kInF16>(b, x, out, M, N, batch, a, out_dtype, st); break;
-    default: launch_apply<kInE5m2>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    case HIMUON_DTYPE_F32: launch_apply<kInF32>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
+    case HIMUON_DTYPE_BF16: launch_apply<kInBf16>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
+    case HIMUON_DTYPE_F16: launch_apply<kInF16>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
+    default: launch_apply<kInE5m2>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
   }
   return (int)hipGetLastError();
 }

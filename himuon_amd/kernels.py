@@ -62,9 +62,11 @@ def _bytes_view(t: torch.Tensor) -> torch.Tensor:
 
 
 def _padded(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
-    """(B, r, c) -> contiguous (B, rows, cols) with zero padding (or t itself)."""
+    """(B, r, c) -> contiguous (B, rows, cols) with zero padding (or t itself).
+    A bf16 operand off 16-byte boundaries is copied too: its kernels load straight
+    into LDS there and take the slower way through registers otherwise."""
     if t.shape[-2:] == (rows, cols) and t.is_contiguous():
-        return t
+        return t.clone() if t.dtype == torch.bfloat16 and t.data_ptr() % 16 else t
     out = torch.zeros((t.shape[0], rows, cols), device=t.device, dtype=t.dtype)
     _bytes_view(out)[:, : t.shape[-2], : t.shape[-1]] = _bytes_view(t)
     return out

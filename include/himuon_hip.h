@@ -140,7 +140,8 @@ size_t himuon_ns5_workspace_bytes(int64_t sub_batch, int mp, int np);
  * in x when `steps` is even and in y when it is odd (the other buffer's
  * contents are unspecified afterwards; x and y must not alias). X0 is formed
  * by the first iteration's kernels as they read x, or, for three products of
- * mp >= 768, written over x by one pass before them.
+ * mp >= 768, written over x by one pass before them. Buffers that are not on
+ * 16-byte boundaries give the same result, more slowly.
  * Tiles with mp == 128 and np in {128, 256, 512} run all iterations
  * of a tile inside one workgroup's LDS, 256 x 256 tiles with X in registers; more
  * than 16 512 x 512 tiles run the first product on a persistent 256x256-block
@@ -208,7 +209,8 @@ int himuon_ns5_ex(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles,
  * M, N, K multiples of HIMUON_NS_ALIGN (pad with zeros: zero rows and columns
  * are exact). `flags` takes a kernel family (HIMUON_NS_FAMILY_*) and, for
  * himuon_bmm_add, HIMUON_NS_ROUND_ONCE. Outputs must not alias inputs. The
- * Gram outputs are exactly symmetric.
+ * Gram outputs are exactly symmetric. Operands that are not on 16-byte
+ * boundaries give the same bits, more slowly.
  */
 int himuon_xxt(const uint16_t* x, uint16_t* out, int64_t batch, int M, int K,
                int flags, void* stream);
@@ -251,8 +253,8 @@ int himuon_bmm_add(const uint16_t* b, const uint16_t* x, uint16_t* out,
  * counterpart: it equals ba_plus_cAA (ba_plus_cAA.py:90-120) followed by
  * fused_bmm_add (fused_bmm_add.py:98-135), bit for bit. A: (batch, 512, 512)
  * bf16, exactly symmetric (an XXT output); X, out: (batch, 512, 512) bf16;
- * M == N == 512, batch < 2^29 (32-bit work-item indices; larger batches
- * return HIMUON_EINVAL); `flags` takes only HIMUON_NS_ROUND_ONCE.
+ * M == N == 512, on 16-byte boundaries, batch < 2^29 (32-bit work-item indices;
+ * larger batches return HIMUON_EINVAL); `flags` takes only HIMUON_NS_ROUND_ONCE.
  */
 int himuon_ba_bmm_add(const uint16_t* a, const uint16_t* x, uint16_t* out,
                       int64_t batch, int M, int N, float alpha, float beta,
@@ -375,7 +377,8 @@ int himuon_untile_apply(const HimuonParamDesc* params_dev, int n_params,
  * Supported (else HIMUON_EINVAL, nothing launched; the caller runs the two
  * calls instead) for 512 x 512 NS tiles (mp == np == 512) that are not
  * transposed (tile_h <= tile_w), family AUTO, steps >= 2 and fp32 or bf16
- * parameters; himuon_ns5_untile_apply_supported answers for a geometry.
+ * parameters; himuon_ns5_untile_apply_supported answers for a geometry. x, y and
+ * the workspace lie on 16-byte boundaries.
  * Replaces newton_schulz + _post_ns_per_param + the Muon parameters'
  * outside-graph WD/LR of one chunk (himuon.py:232-284, 315-348, 215-228).
  */

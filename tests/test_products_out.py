@@ -1,12 +1,13 @@
 """Which ``out`` the kernel API writes without a scratch tensor: never one whose
-memory an operand reaches into, however the two tensors came to share it."""
+memory an operand reaches into, however the two tensors came to share it. And
+which operands it hands on uncopied: no bf16 one off a 16-byte boundary."""
 
 from __future__ import annotations
 
 import pytest
 import torch
 
-from himuon_amd.kernels import _result, _span
+from himuon_amd.kernels import _padded, _result, _span
 
 M = 128
 SHAPE = (1, M, M)
@@ -40,3 +41,13 @@ def test_a_strided_operand_around_out():
     assert _result(out, SHAPE, wide[..., :M]) is None
     assert _span(wide[..., :M])[1] - wide.data_ptr() == 4 * (2 * M * M - M)
     assert _span(torch.empty(0, M, M)) == (0, 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("off", [0, 1, 4, 8])
+def test_operands_handed_to_the_kernels(dtype, off):
+    t = _aligned(M * M + 8).to(dtype)
+    t = t[-t.data_ptr() % 16 // t.element_size():][off: off + 64 * 128].view(1, 64, 128).normal_()
+    got = _padded(t, 64, 128)
+    assert torch.equal(got, t) and (got is t) == (dtype == torch.float32 or off % 8 == 0)
+    assert dtype == torch.float32 or got.data_ptr() % 16 == 0
