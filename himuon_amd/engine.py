@@ -25,6 +25,25 @@ import torch
 from . import _native as nat
 
 
+def mem_span(t: torch.Tensor) -> "tuple[int, int]":
+    """First byte and end of the memory that t's elements lie in."""
+    p = t.data_ptr()
+    last = sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
+    return p, p + (last + 1) * t.element_size() if t.numel() else p
+
+
+def sharing(tensors) -> "set[int]":
+    """Indexes of the tensors whose memory another of them reaches into."""
+    spans = sorted((*mem_span(t), i) for i, t in enumerate(tensors))
+    out, top, end = set(), -1, -1  # top: the tensor that reaches furthest so far
+    for lo, hi, i in spans:
+        if lo < min(hi, end):
+            out |= {i, top}
+        if hi > end:
+            top, end = i, hi
+    return out
+
+
 def update_dtype(params, grad_dtype: torch.dtype) -> torch.dtype:
     """Storage dtype of a group's update tensors. The update's only consumer
     is the WD/LR application, which (as torch's in-place add does) first rounds

@@ -35,7 +35,7 @@ from __future__ import annotations
 import torch
 
 from . import _native as nat
-from .engine import newton_schulz as _newton_schulz
+from .engine import mem_span as _span, newton_schulz as _newton_schulz
 
 __all__ = ("XXT", "ba_plus_cAA", "fused_bmm_add", "ns5_smem")
 
@@ -70,13 +70,6 @@ def _padded(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
     out = torch.zeros((t.shape[0], rows, cols), device=t.device, dtype=t.dtype)
     _bytes_view(out)[:, : t.shape[-2], : t.shape[-1]] = _bytes_view(t)
     return out
-
-
-def _span(t: torch.Tensor) -> "tuple[int, int]":
-    """First byte and end of the memory that t's elements lie in."""
-    p = t.data_ptr()
-    last = sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
-    return p, p + (last + 1) * t.element_size() if t.numel() else p
 
 
 def _result(out: torch.Tensor, shape: tuple, *operands: torch.Tensor) -> "torch.Tensor | None":

@@ -33,7 +33,7 @@ import torch
 from torch.optim import Optimizer
 
 from .. import _native as nat
-from ..engine import AdamwTables, ApplyTables, TileGroup, update_dtype
+from ..engine import AdamwTables, ApplyTables, TileGroup, sharing, update_dtype
 from ..engine import newton_schulz as _hip_newton_schulz
 
 try:
@@ -390,10 +390,13 @@ class HiMuon(Optimizer):
         if sig != self._adamw_sig:
             self._adamw_sig = sig
             entries, fuse = [], []
-            for p, gi in params:
+            # parameters over one memory (weights tied by their data) are updated one
+            # after the other, as their order is, not side by side in one launch
+            shared = sharing([self._local(p) for p, _ in params])
+            for k, (p, gi) in enumerate(params):
                 g, st, u = p.grad, self.state[p], self._adamw_updates.get(p)
                 e = (g, st["moment1"], st["moment2"], u, st["step"], gi)
-                fuse.append(p.data if self._adamw_fusable(p, graph) else None)
+                fuse.append(p.data if k not in shared and self._adamw_fusable(p, graph) else None)
                 if AdamwTables.applies(e, fuse[-1]):
                     self._adamw_updates.pop(p, None)
                 elif u is None or u.shape != g.shape or u.dtype != g.dtype or u.device != g.device:

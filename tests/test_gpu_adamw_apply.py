@@ -117,6 +117,31 @@ def test_optimizer_of_mixed_dtypes(pdt, gdt, cuda_graph):
         assert torch.equal(a.view(BITS[a.element_size()]), b.view(BITS[b.element_size()])), tuple(a.shape)
 
 
+@pytest.mark.parametrize("pdt,gdt", [(F32, F32), (BF16, BF16), (F32, BF16)])
+def test_parameters_over_one_memory_are_updated_in_turn(pdt, gdt):
+    """Weights tied by their data (two Parameters over one tensor, and one that
+    overlaps it in part): each one's decay and update, in order, as torch's ops
+    apply them; their neighbours stay in the fused pass."""
+    n = 6000
+    runs = []
+    for fuse in (True, False):
+        gen = torch.Generator().manual_seed(8)
+        data = (torch.randn(3 * n, generator=gen) * 0.02).to(pdt).to(DEV)
+        ps = [torch.nn.Parameter(d) for d in (data[:n], data[:n], data[n // 2: n // 2 + n], data[2 * n:])]
+        for p in ps:
+            if pdt != gdt:
+                p.grad_dtype = gdt
+            p.grad = torch.randn(n, generator=gen).to(gdt).to(DEV)
+        opt = HiMuon([{"params": ps, "use_muon": False, "lr": 2e-2, "weight_decay": 0.1}], lr=0.02, tile_size=128,
+                     cuda_graph=False)
+        opt._fuse_adamw = fuse
+        for _ in range(3):
+            opt.step()
+        assert [a for a in opt._adamw_tables.applied] == [False, False, False, fuse]
+        runs.append(data)
+    assert torch.equal(*runs)
+
+
 def test_adamw_apply_argument_errors():
     import ctypes
 
