@@ -384,7 +384,8 @@ class HiMuon(Optimizer):
                     st["moment2"] = torch.zeros_like(g)
                 params.append((p, group_idx))
         sig = tuple(
-            (id(p), self._local(p).data_ptr(), p.grad.data_ptr(), p.grad.dtype, self.state[p]["moment1"].data_ptr(), gi)
+            (id(p), self._local(p).data_ptr(), p.dtype, p.stride(), p.grad.data_ptr(), p.grad.dtype,
+             self.state[p]["moment1"].data_ptr(), gi)
             for p, gi in params
         ) + (self._fuse_adamw, graph)
         if sig != self._adamw_sig:

@@ -142,6 +142,25 @@ def test_parameters_over_one_memory_are_updated_in_turn(pdt, gdt):
     assert torch.equal(*runs)
 
 
+def test_a_parameter_whose_layout_changes_between_steps():
+    """The same memory with other strides (``p.data = p.data.t()``): the update is
+    added element by element, as torch's ops do, not in the old layout."""
+    runs = []
+    for fuse in (True, False):
+        gen = torch.Generator().manual_seed(9)
+        p = torch.nn.Parameter((torch.randn(96, 96, generator=gen) * 0.02).to(DEV))
+        p.grad = torch.randn(96, 96, generator=gen).to(DEV)
+        opt = HiMuon([{"params": [p], "use_muon": False, "lr": 2e-2, "weight_decay": 0.1}], lr=0.02, tile_size=128,
+                     cuda_graph=False)
+        opt._fuse_adamw = fuse
+        opt.step()
+        p.data = p.data.t()
+        opt.step()
+        assert opt._adamw_tables.applied == [False]
+        runs.append(p.data)
+    assert torch.equal(*runs)
+
+
 def test_adamw_apply_argument_errors():
     import ctypes
 
