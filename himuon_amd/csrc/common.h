@@ -177,6 +177,17 @@ inline int64_t xcd_grid(int64_t total) {
   return per_xcd * kNumXcd;
 }
 
+// A grid holds fewer than 2^32 threads: workgroups of `threads` per launch.
+constexpr int64_t launch_wgs(int threads) { return (int64_t)0xffffffff / threads; }
+
+// run(off, n) for off .. off + n - 1 of `cnt` items, one workgroup each, n the
+// most that a launch takes.
+template <class F>
+void per_launch(int64_t cnt, int threads, F&& run) {
+  const int64_t most = launch_wgs(threads);
+  for (int64_t off = 0; off < cnt; off += most) run(off, std::min(cnt - off, most));
+}
+
 // Find the parameter owning tile t: the last p with params[p].tile0 <= t.
 HM_DEV int find_param(const HimuonParamDesc* __restrict__ params, int n_params, int64_t t) {
   int lo = 0, hi = n_params - 1;

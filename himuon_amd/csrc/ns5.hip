@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kThreads) void ns_scale_kernel(uint16_t* __restrict
 
 void ns_scale(uint16_t* x, const float* inv, int64_t n_tiles, int64_t rect, hipStream_t s) {
   const int64_t vpt = rect / 8, wgs = (vpt + kThreads * kScaleVec - 1) / (kThreads * kScaleVec);
-  const int64_t most = ((int64_t)1 << 30) / wgs;  // tiles per launch
+  const int64_t most = std::max<int64_t>(1, launch_wgs(kThreads) / wgs);  // tiles per launch
   for (int64_t t = 0; t < n_tiles; t += most)
     hipLaunchKernelGGL(ns_scale_kernel, dim3((unsigned)(std::min(most, n_tiles - t) * wgs)), dim3(kThreads), 0, s,
                        x + t * rect, inv + t, vpt, wgs);

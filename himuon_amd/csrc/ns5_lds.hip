@@ -473,9 +473,12 @@ __global__ __launch_bounds__(NT, 3) void ns_direct_lds_kernel(const void* __rest
 
 void ns_direct_lds_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
                        float b, float c, float eps, bool round_once, hipStream_t s) {
+  const int64_t bytes = (int64_t)rows * cols * (dtype == HIMUON_DTYPE_F32 ? 4 : 2);
   const auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)cnt), dim3(NT), 0, s, g, out, cnt, rows, cols, steps, a, b, c, eps,
-                       round_once ? 1 : 0);
+    per_launch(cnt, NT, [&](int64_t off, int64_t n) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(NT), 0, s, static_cast<const char*>(g) + off * bytes,
+                         static_cast<char*>(out) + off * bytes, n, rows, cols, steps, a, b, c, eps, round_once ? 1 : 0);
+    });
   };
   switch (dtype) {
     case HIMUON_DTYPE_F32: run(ns_direct_lds_kernel<HIMUON_DTYPE_F32>); break;
@@ -493,11 +496,10 @@ bool lds_step_supported(int tile_h, int tile_w, int dtype, int param_dtype) {
 void lds_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
                   int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
                   bool round_once, const float* sa, hipStream_t s) {
-  // one workgroup per tile, in launches of at most 2^30 workgroups
+  // one workgroup per tile
   const int ro = round_once ? 1 : 0;
   const dim3 block(NT);
-  for (int64_t off = 0; off < cnt; off += (int64_t)1 << 30) {
-    const int64_t n = std::min<int64_t>(cnt - off, (int64_t)1 << 30);
+  per_launch(cnt, NT, [&](int64_t off, int64_t n) {
     const dim3 grid((unsigned)n);
 #define HM_LDS_STEP(D, PD)                                                                                    \
   hipLaunchKernelGGL((lds_step_kernel<D, PD>), grid, block, 0, s, params, n_params, tile_begin + off, n, tile_h, \
@@ -509,7 +511,7 @@ void lds_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begi
       if (param_dtype == HIMUON_DTYPE_F32) HM_LDS_STEP(HIMUON_DTYPE_BF16, HIMUON_DTYPE_F32);
       else HM_LDS_STEP(HIMUON_DTYPE_BF16, HIMUON_DTYPE_BF16);
     }
-  }
+  });
 #undef HM_LDS_STEP
 }
 
@@ -519,10 +521,10 @@ void ns5_lds_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int mp
                  float a, float b, float c, bool round_once, hipStream_t s) {
   (void)mp;
   uint16_t* out = (steps & 1) ? y : x;
-  // np = 128: one workgroup per tile (up to 2^30 per launch; the kernel's tile
-  // loop takes the rest), 4 % faster than persistent workgroups; wider tiles:
+  // np = 128: one workgroup per tile (up to what a launch holds; the kernel's
+  // tile loop takes the rest), 4 % faster than persistent workgroups; wider tiles:
   // persistent, prefetching the next tile (np = 256)
-  const int64_t wgs = np == 128 ? std::min<int64_t>(cnt, (int64_t)1 << 30)
+  const int64_t wgs = np == 128 ? std::min<int64_t>(cnt, launch_wgs(NT))
                                 : std::min<int64_t>(cnt, (int64_t)4 * num_cus());
   if (np == 128)
     hipLaunchKernelGGL(ns5_lds_kernel<1>, dim3((unsigned)wgs), dim3(lds_threads<1>()), 0, s, x, out, inv, cnt, steps, a, b, c, round_once ? 1 : 0);

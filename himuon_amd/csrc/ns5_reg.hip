@@ -140,9 +140,12 @@ __global__ __launch_bounds__(NT, 1) void ns_direct_reg_kernel(const void* __rest
 
 void ns_direct_reg_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
                        float b, float c, float eps, bool round_once, hipStream_t s) {
+  const int64_t bytes = (int64_t)rows * cols * (dtype == HIMUON_DTYPE_F32 ? 4 : 2);
   const auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)cnt), dim3(NT), 0, s, g, out, cnt, rows, cols, steps, a, b, c, eps,
-                       round_once ? 1 : 0);
+    per_launch(cnt, NT, [&](int64_t off, int64_t n) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(NT), 0, s, static_cast<const char*>(g) + off * bytes,
+                         static_cast<char*>(out) + off * bytes, n, rows, cols, steps, a, b, c, eps, round_once ? 1 : 0);
+    });
   };
   switch (dtype) {
     case HIMUON_DTYPE_F32: run(ns_direct_reg_kernel<HIMUON_DTYPE_F32>); break;
@@ -160,8 +163,7 @@ bool reg_step_supported(int tile_h, int tile_w, int dtype, int param_dtype) {
 void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begin, int64_t cnt, int tile_h,
                   int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
                   bool round_once, const float* sa, hipStream_t s) {
-  for (int64_t off = 0; off < cnt; off += (int64_t)1 << 30) {
-    const int64_t n = std::min<int64_t>(cnt - off, (int64_t)1 << 30);
+  per_launch(cnt, NT, [&](int64_t off, int64_t n) {
     const auto run = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(NT), 0, s, params, n_params, tile_begin + off, n, tile_h,
                          tile_w, steps, a, b, c, eps, round_once ? 1 : 0, sa);
@@ -173,7 +175,7 @@ void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begi
       if (param_dtype == HIMUON_DTYPE_F32) run(reg_step_kernel<HIMUON_DTYPE_BF16, HIMUON_DTYPE_F32>);
       else run(reg_step_kernel<HIMUON_DTYPE_BF16, HIMUON_DTYPE_BF16>);
     }
-  }
+  });
 }
 
 bool ns5_reg_supported(int mp, int np) { return mp == T && np == T; }
@@ -181,9 +183,8 @@ bool ns5_reg_supported(int mp, int np) { return mp == T && np == T; }
 void ns5_reg_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int steps, float a, float b, float c,
                  bool round_once, hipStream_t s) {
   uint16_t* out = (steps & 1) ? y : x;
-  for (int64_t off = 0; off < cnt; off += (int64_t)1 << 30) {
-    const int64_t n = std::min<int64_t>(cnt - off, (int64_t)1 << 30);
+  per_launch(cnt, NT, [&](int64_t off, int64_t n) {
     hipLaunchKernelGGL(ns5_reg_kernel, dim3((unsigned)n), dim3(NT), 0, s, x + off * T * T, out + off * T * T,
                        inv + off, n, steps, a, b, c, round_once ? 1 : 0);
-  }
+  });
 }

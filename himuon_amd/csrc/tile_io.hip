@@ -399,7 +399,7 @@ extern "C" int himuon_momentum_gather(const HimuonParamDesc* params_dev, int n_p
       default: return HIMUON_EINVAL;
     }
   } else {
-    const dim3 grid((unsigned)std::min<int64_t>(items, (int64_t)1 << 30));
+    const dim3 grid((unsigned)std::min<int64_t>(items, launch_wgs(kThreads)));
     switch (dtype) {
       case HIMUON_DTYPE_F32: hipLaunchKernelGGL(gather_rows_kernel<HIMUON_DTYPE_F32>, grid, block, 0, s, params_dev, n_params, n_tiles, geo, tiles_bf16, partials); break;
       case HIMUON_DTYPE_BF16: hipLaunchKernelGGL(gather_rows_kernel<HIMUON_DTYPE_BF16>, grid, block, 0, s, params_dev, n_params, n_tiles, geo, tiles_bf16, partials); break;
@@ -446,7 +446,7 @@ int untile_launch(const HimuonParamDesc* params_dev, int n_params, int64_t n_til
       default: return HIMUON_EINVAL;
     }
   } else {
-    const dim3 grid((unsigned)std::min<int64_t>(n_tiles * (mp / slab_rows(mp, np)), (int64_t)1 << 30));
+    const dim3 grid((unsigned)std::min<int64_t>(n_tiles * (mp / slab_rows(mp, np)), launch_wgs(kThreads)));
     switch (dtype) {
       case HIMUON_DTYPE_F32: hipLaunchKernelGGL((untile_rows_kernel<APPLY, HIMUON_DTYPE_F32>), grid, block, 0, s, params_dev, n_params, n_tiles, geo, tiles_bf16, sa); break;
       case HIMUON_DTYPE_BF16: hipLaunchKernelGGL((untile_rows_kernel<APPLY, HIMUON_DTYPE_BF16>), grid, block, 0, s, params_dev, n_params, n_tiles, geo, tiles_bf16, sa); break;

@@ -294,12 +294,15 @@ int himuon_reg_step(const HimuonParamDesc* params_dev, int n_params,
                     const float* scale_alpha_dev, void* stream);
 
 /*
- * newton_schulz (himuon.py:232-284) of `batch` contiguous M x N matrices of
- * dtype (HIMUON_DTYPE_F32 / BF16 / F16) from g into out (same shape and dtype,
- * contiguous, any element alignment; out may be g itself) in one launch: cast to bf16, normaliser, `steps` iterations, cast back, with
- * the values of himuon_momentum_gather (no momentum) + himuon_tile_scale +
- * himuon_ns5_ex + himuon_untile bit for bit. flags: HIMUON_NS_ROUND_ONCE only.
- * Supported (else HIMUON_EINVAL) for 64 < M <= N <= 128 and 128 < M <= N <= 256.
+ * newton_schulz (himuon.py:232-284) of `batch` < 2^31 contiguous M x N matrices
+ * of dtype (HIMUON_DTYPE_F32 / BF16 / F16) from g into out (same shape and
+ * dtype, contiguous, any element alignment; out may be g itself) in one launch
+ * (of one workgroup per matrix; more launches where a grid, of less than 2^32
+ * threads, does not hold the batch): cast to bf16, normaliser, `steps`
+ * iterations, cast back, with the values of himuon_momentum_gather (no momentum)
+ * + himuon_tile_scale + himuon_ns5_ex + himuon_untile bit for bit. flags:
+ * HIMUON_NS_ROUND_ONCE only. Supported (else HIMUON_EINVAL) for 64 < M <= N <=
+ * 128 and 128 < M <= N <= 256.
  */
 int himuon_ns_direct_supported(int M, int N, int dtype);
 int himuon_ns_direct(const void* g, void* out, int64_t batch, int M, int N, int dtype, int steps, float a, float b,

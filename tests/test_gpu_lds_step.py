@@ -124,3 +124,19 @@ def test_lds_step_refuses_other_buckets():
             a[5] = 64  # tile_h > tile_w: a transposed tile
         assert lib.himuon_lds_step(*a) == -22, (pos, val)
     torch.cuda.synchronize()
+
+
+def test_more_tiles_than_one_launch_holds():
+    """A grid holds fewer than 2^32 threads, 2^24 - 1 workgroups of 256: the tiles
+    beyond are another launch's. Equal 1 x 2 tiles, so every parameter ends equal."""
+    n = (1 << 24) + 5
+    p = torch.nn.Parameter(torch.full((1, 2 * n), 0.5, device=DEV, dtype=torch.bfloat16))
+    g = torch.full((1, 2 * n), 1e-3, device=DEV, dtype=torch.bfloat16)
+    sa = torch.zeros(2 * nat.APPLY_MAX_GROUPS, device=DEV)
+    nat.write_scale_alpha(sa, [1.0], [-0.25])
+    grp = TileGroup(params=[p], grads=[g], moms=[None], tile_h=1, tile_w=2, upd_scales=[1.0], mus=[0.0],
+                    nesterovs=[False], device=g.device, dtype=g.dtype, apply_groups=[0])
+    assert grp.n_tiles == n and grp.lds_step_ok()
+    grp.lds_step(0, n, 1, sa)
+    first = p.data[0, 0].item()
+    assert first != 0.5 and bool((p.data == first).all())
