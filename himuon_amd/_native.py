@@ -222,7 +222,9 @@ def _check(rc: int, what: str) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle (torch.cuda.current_stream().cuda_stream
+    without the stream object: 0.4 against 2.9 us of a launch's host time)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -291,6 +293,13 @@ def few_rows_supported(m: int, mp: int, np_: int) -> bool:
     if m <= 32 and np_ in (768, 1024):
         return True
     return m <= 16 and np_ in (1536, 2048)
+
+
+def one_launch(m: int, mp: int, np_: int, family: str = "auto") -> bool:
+    """Whether all iterations of an NS sub-batch are one launch (few rows, or the
+    tile held on chip), not two or three per iteration."""
+    return family == "auto" and (few_rows_supported(m, mp, np_) or (mp == 128 and np_ in (128, 256, 512))
+                                 or mp == np_ == 256)
 
 
 def default_sub_batch(n_tiles: int, mp: int, np_: int) -> int:

@@ -28,8 +28,10 @@ from . import _native as nat
 def mem_span(t: torch.Tensor) -> "tuple[int, int]":
     """First byte and end of the memory that t's elements lie in."""
     p = t.data_ptr()
+    if t.is_contiguous():
+        return p, p + t.nbytes
     last = sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
-    return p, p + (last + 1) * t.element_size() if t.numel() else p
+    return p, p + (last + 1) * t.element_size()  # (empty tensors are contiguous)
 
 
 def sharing(tensors) -> "set[int]":
@@ -436,12 +438,12 @@ class _NsPlan:
     """Device state of ``newton_schulz`` for one (batch shape, dtype, device,
     rounding form, kernel family): the tile buffers, the NS workspace and a
     descriptor table of one entry, and per step count a hipGraph of the launches
-    (gather, normaliser, NS, untile), captured on first use. The launches read
+    (gather, normaliser, NS, untile) where NS is many, captured on first use. The launches read
     and write what the descriptor points at, which run() sets to the call's own
     input and result (a launch that carries the descriptor in its arguments), so
     neither is copied. A call neither allocates device state (beyond the returned
-    tensor) nor synchronises, and costs two launches from the host instead of a
-    dozen.
+    tensor) nor synchronises, and costs two launches from the host, or five where
+    NS is one.
 
     Calls that use one plan must be ordered on one stream, each from its
     descriptor write to its last launch: a later call's descriptor would
@@ -463,7 +465,14 @@ class _NsPlan:
         self.tiles, self.alt = (buffer((n, self.mp, self.np), torch.bfloat16) for _ in range(2))
         self.partials, self.inv = buffer((n, self.ppt), torch.float32), buffer(n, torch.float32)
         self.ws = buffer(max(1, nat.ns5_workspace_bytes(self.sub_batch, self.mp, self.np)), torch.uint8)
+        # A replay takes 17 us of host time and a launch 4.5: chains of four launches
+        # go out one by one (a call on a 16 x 16 matrix 30-33 us against 38-40, on a
+        # transposed view of one 35-38 against 48), those of a dozen and more as a
+        # graph.
+        self.recorded = n > self.sub_batch or not nat.one_launch(self.m, self.mp, self.np, family)
         self.graphs: "dict[int, torch.cuda.CUDAGraph]" = {}
+        d = self._host_desc = nat.ParamDesc()
+        d.h, d.w, d.ld_grad, d.ld_upd, d.R, d.C, d.upd_scale = n * M, N, N, N, n, 1, 1.0
 
     # an input and a result of the plan's own, for _launches() without others
     @functools.cached_property
@@ -477,9 +486,8 @@ class _NsPlan:
     def _point(self, G: torch.Tensor, out: torch.Tensor) -> None:
         """The descriptor to G and out, as a launch: ordered after the launches of
         earlier calls and before this one's."""
-        d = nat.ParamDesc()
+        d = self._host_desc
         d.grad, d.update = G.data_ptr(), out.data_ptr()
-        d.h, d.w, d.ld_grad, d.ld_upd, d.R, d.C, d.upd_scale = self.n * self.M, self.N, self.N, self.N, self.n, 1, 1.0
         nat.write_desc(d, self.desc)
 
     def _ns(self, steps: int) -> None:
@@ -501,7 +509,7 @@ class _NsPlan:
         tensor; capturing: inside the caller's capture, which records the launches."""
         out = torch.empty(G.shape, device=G.device, dtype=G.dtype)
         graph = None
-        if not capturing:
+        if self.recorded and not capturing:
             graph = self.graphs.get(steps)
             if graph is None:
                 graph = torch.cuda.CUDAGraph()

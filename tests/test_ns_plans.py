@@ -34,3 +34,16 @@ def test_the_least_recently_used_plans_make_room(plans):
         E._ns_plan(s, s)
         assert len(plans) <= E._NS_PLANS_TOTAL
         assert sum(k[0] == 0 for k in plans) <= E._NS_PLANS_MAX
+
+
+def test_what_is_launched_unrecorded():
+    """The shapes whose iterations are one launch, as bench.ns_family names their kernels."""
+    from bench import ns_family
+    from himuon_amd import _native as nat
+
+    for M in (1, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257, 512):
+        for N in (16, 128, 129, 256, 257, 384, 512, 513, 768, 1024, 1280, 1536, 2048, 2300):
+            m, _, mp, np_, _ = nat.ns_geometry(M, N)
+            for family in nat.NS_FAMILIES:
+                one = family == "auto" and ns_family(mp, np_, family, m) in ("few_rows", "lds")
+                assert nat.one_launch(m, mp, np_, family) == one, (M, N, family)
