@@ -23,14 +23,16 @@
 // The bf16-in / bf16-out products keep their own kernels (ns5_blk.hip,
 // ns5_stream.hip), bit-identical to torch; these kernels serve every other
 // dtype pair, and bf16 operands off 16-byte boundaries (ns_any_product: the same
-// bits), which those kernels' direct-to-LDS loads do not take. Block tile 64 x 64 x 64, four waves of one MFMA 32x32 tile each;
+// bits), which those kernels' direct-to-LDS loads do not take. Block tile 64 x 64
+// x 64 or 128 x 128 x 64, four waves of one MFMA 32x32 tile each or of 2 x 2;
 // operands are converted as they are staged through registers into a double
 // buffer in LDS; the Gram products compute the lower blocks and store each block
 // and its mirror.
 //
 // What bounds them: each K unit's loads, conversions and barrier in turn, so
-// what counts is how many workgroups share a CU. 64 x 64 blocks were faster than
-// 128 x 128 at every size (us, fp32 XXT / ba_plus_cAA / bmm_add): 8 of 512 x 1024
+// what counts is how many workgroups share a CU, until the operand stream of 64 x
+// 64 blocks does (16-bit operands of long contractions: gram_128). us for XXT /
+// ba_plus_cAA / bmm_add in fp32, 64 x 64 against 128 x 128 blocks: 8 of 512 x 1024
 // 27 / 19 / 42 against 49 / 39 / 54 (59 / 49 / 55 with the mirrored block stored
 // element by element and twice the instructions per conversion), 64 of 1024 x
 // 2048 950 / 548 / 2370 against 1031 / 692 / 3121; fp16 8 of 512 x 1024 21 / 19 /
@@ -42,9 +44,7 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int BT = 64;       // output block edge
 constexpr int BK = 64;       // K per unit
-constexpr int R = BT / 32;   // loader rows per thread
 constexpr int kAlign = 128;  // operand dimensions
 constexpr int kLd = BK + 8;  // padded LDS row pitch (16-bit elements)
 
@@ -126,6 +126,16 @@ HM_DEV void store_out(void* base, int64_t idx, float v, int out_dtype) {
 
 constexpr int planes(int in) { return in == kInF32 ? 2 : 1; }
 
+// acc += a b of one MFMA tile and k-step (fp32 operands: lo hi, hi lo, hi hi).
+template <int IN>
+HM_DEV void product(const u32x4_t (&a)[planes(IN)], const u32x4_t (&b)[planes(IN)], f32x16_t& acc) {
+  if constexpr (planes(IN) == 2) {
+    acc = mfma_in<IN>(a[1], b[0], acc);
+    acc = mfma_in<IN>(a[0], b[1], acc);
+  }
+  acc = mfma_in<IN>(a[0], b[0], acc);
+}
+
 // 4 consecutive outputs, at any element alignment.
 HM_DEV void store_out4(void* base, int64_t idx, const float (&v)[4], int out_dtype) {
   if (out_dtype == HIMUON_DTYPE_F32) {
@@ -144,12 +154,14 @@ HM_DEV void store_out4(void* base, int64_t idx, const float (&v)[4], int out_dty
 // C = alpha S S^T (+ beta S when add_s; K == M) for each batch entry; S:
 // M x K, C: M x M. Lower BT x BT blocks only, each stored at (bi, bj) and
 // mirrored (a lane holds 4 consecutive rows of a column: 4 consecutive
-// elements of the mirrored row).
-template <int IN>
+// elements of the mirrored row). BT: the block's edge, 64 or 128.
+template <int IN, int BT>
 __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restrict__ S, void* __restrict__ C,
                                                              int M, int K, int64_t first, int64_t count,
                                                              float alpha, float beta, int add_s, int out_dtype) {
   constexpr int NP = planes(IN);
+  constexpr int R = BT / 32;   // loader rows per thread
+  constexpr int WT = BT / 64;  // MFMA tiles per wave and direction
   __shared__ __attribute__((aligned(16))) uint16_t sI[2][NP][BT * kLd];
   __shared__ __attribute__((aligned(16))) uint16_t sJ[2][NP][BT * kLd];
 
@@ -191,9 +203,13 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
     }
   };
 
-  f32x16_t acc;
+  f32x16_t acc[WT][WT];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  for (int mi = 0; mi < WT; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < WT; ++ni)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
 
   const int nk = K / BK;
   gload(0);
@@ -205,17 +221,18 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
 #pragma unroll
     for (int ks = 0; ks < BK / 16; ++ks) {
       const int kk = ks * 16 + (lane >> 5) * 8;
-      u32x4_t a[NP], b[NP];
+      u32x4_t a[WT][NP], b[WT][NP];
 #pragma unroll
-      for (int pl = 0; pl < NP; ++pl) {
-        a[pl] = *reinterpret_cast<const u32x4_t*>(&sI[cur][pl][(wm * 32 + (lane & 31)) * kLd + kk]);
-        b[pl] = *reinterpret_cast<const u32x4_t*>(&sJ[cur][pl][(wn * 32 + (lane & 31)) * kLd + kk]);
-      }
-      if constexpr (NP == 2) {
-        acc = mfma_in<IN>(a[1], b[0], acc);
-        acc = mfma_in<IN>(a[0], b[1], acc);
-      }
-      acc = mfma_in<IN>(a[0], b[0], acc);
+      for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int pl = 0; pl < NP; ++pl) {
+          a[t][pl] = *reinterpret_cast<const u32x4_t*>(&sI[cur][pl][(wm * 32 * WT + 32 * t + (lane & 31)) * kLd + kk]);
+          b[t][pl] = *reinterpret_cast<const u32x4_t*>(&sJ[cur][pl][(wn * 32 * WT + 32 * t + (lane & 31)) * kLd + kk]);
+        }
+#pragma unroll
+      for (int mi = 0; mi < WT; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < WT; ++ni) product<IN>(a[mi], b[ni], acc[mi][ni]);
     }
     if (kt + 1 < nk) lstore(cur ^ 1);
     __syncthreads();
@@ -226,24 +243,28 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
   const int64_t c0 = tile * (int64_t)M * M;
   const bool offdiag = bi > bj;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int i0 = bi * BT + wm * 32 + 8 * q + 4 * (lane >> 5);
-    const int j = bj * BT + wn * 32 + (lane & 31);
-    float v[4];
+  for (int mi = 0; mi < WT; ++mi)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[e] = alpha * acc[4 * q + e];
-      if (add_s) v[e] = fmaf(beta, load_elem_in<IN>(S, s0 + (int64_t)(i0 + e) * K + j), v[e]);
-      if (offdiag || i0 + e >= j) store_out(C, c0 + (int64_t)(i0 + e) * M + j, v[e], out_dtype);
-    }
-    if (offdiag || i0 > j) {  // all 4 below the diagonal
-      store_out4(C, c0 + (int64_t)j * M + i0, v, out_dtype);
-    } else {
+    for (int ni = 0; ni < WT; ++ni)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (i0 + e > j) store_out(C, c0 + (int64_t)j * M + i0 + e, v[e], out_dtype);
-    }
-  }
+      for (int q = 0; q < 4; ++q) {
+        const int i0 = bi * BT + wm * 32 * WT + 32 * mi + 8 * q + 4 * (lane >> 5);
+        const int j = bj * BT + wn * 32 * WT + 32 * ni + (lane & 31);
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = alpha * acc[mi][ni][4 * q + e];
+          if (add_s) v[e] = fmaf(beta, load_elem_in<IN>(S, s0 + (int64_t)(i0 + e) * K + j), v[e]);
+          if (offdiag || i0 + e >= j) store_out(C, c0 + (int64_t)(i0 + e) * M + j, v[e], out_dtype);
+        }
+        if (offdiag || i0 > j) {  // all 4 below the diagonal
+          store_out4(C, c0 + (int64_t)j * M + i0, v, out_dtype);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (i0 + e > j) store_out(C, c0 + (int64_t)j * M + i0 + e, v[e], out_dtype);
+        }
+      }
 }
 
 // C = out(Bm X) + gamma X for each batch entry (Bm X rounded to the output
@@ -251,12 +272,14 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
 // and C: M x N.
 // X is the MFMA B operand with the contraction along its rows: each 4 x 8
 // block of X is transposed into the k-octet-major LDS layout sX[k/8][j][k%8].
-template <int IN>
+template <int IN, int BT>
 __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __restrict__ Bm,
                                                               const void* __restrict__ X, void* __restrict__ C,
                                                               int M, int N, int64_t first, int64_t count,
                                                               float gamma, int round_once, int out_dtype) {
   constexpr int NP = planes(IN);
+  constexpr int R = BT / 32;   // loader rows per thread
+  constexpr int WT = BT / 64;  // MFMA tiles per wave and direction
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][NP][BT * kLd];
   __shared__ __attribute__((aligned(16))) uint16_t sX[2][NP][(BK / 8) * BT * 8];
 
@@ -299,14 +322,20 @@ __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __rest
       for (int e = 0; e < 8; ++e) {
         const int w = e >> 1, h = e & 1;
         auto v = [&](int rr) { return half16(pl == 0 ? rx[rr].hi[w] : rx[rr].lo[w], h); };
-        *reinterpret_cast<uint32_t*>(base + (xjo + e) * 8) = pack2(v(0), v(1));
+#pragma unroll
+        for (int rr = 0; rr < R; rr += 2)
+          *reinterpret_cast<uint32_t*>(base + (xjo + e) * 8 + rr) = pack2(v(rr), v(rr + 1));
       }
     }
   };
 
-  f32x16_t acc;
+  f32x16_t acc[WT][WT];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  for (int mi = 0; mi < WT; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < WT; ++ni)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
 
   const int nk = M / BK;
   gload(0);
@@ -319,30 +348,36 @@ __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __rest
     for (int ks = 0; ks < BK / 16; ++ks) {
       const int kk = ks * 16 + (lane >> 5) * 8;
       const int koct = ks * 2 + (lane >> 5);
-      u32x4_t av[NP], bv[NP];
+      u32x4_t a[WT][NP], b[WT][NP];
 #pragma unroll
-      for (int pl = 0; pl < NP; ++pl) {
-        av[pl] = *reinterpret_cast<const u32x4_t*>(&sA[cur][pl][(wm * 32 + (lane & 31)) * kLd + kk]);
-        bv[pl] = *reinterpret_cast<const u32x4_t*>(&sX[cur][pl][(koct * BT + wn * 32 + (lane & 31)) * 8]);
-      }
-      if constexpr (NP == 2) {
-        acc = mfma_in<IN>(av[1], bv[0], acc);
-        acc = mfma_in<IN>(av[0], bv[1], acc);
-      }
-      acc = mfma_in<IN>(av[0], bv[0], acc);
+      for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int pl = 0; pl < NP; ++pl) {
+          a[t][pl] = *reinterpret_cast<const u32x4_t*>(&sA[cur][pl][(wm * 32 * WT + 32 * t + (lane & 31)) * kLd + kk]);
+          b[t][pl] =
+              *reinterpret_cast<const u32x4_t*>(&sX[cur][pl][(koct * BT + wn * 32 * WT + 32 * t + (lane & 31)) * 8]);
+        }
+#pragma unroll
+      for (int mi = 0; mi < WT; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < WT; ++ni) product<IN>(a[mi], b[ni], acc[mi][ni]);
     }
     if (kt + 1 < nk) lstore(cur ^ 1);
     __syncthreads();
   }
 
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = bi * BT + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    const int j = bj * BT + wn * 32 + (lane & 31);
-    const int64_t e = x0 + (int64_t)i * N + j;
-    const float bx = round_once ? acc[r] : round_out(acc[r], out_dtype);
-    store_out(C, e, bx + gamma * load_elem_in<IN>(X, e), out_dtype);
-  }
+  for (int mi = 0; mi < WT; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < WT; ++ni)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = bi * BT + wm * 32 * WT + 32 * mi + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        const int j = bj * BT + wn * 32 * WT + 32 * ni + (lane & 31);
+        const int64_t e = x0 + (int64_t)i * N + j;
+        const float bx = round_once ? acc[mi][ni][r] : round_out(acc[mi][ni][r], out_dtype);
+        store_out(C, e, bx + gamma * load_elem_in<IN>(X, e), out_dtype);
+      }
 }
 
 bool dtype_in_ok(int d) {
@@ -354,26 +389,76 @@ bool dtype_out_ok(int d) { return d == HIMUON_DTYPE_F32 || d == HIMUON_DTYPE_BF1
 // which a result near the size of the memory exceeds in 64 x 64 blocks.
 constexpr int64_t kLaunchItems = int64_t(1) << 23;
 
-template <int IN>
-void launch_gram(const void* s, void* c, int M, int K, int64_t batch, float alpha, float beta, int add_s, int od,
-                 hipStream_t st) {
+template <int IN, int BT>
+void launch_gram_blocks(const void* s, void* c, int M, int K, int64_t batch, float alpha, float beta, int add_s, int od,
+                        hipStream_t st) {
   const int64_t nb = M / BT, items = batch * (nb * (nb + 1) / 2);
   for (int64_t first = 0; first < items; first += kLaunchItems) {
     const int64_t count = std::min(kLaunchItems, items - first);
-    hipLaunchKernelGGL(prod_gram_kernel<IN>, dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, s, c, M, K, first,
+    hipLaunchKernelGGL((prod_gram_kernel<IN, BT>), dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, s, c, M, K, first,
                        count, alpha, beta, add_s, od);
   }
+}
+
+template <int IN, int BT>
+void launch_apply_blocks(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma,
+                         int round_once, int od, hipStream_t st) {
+  const int64_t items = batch * (M / BT) * (N / BT);
+  for (int64_t first = 0; first < items; first += kLaunchItems) {
+    const int64_t count = std::min(kLaunchItems, items - first);
+    hipLaunchKernelGGL((prod_apply_kernel<IN, BT>), dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, b, x, c, M, N,
+                       first, count, gamma, round_once, od);
+  }
+}
+
+// 128 x 128 blocks where 64 x 64 ones, which stream each operand twice as often,
+// would be bound by that: long contractions of many blocks. `items`: 128 x 128
+// blocks, K: the contraction. The lines lie between shapes measured both ways (us,
+// 64 x 64 / 128 x 128; MxK the operand of XXT, a square one that of ba_plus_cAA):
+//   Gram, 16-bit to fp32, K >= 1024 and items K >= 2^21: 64 of 1024 x 1024 214 / 178,
+//     8 of 2048 x 2048 132 / 123, 4096 x 4096 167 / 132, 8192 x 8192 1267 / 748; below
+//     it 4 of 2048 x 2048 83 / 102, 16 of 1024 x 1024 52 / 75.
+//   Gram, 16-bit to 16-bit (dearer stores), K >= 4096 and items K >= 3.5 2^20: 3072 x
+//     12288 277 / 215, 64 of 1024 x 4096 593 / 489, 8192 x 8192 1254 / 802, below it
+//     8 of 2048 x 2048 150 / 170; and from 6144 rows on, 6144 x 2048 203 / 177.
+//   Gram, e5m2 (half the bytes), K >= 4096 and items K >= 7 2^20: 4 of 4096 x 4096
+//     541 / 516, 8192 x 8192 1050 / 893, below it 2 of 4096 x 4096 278 / 313.
+//   Apply, 16-bit to fp32, M >= 2048 and items M >= 2^22: 8 of 2048 x 2048 385 / 361,
+//     8192 x 8192 2773 / 2568, below it 64 of 1024 x 1024 407 / 438.
+//   Apply, 16-bit to 16-bit, M >= 4096 and items M >= 2^23: 4 of 4096 x 2048 758 /
+//     703, 8192 x 8192 2786 / 2637, below it 4096 x 4096 370 / 376.
+//   Apply of e5m2 and every product of fp32 operands: 64 x 64 throughout.
+template <int IN>
+bool gram_128(int64_t items, int M, int K, int od) {
+  const int64_t work = items * K;
+  if (IN == kInE5m2) return K >= 4096 && work >= 7 << 20;
+  if (od == HIMUON_DTYPE_F32) return K >= 1024 && work >= 1 << 21;
+  return (K >= 4096 && work >= 7 << 19) || (M >= 6144 && K >= 1024);
+}
+
+bool apply_128(int64_t items, int M, int od) {
+  return od == HIMUON_DTYPE_F32 ? M >= 2048 && items * M >= 1 << 22 : M >= 4096 && items * M >= 1 << 23;
+}
+
+template <int IN>
+void launch_gram(const void* s, void* c, int M, int K, int64_t batch, float alpha, float beta, int add_s, int od,
+                 hipStream_t st) {
+  if constexpr (IN != kInF32) {
+    const int64_t nb = M / 128;
+    if (gram_128<IN>(batch * (nb * (nb + 1) / 2), M, K, od))
+      return launch_gram_blocks<IN, 128>(s, c, M, K, batch, alpha, beta, add_s, od, st);
+  }
+  launch_gram_blocks<IN, 64>(s, c, M, K, batch, alpha, beta, add_s, od, st);
 }
 
 template <int IN>
 void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int round_once,
                   int od, hipStream_t st) {
-  const int64_t items = batch * (M / BT) * (N / BT);
-  for (int64_t first = 0; first < items; first += kLaunchItems) {
-    const int64_t count = std::min(kLaunchItems, items - first);
-    hipLaunchKernelGGL(prod_apply_kernel<IN>, dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, b, x, c, M, N,
-                       first, count, gamma, round_once, od);
+  if constexpr (IN != kInF32 && IN != kInE5m2) {
+    if (apply_128(batch * (M / 128) * (N / 128), M, od))
+      return launch_apply_blocks<IN, 128>(b, x, c, M, N, batch, gamma, round_once, od, st);
   }
+  launch_apply_blocks<IN, 64>(b, x, c, M, N, batch, gamma, round_once, od, st);
 }
 
 // 128 x 128 output blocks a call takes.
