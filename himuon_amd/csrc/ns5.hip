@@ -302,34 +302,53 @@ extern "C" int himuon_ns5(uint16_t* x, uint16_t* y, const float* inv, int64_t n_
 }
 
 // ---------------------------------------------------------------------------
-// One product on the faster block size. Rounds of 256 x 256 blocks (one per
-// CU) cost about the same whether full or not, so r = blocks / CUs of them cost
-// ceil(r); 64 x 64 and 128 x 128 blocks (two workgroups per CU) fill the chip
-// at any count at a lower rate, about 1.25 r for Apply and 1.3 r for a Gram
-// product; a large Gram product on 128 x 128 blocks computes fewer elements (36 of
-// 64 blocks against 10 of 16 at 1024), and takes 1.26 r. Beyond three rounds the
-// 256 x 256 blocks are ahead, or 3 % behind, for every Gram product. Measured (us, smaller blocks / 256 x 256): Apply of 28 1024 x 1024 (448 blocks) 76 / 66,
-// of 7 1024 x 2560 (280) 52 / 63, of one 1024 x 3072 (48) 15 / 30; GramA of 20
-// 1024 x 1024 (r = 0.78) 40 / 35, of 28 (1.09) 43 / 62, of 50 (1.95) 78 / 69, of 60
-// (2.34) 86 / 94, of 80 (3.13) 133 / 121, of 340 (13.3) 537 / 478 (GramB 41 / 39,
-// 45 / 70, 79 / 80, 92 / 106, 133 / 137, 564 / 529), of 56 1024 x 3072 (2.19) 230 /
-// 245, of 150 610 / 570, of 3 4096 x 4096 (1.59) 240 / 220, of 12 (6.4) 968 / 819,
-// of one 1024 x 3072 24 / 75, of 128 512 x 512 (1.5) 32 / 34, of 256 (3) 58 / 53,
-// of 1,024 272 / 250, of 200 256 x 2048 (0.78) 59 / 47. Gram products of M >= 512
-// and K >= 1024 at any count on smaller blocks: the step of 340 tiles of 1024 x
-// 1024 11.68 ms against 10.97.
+// One product on the faster block size. 256 x 256 blocks run one per CU, so r =
+// blocks / CUs of them take ceil(r) rounds, full or not; 64 x 64 and 128 x 128
+// blocks (ns_blk_product), two workgroups of 128 per CU, take a time that grows
+// evenly with r: blk_rounds(), in those rounds. Beyond three rounds the 256 x 256
+// blocks are ahead, or a few per cent behind, throughout. Below one round (r < 1)
+// the 128 x 128 blocks win while they are one round themselves, two per CU, or
+// little more.
+//
+// The constants are fitted to 1,689 products measured both ways (M 256 .. 8192,
+// K up to 11 M, r 0.1 .. 8): the choice is within 0.6 % of always taking the faster
+// one, 1.13 times as fast as 256 x 256 blocks alone, and more than 3 % behind those in
+// four of the products. Points near the lines (us, smaller blocks / 256 x 256):
+//
+//   Apply M <= 256   269 of 256 x 256, r 1.05: 26 / 34      794, r 3.10: 75 / 68
+//   Apply M <= 2048  42 of 1024 x 1024, r 2.62: 116 / 99    33, r 2.06: 90 / 96
+//                    8 of 2048 x 2048, r 2.0: 153 / 124     5, r 1.25: 93 / 107
+//   Apply beyond     5120 x 5120, r 1.56: 322 / 260         4096 x 4352, r 1.06: 184 / 198
+//   Gram r < 1       13 of 1024 x 1024 (468 of 128): 25 / 36   17 (612): 35 / 33
+//   Gram M < 512     269 of 256 x 256, r 1.05: 16 / 21      (or K < 1024)
+//   Gram otherwise   33 of 1024 x 1024, r 1.29: 55 / 63     50, r 1.95: 76 / 70
+//   Gram M >= 2560   7 of 3072 x 3072, r 2.13: 239 / 258    7 of 3072 x 12288: 1021 / 930
+//   Gram M >= 5120   6144 x 6144, r 1.17: 289 / 306         7168 x 7168, r 1.59: 448 / 377
 // ---------------------------------------------------------------------------
+namespace {
+double blk_rounds(int mode, int M, int K, double r) {
+  if (mode == kApply) return M <= 256 ? 0.2 + 1.15 * r : M <= 2048 ? 0.2 + 1.25 * r : 0.05 + 1.56 * r;
+  if (M >= 5120 || (M >= 2560 && K / 2 >= M)) return 1.55 * r;
+  if (M >= 2560) return 1.33 * r;
+  return (M >= 512 && K >= 1024 ? 1.26 : 1.3) * r;
+}
+
+bool smaller_blocks(int mode, const NsProduct& g) {
+  if (g.M % 256 || g.N % 256 || g.K % 256) return true;
+  const int64_t nb = g.M / 256, cus = num_cus();
+  const int64_t items = g.ntiles * (mode == kApply ? nb * (g.N / 256) : nb * (nb + 1) / 2);
+  if (items > 3 * cus) return false;
+  if (items >= cus) return blk_rounds(mode, g.M, g.K, (double)items / cus) < (double)((items + cus - 1) / cus);
+  // 128 x 128 blocks against one round of two per CU
+  const int64_t blocks = mode == kApply ? 4 * items : g.ntiles * nb * (2 * nb + 1);
+  const double rounds = blocks / (2.0 * cus);
+  if (mode == kApply) return rounds <= (g.M <= 1024 ? 1.24 : 1.0);
+  return rounds <= (g.M < 2560 ? 1.15 : 1.0);
+}
+}  // namespace
+
 void ns_product(int mode, const NsProduct& g, hipStream_t s) {
-  bool small = g.M % 256 || g.N % 256 || g.K % 256;
-  if (!small) {
-    const int64_t nb = g.M / 256, cus = num_cus();
-    const int64_t items = g.ntiles * (mode == kApply ? nb * (g.N / 256) : nb * (nb + 1) / 2);
-    const double r = (double)items / cus;
-    const bool large = g.M >= 512 && g.K >= 1024 && r > 1.0;
-    const double rate = mode == kApply ? 1.25 : large ? 1.26 : 1.3;
-    small = rate * r < (double)((items + cus - 1) / cus) && (mode == kApply || r <= 3.0);
-  }
-  if (small) ns_blk_product(mode, g, s);
+  if (smaller_blocks(mode, g)) ns_blk_product(mode, g, s);
   else ns_stream_product(mode, g, s);
 }
 

@@ -1,5 +1,5 @@
-"""The block sizes of the typed products (himuon_*_typed): 128 x 128 output
-blocks for long contractions of many blocks, 64 x 64 otherwise, one result."""
+"""The block sizes of the products: 64 x 64, 128 x 128 and, for bf16, 256 x 256
+output blocks, chosen by size and dtypes, one result."""
 
 from __future__ import annotations
 
@@ -34,3 +34,19 @@ def test_block_sizes_give_the_same_bits(idt, odt, B, M, N):
         for k in range(0, B, max(1, B // 4)):
             call(slice(k, k + 1), one)
             assert torch.equal(one[0], whole[k])
+
+
+@pytest.mark.parametrize("B,M,N", [(269, 256, 256), (198, 512, 512), (13, 1024, 1024), (17, 1024, 1024), (50, 1024, 1024),
+                                   (2, 2560, 2560), (2, 3072, 6144), (1, 5120, 5120)])
+def test_bf16_block_choice(B, M, N):
+    """On either side of the lines between the 256 x 256 blocks and the smaller
+    ones (himuon_xxt, himuon_ba_plus_caa, himuon_bmm_add): the smaller blocks' bits."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = (torch.randn(B, M, N, device=DEV, generator=g) / N ** 0.5).bfloat16()
+    s = (torch.randn(B, M, M, device=DEV, generator=g) / M ** 0.5).bfloat16()
+    for shape, call in (((B, M, M), lambda o, f: nat.xxt(x, o, B, M, N, family=f)),
+                        ((B, M, M), lambda o, f: nat.ba_plus_caa(s, o, B, M, 0.5, -1.5, family=f)),
+                        ((B, M, N), lambda o, f: nat.bmm_add(s, x, o, B, M, N, 2.0, family=f))):
+        a, b = (torch.empty(shape, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        call(a, "auto"), call(b, "block128")
+        assert torch.equal(a, b)
