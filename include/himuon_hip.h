@@ -202,7 +202,8 @@ int himuon_ns5_ex(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles,
  * beta, out) (ba_plus_cAA.py:90-120) and fused_bmm_add(B, X, a, out)
  * (fused_bmm_add.py:98-135) with the same rounding points as himuon_ns5:
  *   himuon_xxt:         out = bf16(x x^T)            x: (batch, M, K), out: (batch, M, M)
- *   himuon_ba_plus_caa: out = bf16(alpha a a^T + beta a)   a, out: (batch, M, M)
+ *   himuon_ba_plus_caa: out = bf16(alpha a a^T + beta a)   a, out: (batch, M, M), a
+ *                       symmetric (an XXT output: only lower blocks are computed)
  *   himuon_bmm_add:     out = bf16(bf16(b x) + a x)   b: (batch, M, M), x, out: (batch, M, N)
  *                       (bf16(b x + a x), one rounding, with HIMUON_NS_ROUND_ONCE:
  *                       torch.addmm(X, B, X, beta=a) of himuon.py:252-253)

@@ -43,7 +43,8 @@ def test_bf16_block_choice(B, M, N):
     ones (himuon_xxt, himuon_ba_plus_caa, himuon_bmm_add): the smaller blocks' bits."""
     g = torch.Generator(device=DEV).manual_seed(M + N)
     x = (torch.randn(B, M, N, device=DEV, generator=g) / N ** 0.5).bfloat16()
-    s = (torch.randn(B, M, M, device=DEV, generator=g) / M ** 0.5).bfloat16()
+    s = torch.randn(B, M, M, device=DEV, generator=g) / M ** 0.5
+    s = (s + s.transpose(1, 2)).bfloat16().contiguous()  # (ba_plus_cAA's operand is symmetric)
     for shape, call in (((B, M, M), lambda o, f: nat.xxt(x, o, B, M, N, family=f)),
                         ((B, M, M), lambda o, f: nat.ba_plus_caa(s, o, B, M, 0.5, -1.5, family=f)),
                         ((B, M, N), lambda o, f: nat.bmm_add(s, x, o, B, M, N, 2.0, family=f))):
