@@ -268,15 +268,15 @@ __global__ __launch_bounds__(kThreads) void prod_gram_kernel(const void* __restr
 }
 
 // C = out(Bm X) + gamma X for each batch entry (Bm X rounded to the output
-// dtype before the add, fused_bmm_add.py:73-88, unless round_once); Bm: M x M, X
-// and C: M x N.
+// dtype before the add, fused_bmm_add.py:73-88, unless ONCE); Bm: M x M, X and
+// C: M x N.
 // X is the MFMA B operand with the contraction along its rows: each 4 x 8
 // block of X is transposed into the k-octet-major LDS layout sX[k/8][j][k%8].
-template <int IN, int BT>
+template <int IN, int BT, bool ONCE>
 __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __restrict__ Bm,
                                                               const void* __restrict__ X, void* __restrict__ C,
                                                               int M, int N, int64_t first, int64_t count,
-                                                              float gamma, int round_once, int out_dtype) {
+                                                              float gamma, int out_dtype) {
   constexpr int NP = planes(IN);
   constexpr int R = BT / 32;   // loader rows per thread
   constexpr int WT = BT / 64;  // MFMA tiles per wave and direction
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(kThreads) void prod_apply_kernel(const void* __rest
         const int i = bi * BT + wm * 32 * WT + 32 * mi + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         const int j = bj * BT + wn * 32 * WT + 32 * ni + (lane & 31);
         const int64_t e = x0 + (int64_t)i * N + j;
-        const float bx = round_once ? acc[mi][ni][r] : round_out(acc[mi][ni][r], out_dtype);
+        const float bx = ONCE ? acc[mi][ni][r] : round_out(acc[mi][ni][r], out_dtype);
         store_out(C, e, bx + gamma * load_elem_in<IN>(X, e), out_dtype);
       }
 }
@@ -400,14 +400,14 @@ void launch_gram_blocks(const void* s, void* c, int M, int K, int64_t batch, flo
   }
 }
 
-template <int IN, int BT>
-void launch_apply_blocks(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma,
-                         int round_once, int od, hipStream_t st) {
+template <int IN, int BT, bool ONCE>
+void launch_apply_blocks(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int od,
+                         hipStream_t st) {
   const int64_t items = batch * (M / BT) * (N / BT);
   for (int64_t first = 0; first < items; first += kLaunchItems) {
     const int64_t count = std::min(kLaunchItems, items - first);
-    hipLaunchKernelGGL((prod_apply_kernel<IN, BT>), dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, b, x, c, M, N,
-                       first, count, gamma, round_once, od);
+    hipLaunchKernelGGL((prod_apply_kernel<IN, BT, ONCE>), dim3((unsigned)xcd_grid(count)), dim3(kThreads), 0, st, b, x, c, M, N,
+                       first, count, gamma, od);
   }
 }
 
@@ -451,14 +451,14 @@ void launch_gram(const void* s, void* c, int M, int K, int64_t batch, float alph
   launch_gram_blocks<IN, 64>(s, c, M, K, batch, alpha, beta, add_s, od, st);
 }
 
-template <int IN>
-void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int round_once,
-                  int od, hipStream_t st) {
+template <int IN, bool ONCE = false>
+void launch_apply(const void* b, const void* x, void* c, int M, int N, int64_t batch, float gamma, int od,
+                  hipStream_t st) {
   if constexpr (IN != kInF32 && IN != kInE5m2) {
     if (apply_128(batch * (M / 128) * (N / 128), M, od))
-      return launch_apply_blocks<IN, 128>(b, x, c, M, N, batch, gamma, round_once, od, st);
+      return launch_apply_blocks<IN, 128, ONCE>(b, x, c, M, N, batch, gamma, od, st);
   }
-  launch_apply_blocks<IN, 64>(b, x, c, M, N, batch, gamma, round_once, od, st);
+  launch_apply_blocks<IN, 64, ONCE>(b, x, c, M, N, batch, gamma, od, st);
 }
 
 // 128 x 128 output blocks a call takes.
@@ -485,8 +485,10 @@ int gram(const void* s, void* c, int M, int K, int64_t batch, float alpha, float
 }  // namespace
 
 void ns_any_product(int mode, const NsProduct& g, hipStream_t s) {
-  if (mode == kApply)
-    launch_apply<kInBf16>(g.P, g.Q, g.C, g.M, g.N, g.ntiles, g.beta, g.round_once, HIMUON_DTYPE_BF16, s);
+  if (mode == kApply && g.round_once)
+    launch_apply<kInBf16, true>(g.P, g.Q, g.C, g.M, g.N, g.ntiles, g.beta, HIMUON_DTYPE_BF16, s);
+  else if (mode == kApply)
+    launch_apply<kInBf16>(g.P, g.Q, g.C, g.M, g.N, g.ntiles, g.beta, HIMUON_DTYPE_BF16, s);
   else
     launch_gram<kInBf16>(g.P, g.C, g.M, g.K, g.ntiles, g.alpha, g.beta, mode == kGramB, HIMUON_DTYPE_BF16, s);
 }
@@ -511,10 +513,10 @@ extern "C" int himuon_bmm_add_typed(const void* b, const void* x, void* out, int
   if (batch > kMaxItems / blocks) return HIMUON_EINVAL;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   switch (in_dtype) {
-    case HIMUON_DTYPE_F32: launch_apply<kInF32>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
-    case HIMUON_DTYPE_BF16: launch_apply<kInBf16>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
-    case HIMUON_DTYPE_F16: launch_apply<kInF16>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
-    default: launch_apply<kInE5m2>(b, x, out, M, N, batch, a, 0, out_dtype, st); break;
+    case HIMUON_DTYPE_F32: launch_apply<kInF32>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    case HIMUON_DTYPE_BF16: launch_apply<kInBf16>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    case HIMUON_DTYPE_F16: launch_apply<kInF16>(b, x, out, M, N, batch, a, out_dtype, st); break;
+    default: launch_apply<kInE5m2>(b, x, out, M, N, batch, a, out_dtype, st); break;
   }
   return (int)hipGetLastError();
 }
