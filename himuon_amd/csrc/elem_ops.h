@@ -60,9 +60,10 @@ HM_DEV float add_update(float alpha, float u, float p1) {
 
 // Untile store of 8 consecutive update values y (fp32, already scaled by the
 // parameter's upd_scale) at element offset o of descriptor P's `update`;
-// `full`: all 8 in range, else the first `valid` one at a time. APPLY: `update` is the parameter itself (ld_upd its row stride) and
-// the weight decay and learning rate of its group are applied in place
-// instead of storing the update (himuon_untile_apply):
+// `full`: all 8 in range, else the first `valid` one at a time. APPLY: `update` is
+// the parameter itself (ld_upd its row stride) and the weight decay and learning
+// rate of its group are applied in place instead of storing the update
+// (himuon_untile_apply):
 //     p = rd(fma(alpha_g, rd(u), rd(p * s_g))),  u = upd_scale * NS (fp32)
 // rd the rounding to DT; sa holds (s_g, alpha_g) per group, in device memory.
 template <bool APPLY, int DT>

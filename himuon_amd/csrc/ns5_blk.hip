@@ -7,9 +7,9 @@
 // (ns5_smem.py:89-101, XXT.py:55-75, ba_plus_cAA.py:58-85, fused_bmm_add.py:65-88).
 //
 // One workgroup per block: 4 waves in 2 x 2, each 64 x 64 as 2 x 2 (BT = 64: 32 x
-// 32 as one) v_mfma_f32_32x32x16_bf16 tiles; two workgroups fit a CU (64 KiB of
-// LDS each at BT = 128), so one's MFMAs run while the other waits at a barrier, starts or
-// stores. K advances in units of 64, straight from global memory into one of
+// 32 as one) v_mfma_f32_32x32x16_bf16 tiles; two workgroups fit a CU at BT = 128
+// (64 KiB of LDS each), five at BT = 64 (32 KiB), so one's MFMAs run while another
+// waits at a barrier, starts or stores. K advances in units of 64, straight from global memory into one of
 // two LDS slots (32 KiB each at BT = 128), one unit ahead of the MFMAs; the epilogue operand R
 // (A for GramB, X for Apply) follows as one more unit. The swapped MFMA
 // operand order and the mirrored store are those of the 256-block kernels

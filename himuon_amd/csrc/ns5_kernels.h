@@ -241,9 +241,6 @@ inline int num_cus() {
   return n;
 }
 
-// Fused LDS-resident path (ns5_lds.hip): mp == 128, np = 128 or 256. Runs
-// `steps` >= 1 iterations of `cnt` tiles in one launch; reads X from x and
-// leaves the result in x (even `steps`) or y (odd), as the other paths do.
 // The whole step of a bucket of NS tiles with tile_h <= tile_w <= 128 in one
 // launch (ns5_lds.hip): momentum + gather + normaliser + NS5 + untile with
 // WD/LR, on bucket tiles tile_begin .. tile_begin + cnt - 1; grad/momentum
@@ -260,6 +257,9 @@ void lds_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begi
 bool ns5_small_supported(int m, int mp, int np);
 bool ns5_small_run(const uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int m, int np, int steps,
                    float a, float b, float c, bool round_once, hipStream_t s);
+// Fused LDS-resident path (ns5_lds.hip): mp == 128, np in {128, 256, 512}. Runs
+// `steps` >= 1 iterations of `cnt` tiles in one launch; reads X from x and
+// leaves the result in x (even `steps`) or y (odd), as the other paths do.
 bool ns5_lds_supported(int mp, int np);
 void ns5_lds_run(uint16_t* x, uint16_t* y, const float* inv, int64_t cnt, int mp, int np, int steps,
                  float a, float b, float c, bool round_once, hipStream_t s);
@@ -276,8 +276,8 @@ void reg_step_run(const HimuonParamDesc* params, int n_params, int64_t tile_begi
                   int tile_w, int dtype, int param_dtype, int steps, float a, float b, float c, float eps,
                   bool round_once, const float* sa, hipStream_t s);
 // newton_schulz of cnt contiguous rows x cols matrices (64 < rows <= cols <=
-// 128 / 128 < rows <= cols <= 256, cnt < 2^31) in one launch (ns5_lds.hip,
-// ns5_reg.hip).
+// 128 / 128 < rows <= cols <= 256, cnt < 2^31), one workgroup each, in as few
+// launches as hold them (ns5_lds.hip, ns5_reg.hip).
 void ns_direct_lds_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,
                        float b, float c, float eps, bool round_once, hipStream_t s);
 void ns_direct_reg_run(const void* g, void* out, int64_t cnt, int rows, int cols, int dtype, int steps, float a,

@@ -410,7 +410,9 @@ __global__ __launch_bounds__(NTQ, NQ == 1 ? 3 : 1) void ns5_lds_kernel(const uin
 // 42-43 against 40) and keep the LDS form.
 // (The untile issues all 8 of a thread's parameter loads before using any,
 // 8 VGPRs each; the gather 4 grad and momentum pairs, 16 VGPRs each: 8 would
-// spill.)
+// spill. The instantiations for bf16 grads spill 3 VGPRs and are ahead all the
+// same: the step of 4,608 tiles in bf16 410 us against 447 with X and A / B in
+// LDS.)
 template <int DT, int PDT>
 __global__ __launch_bounds__(NT, 4) void lds_step_kernel(const HimuonParamDesc* __restrict__ params, int n_params,
                                                          int64_t tile_begin, int64_t ntiles, int tile_h,

@@ -84,7 +84,8 @@ HM_DEV float tile_inv(const float (&red)[2][NT / 64], float eps) {
 // (6,720 tiles, bf16 parameters, fp32 grads): 3.53-3.54 ms a step against 4.24
 // with the separate gather and untile launches; one 1024 x 1024 matrix (16
 // tiles) 0.108 against 0.110 ms. 2 or 8 vectors in the gather's load batch and
-// 4 in the untile's: within 0.6 %.
+// 4 in the untile's: within 0.6 %. (256 VGPRs and one spilled, here and in
+// ns_direct_reg_kernel; ns5_reg_kernel takes 203.)
 template <int DT, int PDT>
 __global__ __launch_bounds__(NT, 1) void reg_step_kernel(const HimuonParamDesc* __restrict__ params, int n_params,
                                                          int64_t tile_begin, int64_t ntiles, int tile_h, int tile_w,

@@ -142,14 +142,13 @@ size_t himuon_ns5_workspace_bytes(int64_t sub_batch, int mp, int np);
  * by the first iteration's kernels as they read x, or, for three products of
  * mp >= 768, written over x by one pass before them. Buffers that are not on
  * 16-byte boundaries give the same result, more slowly.
- * Tiles with mp == 128 and np in {128, 256, 512} run all iterations
- * of a tile inside one workgroup's LDS, 256 x 256 tiles with X in registers; more
- * than 16 512 x 512 tiles run the first product on a persistent 256x256-block
- * kernel and the other two fused (himuon_ba_bmm_add's kernel); other
- * geometries run three products, each on the faster of 64x64, 128x128 and
- * (edges that are multiples of 256) 256x256 blocks. Tiles are processed in sub-batches of `sub_batch`;
- * the workspace must hold himuon_ns5_workspace_bytes(sub_batch, mp, np)
- * bytes whenever steps > 0.
+ * Tiles with mp == 128 and np in {128, 256, 512} run all iterations of a tile
+ * inside one workgroup's LDS, 256 x 256 tiles with X in registers; more than 16
+ * 512 x 512 tiles run the second and third product fused (himuon_ba_bmm_add's
+ * kernel); every other product runs on the faster of 64x64, 128x128 and (edges
+ * that are multiples of 256) 256x256 blocks. Tiles are processed in sub-batches
+ * of `sub_batch`; the workspace must hold himuon_ns5_workspace_bytes(sub_batch,
+ * mp, np) bytes whenever steps > 0.
  */
 int himuon_ns5(uint16_t* x, uint16_t* y, const float* inv, int64_t n_tiles,
                int mp, int np, int steps, float a, float b, float c,
