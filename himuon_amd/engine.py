@@ -451,6 +451,8 @@ class _NsPlan:
     stream and per caller's capture, and holds a lock from the one to the other."""
 
     def __init__(self, n: int, M: int, N: int, dtype: torch.dtype, device, round_once: bool, family: str):
+        if family not in nat.NS_FAMILIES:
+            raise ValueError(f"unknown NS kernel family {family!r}")
         self.n, self.M, self.N, self.dtype = n, M, N, dtype
         self.round_once, self.family = round_once, family
         self.m, _, self.mp, self.np, _ = nat.ns_geometry(M, N)

@@ -4,6 +4,7 @@ shape, and nothing else; the kept plans are bounded."""
 from __future__ import annotations
 
 import pytest
+import torch
 
 from himuon_amd import engine as E
 
@@ -34,6 +35,14 @@ def test_the_least_recently_used_plans_make_room(plans):
         E._ns_plan(s, s)
         assert len(plans) <= E._NS_PLANS_TOTAL
         assert sum(k[0] == 0 for k in plans) <= E._NS_PLANS_MAX
+
+
+def test_an_unknown_family_is_refused_and_not_kept(monkeypatch):
+    kept: dict = {}
+    monkeypatch.setattr(E, "_NS_PLANS", kept)
+    with pytest.raises(ValueError):
+        E._ns_plan(0, 2, 300, 300, torch.float32, torch.device("cpu"), False, "fastest")
+    assert not kept
 
 
 def test_what_is_launched_unrecorded():
